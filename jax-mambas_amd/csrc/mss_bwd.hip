@@ -24,6 +24,8 @@
 // no workgroup barrier per state), flushed once per chunk to a per-channel-block partial; a second
 // kernel sums the partials in a fixed order. This replaces the reference's
 // one-global-atomic-per-(b,d,n,t) scheme (selective_scan_bwd_kernel.cuh:295-318).
+#include <algorithm>
+
 #include "mss_common.h"
 
 namespace mss {
@@ -181,6 +183,13 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
   const bc_t* __restrict__ Bb = static_cast<const bc_t*>(p.B) + b * p.bc_sb;
   const bc_t* __restrict__ Cb = static_cast<const bc_t*>(p.C) + b * p.bc_sb;
 
+  // Chunks [c_lo, c_end) of the row are this workgroup's.
+  const int n_chunks = (L + kChunk - 1) / kChunk;
+  const int n_live = (len + kChunk - 1) / kChunk;  // chunks holding at least one valid step
+  const int split = blockIdx.z;
+  const int c_lo = split * p.chunks_per_split;
+  const int c_end = min(n_chunks, c_lo + p.chunks_per_split);
+
   const int n_copy = (kW + N - 1) / N;
   const int acc_floats = n_copy * N * 2 * kChunk;
   float* const acc = lds;
@@ -203,7 +212,17 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
     const int d = blk * p.chan_per_block + cl;
     if (lane < kMaxN) {
       float mu0 = 0.f;
-      if (d < p.dim && lane < N && p.dlast) mu0 = p.dlast[(static_cast<size_t>(b) * p.dim + d) * st_ld + lane];
+      if (d < p.dim && lane < N) {
+        const size_t chan = static_cast<size_t>(b) * p.dim + d;
+        if (p.dlast) mu0 = p.dlast[chan * st_ld + lane];
+        // the message through the chunks to the right (those past the row's length pass it on)
+        const int m_end = p.n_split > 1 ? (n_live - p.chunks_per_split + p.chunks_per_msg - 1) / p.chunks_per_msg : 0;
+        const size_t m_ld = static_cast<size_t>(p.batch) * p.dim * N * 2;
+        const float* pq = p.split_msg + (chan * N + lane) * 2;
+#pragma unroll 4
+        for (int m = m_end - 1; m >= c_lo / p.chunks_per_msg; --m)
+          mu0 = __builtin_fmaf(pq[m * m_ld], mu0, pq[m * m_ld + 1]);
+      }
       s_mu[cl][lane] = mu0;
       s_dA[cl][lane] = 0.f;
     }
@@ -213,13 +232,12 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
     }
   }
 
-  const int n_chunks = (L + kChunk - 1) / kChunk;
-  const int n_live = (len + kChunk - 1) / kChunk;  // chunks holding at least one valid step
-  if (n_live > 0) stage_chunk<kT, kW, bc_t>(Bb, Cb, N, (n_live - 1) * kChunk, L, p.bc_sn, dma, stage, tid);
+  const int c_first = min(n_live, c_end) - 1;  // the first chunk worked on
+  if (c_first >= c_lo) stage_chunk<kT, kW, bc_t>(Bb, Cb, N, c_first * kChunk, L, p.bc_sn, dma, stage, tid);
   wait_vmem_all();
   __syncthreads();
 
-  for (int c = n_chunks - 1; c >= 0; --c) {
+  for (int c = c_end - 1; c >= c_lo; --c) {
     const int t0 = c * kChunk;
     const int tl = t0 + seg * kT;  // first step of this lane's segment
     const bool fast = vec_io && (t0 + kChunk <= L);  // wave-uniform
@@ -483,7 +501,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
     // next chunk (to the left), then flush this chunk's dB/dC sums over the block's channels.
     __syncthreads();
     if (tid < kW) s_done[tid] = 0;  // (read again only after the barrier that ends the flush)
-    if (c > 0) stage_chunk<kT, kW, bc_t>(Bb, Cb, N, t0 - kChunk, L, p.bc_sn, dma, stage, tid);
+    if (c > c_lo) stage_chunk<kT, kW, bc_t>(Bb, Cb, N, t0 - kChunk, L, p.bc_sn, dma, stage, tid);
     const size_t nl = static_cast<size_t>(N) * L;
     float* part = p.part_dBC + static_cast<size_t>(blk) * p.part_stride + static_cast<size_t>(b) * 2 * nl;
     const bool vec_part = (L % 4) == 0;
@@ -520,17 +538,110 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
     __syncthreads();
   }
 
-  // ---- per-channel partial sums (over this row's steps)
+  // ---- per-channel partial sums (over this workgroup's steps)
   for (int k = 0; k < K; ++k) {
     const int cl = k * kW + w;
     const int d = blk * p.chan_per_block + cl;
     if (d >= p.dim) continue;
-    const size_t chan = static_cast<size_t>(b) * p.dim + d;
+    const size_t chan = (static_cast<size_t>(split) * p.batch + b) * p.dim + d;
     if (lane < N) p.part_dA[chan * N + lane] = s_dA[cl][lane];
     if (lane == 0) {
       p.part_dD[chan] = s_dD[cl];
       p.part_dbias[chan] = s_db[cl];
     }
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// The adjoint maps of a time-split backward (BwdParams::split_msg): for every (channel, state)
+// and every run of chunks_per_msg chunks right of the first split, (P, Q) with P the product of
+// the run's a_bar and Q the message the run sends left when none enters it from the right. Only
+// delta, the gated dout and C are read, and no state: lambda_t = a_{t+1} lambda_{t+1} + C_t g_t.
+// One wave per (channel, run), lane = 8 steps in reversed order as in bwd_kernel; C rows
+// straight from memory, the next state's loaded while this one computes (the waves of a
+// workgroup share them in the cache). Bound by VALU issue (an exponential and three more
+// instructions per step and state), so the runs are cut short enough to fill the chip.
+constexpr int kMsgW = 8;
+
+template <bool kHasZ, typename io_t, typename bc_t>
+__global__ __launch_bounds__(kMsgW * 64) void bwd_msg_kernel(BwdParams p) {
+  constexpr int kT = kBwdT;
+  constexpr int kChunk = kBwdChunk;
+  __shared__ float s_q[kMsgW][kMaxN];
+  __shared__ float s_a2[kMsgW][kMaxN];
+  const int lane = threadIdx.x & 63;
+  const int seg = 63 - lane;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.y;
+  const int d = blockIdx.x * kMsgW + w;
+  if (d >= p.dim) return;  // no barrier in this kernel: idle waves may leave
+  const int L = p.seqlen;
+  const int N = p.dstate;
+  const int len = p.seq_lens ? min(max(p.seq_lens[b], 0), L) : L;
+  const int n_live = (len + kChunk - 1) / kChunk;
+  const int c_lo = p.chunks_per_split + blockIdx.z * p.chunks_per_msg;
+  const int c_hi = min(n_live, c_lo + p.chunks_per_msg);
+  if (c_lo >= c_hi) return;  // no valid step: bwd_kernel skips the run
+  const size_t chan = static_cast<size_t>(b) * p.dim + d;
+  const long long row = b * p.io_sb + d * p.io_sd;
+  const bc_t* __restrict__ Cb = static_cast<const bc_t*>(p.C) + b * p.bc_sb;
+  if (lane < N) {
+    s_q[w][lane] = 0.f;
+    s_a2[w][lane] = p.A[static_cast<size_t>(d) * p.a_ld + lane] * kLog2e;
+  }
+  const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
+  float dsum = 0.f;  // sum of delta over the run
+  for (int c = c_hi - 1; c >= c_lo; --c) {
+    const int t0 = c * kChunk;
+    const int tl = t0 + seg * kT;
+    const bool inside = t0 + kChunk <= L;  // wave-uniform
+    const bool fast = p.vec_io && inside;
+    const bool fast_c = p.vec_bc && inside;
+    float dlt[kT], g[kT], cv[kT];
+    load_seg<kT>(static_cast<const io_t*>(p.delta) + row, tl, L, fast, dlt);
+    load_seg<kT>(static_cast<const io_t*>(p.dout) + row, tl, L, fast, g);
+    if constexpr (kHasZ) {
+      float zr[kT];
+      load_seg<kT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zr);
+#pragma unroll
+      for (int j = 0; j < kT; ++j) g[j] *= zr[j] * sigmoid(zr[j]);
+    }
+    load_seg<kT>(Cb, tl, L, fast_c, cv);
+#pragma unroll
+    for (int j = 0; j < kT; ++j) dlt[j] += bias;
+    if (p.delta_softplus) {
+#pragma unroll
+      for (int j = 0; j < kT; ++j) dlt[j] = softplus(dlt[j]);
+    }
+    float ssum = 0.f;
+#pragma unroll
+    for (int j = 0; j < kT; ++j) {
+      const bool valid = tl + j < len;
+      dlt[j] = valid ? dlt[j] : 0.f;
+      g[j] = valid ? g[j] : 0.f;
+      ssum += dlt[j];
+    }
+    dsum += wave_sum(ssum);
+    for (int n = 0; n < N; ++n) {
+      const float a2 = s_a2[w][n];
+      const float q_in = s_q[w][n];
+      float cn[kT];
+      load_seg<kT>(Cb + min(n + 1, N - 1) * p.bc_sn, tl, L, fast_c, cn);
+      float lam = 0.f;
+#pragma unroll
+      for (int j = kT - 1; j >= 0; --j)
+        lam = fast_exp2(dlt[j] * a2) * __builtin_fmaf(g[j], cv[j], lam);
+      float P = fast_exp2(a2 * ssum);
+      wave_scan_affine_fwd(P, lam);  // lane 63 (the chunk's first segment): the whole chunk
+      if (lane == 63) s_q[w][n] = __builtin_fmaf(P, q_in, lam);
+#pragma unroll
+      for (int j = 0; j < kT; ++j) cv[j] = cn[j];
+    }
+  }
+  if (lane < N) {
+    float* pq = p.split_msg + ((static_cast<size_t>(blockIdx.z) * p.batch * p.dim + chan) * N + lane) * 2;
+    pq[0] = fast_exp2(s_a2[w][lane] * dsum);
+    pq[1] = s_q[w][lane];
   }
 }
 
@@ -544,8 +655,8 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
 //     either way, so both depths give the same bits. With
 //     seq_lens, steps from live_part_end(len, L) on are zero (the scans write no partials
 //     there);
-//   the remaining blocks: dA[d][n] = sum_b part_dA[b][d][n] (dA rows a_ld apart); dD[d],
-//     dbias[d] likewise (dbias added to its current value when acc_bias: a state group of a
+//   the remaining blocks: dA[d][n] = sum_b part_dA[b][d][n] over the `batch` (times the time
+//     splits) rows of partials (dA rows a_ld apart); dD[d], dbias[d] likewise (dbias added to its current value when acc_bias: a state group of a
 //     wider scan).
 template <bool kVec, typename bc_t, int kDepth>
 __global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ part, int n_blk,
@@ -623,7 +734,7 @@ __global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ p
 
 template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup>
 static hipError_t launch_bwd_a(const BwdParams& p, hipStream_t stream) {
-  dim3 grid(p.n_blocks_d, p.batch);
+  dim3 grid(p.n_blocks_d, p.batch, p.n_split);
   if (p.waves == 16) {
     if (!bwd_waves_fit(16, p.dstate) || p.chan_per_block % 16 != 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL((bwd_kernel<16, kZOH, kHasZ, io_t, bc_t, kGroup>), grid, dim3(16 * 64), 0, stream, p);
@@ -648,6 +759,13 @@ static hipError_t launch_bwd_t(const BwdParams& p, hipStream_t stream) {
 template <typename io_t, typename bc_t>
 static hipError_t launch_bwd_io(const BwdParams& p, int zoh, hipStream_t stream) {
   const bool hz = p.z != nullptr;
+  if (p.n_split > 1) {
+    const dim3 grid((p.dim + kMsgW - 1) / kMsgW, p.batch, p.n_msg);
+    hipLaunchKernelGGL((hz ? bwd_msg_kernel<true, io_t, bc_t> : bwd_msg_kernel<false, io_t, bc_t>), grid,
+                       dim3(kMsgW * 64), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   if (zoh) return hz ? launch_bwd_t<true, true, io_t, bc_t>(p, stream)
                      : launch_bwd_t<true, false, io_t, bc_t>(p, stream);
   return hz ? launch_bwd_t<false, true, io_t, bc_t>(p, stream)
@@ -667,7 +785,47 @@ static int chan_per_block_for(int waves, int batch, int dim, long long target) {
   return static_cast<int>(k) * waves;
 }
 
-BwdPlan bwd_plan(int batch, int dim, int dstate, int varlen) {
+// The plan of a grid whose whole-row workgroups would leave half the CUs or more idle: rows are
+// split in time as well, so that the grid fills one pass. More channel rounds K per workgroup
+// then mean more, shorter splits: fewer dB/dC partials to write and reduce, against more steps
+// in the adjoint maps (every split but the first). The modelled microseconds, from MI355X
+// measurements at B=1 D=1536 L=16384 N=16 bf16: a 12-wave round of a chunk 7 + 1.1 N, the maps
+// 0.25 per million (step, state), partials at 4.5 TB/s each way. There the backward took 840 us
+// as 128 whole-row workgroups (scan 787, reduction 53) and takes 525 as 16 splits of 8 rounds
+// (maps 130, scan 385, reduction 10; two splits of one round: 540); B=2 D=768 L=1024 float32 ZOH
+// 83 -> 62. Grids over half the CUs stay whole: the maps cost a third of the scan.
+static BwdPlan bwd_split_plan(int batch, int dim, int seqlen, int dstate, int n_chunks) {
+  BwdPlan best{};
+  double best_us = 0;
+  for (int waves = 12; waves <= 16; waves += 4) {
+    if (!bwd_waves_fit(waves, dstate)) continue;
+    for (int k = 1; k * waves <= kMaxChanPerBlock && (k == 1 || (k - 1) * waves < dim); k *= 2) {
+      BwdPlan plan{waves, k * waves};
+      const int blocks = (dim + plan.chan_per_block - 1) / plan.chan_per_block;
+      const int s = static_cast<int>(std::min<long long>(kCUs / (static_cast<long long>(batch) * blocks), n_chunks));
+      plan.chunks_per_split = (n_chunks + s - 1) / s;
+      // Maps as long as they can be with 24 waves for every CU.
+      const long long map_chunks = static_cast<long long>(batch) * dim * (n_chunks - plan.chunks_per_split);
+      const long long want = std::max(1LL, map_chunks / (24LL * kCUs));
+      const int per_split = static_cast<int>((plan.chunks_per_split + want - 1) / want);
+      plan.chunks_per_msg = (plan.chunks_per_split + per_split - 1) / per_split;
+      plan.chunks_per_split = plan.chunks_per_msg * per_split;
+      plan.n_split = (n_chunks + plan.chunks_per_split - 1) / plan.chunks_per_split;
+      plan.n_msg = plan.n_split > 1 ? (n_chunks - plan.chunks_per_split + plan.chunks_per_msg - 1) / plan.chunks_per_msg : 0;
+      const double round = (7 + 1.1 * dstate) * (waves == 16 ? 1.2 : 1.0);
+      const double maps = 0.25e-6 * batch * dim * dstate * std::max(0, seqlen - plan.chunks_per_split * kBwdChunk);
+      const double parts = 2.0 * blocks * batch * 2 * dstate * seqlen * 4 / 4.5e6;
+      const double us = round * k * plan.chunks_per_split + maps + parts;
+      if (best.waves == 0 || us < best_us) {
+        best = plan;
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
+BwdPlan bwd_plan(int batch, int dim, int seqlen, int dstate, int varlen, bool split) {
   // One workgroup per CU holds the B/C stage and the dB/dC accumulator (LDS), so the grid
   // should fit one pass over the 256 CUs. With variable lengths rows finish at different
   // times, so workgroups stay ~2x smaller and the hardware balances them (rows are handed
@@ -688,6 +846,10 @@ BwdPlan bwd_plan(int batch, int dim, int dstate, int varlen) {
     const int cpb16 = chan_per_block_for(16, batch, dim, target);
     if (cost(16, cpb16) < cost(12, plan.chan_per_block)) plan = BwdPlan{16, cpb16};
   }
+  const int n_chunks = (seqlen + kBwdChunk - 1) / kBwdChunk;
+  plan.chunks_per_split = n_chunks;
+  const long long grid = static_cast<long long>(batch) * ((dim + plan.chan_per_block - 1) / plan.chan_per_block);
+  if (split && 2 * grid <= kCUs && n_chunks > 1) plan = bwd_split_plan(batch, dim, seqlen, dstate, n_chunks);
   return plan;
 }
 
@@ -714,7 +876,7 @@ hipError_t launch_bwd_reduce(const BwdParams& p, int bc_bf16, int a_width, int a
                      0, stream, p.part_dBC, p.n_blocks_d,                                          \
                      p.part_stride, L, p.dstate, x_blocks, n_bc_blocks, p.bc_sb, p.bc_sn,          \
                      static_cast<T*>(dB), static_cast<T*>(dC), p.part_dA, p.part_dD, p.part_dbias,  \
-                     p.batch, p.dim, a_width, a_ld, acc_bias, static_cast<float*>(dA), dD, dbias, \
+                     p.batch * p.n_split, p.dim, a_width, a_ld, acc_bias, static_cast<float*>(dA), dD, dbias, \
                      p.seq_lens)
   if (bc_bf16) {
     if (vec) MSS_REDUCE(true, bf16_t); else MSS_REDUCE(false, bf16_t);

@@ -27,7 +27,7 @@ hipError_t launch_bwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16
                            hipStream_t stream);
 hipError_t launch_bwd_reduce(const BwdParams& p, int bc_bf16, int a_width, int a_ld, int acc_bias,
                              void* dA, void* dB, void* dC, float* dD, float* dbias, hipStream_t stream);
-BwdPlan bwd_plan(int batch, int dim, int dstate, int varlen);
+BwdPlan bwd_plan(int batch, int dim, int seqlen, int dstate, int varlen, bool split);
 hipError_t launch_cfwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
 hipError_t launch_cbwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
 int cbwd_chan_per_block(int batch, int dim);
@@ -144,29 +144,39 @@ int n_seg_of(int32_t seqlen) { return (seqlen + MSS_SEG_STEPS - 1) / MSS_SEG_STE
 
 struct BwdLayout {
   int waves = 12, chan_per_block = 0, n_blocks_d = 0;
+  int n_split = 1, chunks_per_split = 0, n_msg = 0, chunks_per_msg = 1;
   size_t part_stride = 0;  // floats per channel block of dB/dC partials (multiple of 64)
-  size_t off_dA = 0, off_dD = 0, off_db = 0, total = 0;
+  size_t off_dA = 0, off_dD = 0, off_db = 0, off_msg = 0, total = 0;
 };
 
 // cplx: the complex-A backward (its own channel blocking; dA partials are complex).
+// split: false keeps each row whole where the plan would split it in time (the smallest
+// workspace the call runs with).
 BwdLayout bwd_layout(int32_t batch, int32_t dim, int32_t seqlen, int32_t dstate, bool varlen,
-                     bool cplx = false) {
+                     bool cplx = false, bool split = true) {
   BwdLayout l;
+  l.chunks_per_split = (seqlen + mss::kPartChunk - 1) / mss::kPartChunk;
   if (cplx) {
     l.chan_per_block = mss::cbwd_chan_per_block(batch, dim);
   } else {
-    const mss::BwdPlan plan = mss::bwd_plan(batch, dim, dstate, varlen ? 1 : 0);
+    const mss::BwdPlan plan = mss::bwd_plan(batch, dim, seqlen, dstate, varlen ? 1 : 0, split);
     l.waves = plan.waves;
     l.chan_per_block = plan.chan_per_block;
+    l.n_split = plan.n_split;
+    l.chunks_per_split = plan.chunks_per_split;
+    l.n_msg = plan.n_msg;
+    l.chunks_per_msg = std::max(1, plan.chunks_per_msg);
   }
   l.n_blocks_d = (dim + l.chan_per_block - 1) / l.chan_per_block;
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
   l.part_stride = (static_cast<size_t>(batch) * 2 * dstate * seqlen + 63) / 64 * 64;
   const size_t bc = static_cast<size_t>(l.n_blocks_d) * l.part_stride * sizeof(float);
   l.off_dA = up(bc);
-  l.off_dD = l.off_dA + up(static_cast<size_t>(batch) * dim * dstate * (cplx ? 2 : 1) * sizeof(float));
-  l.off_db = l.off_dD + up(static_cast<size_t>(batch) * dim * sizeof(float));
-  l.total = l.off_db + up(static_cast<size_t>(batch) * dim * sizeof(float));
+  const size_t chans = static_cast<size_t>(batch) * dim;
+  l.off_dD = l.off_dA + up(l.n_split * chans * dstate * (cplx ? 2 : 1) * sizeof(float));
+  l.off_db = l.off_dD + up(l.n_split * chans * sizeof(float));
+  l.off_msg = l.off_db + up(l.n_split * chans * sizeof(float));
+  l.total = l.off_msg + up(l.n_msg * chans * dstate * 2 * sizeof(float));
   return l;
 }
 
@@ -174,11 +184,11 @@ BwdLayout bwd_layout(int32_t batch, int32_t dim, int32_t seqlen, int32_t dstate,
 // one after another in one workspace, sized for the larger of the two group sizes (its
 // plan is the one reported for the call).
 BwdLayout bwd_layout_call(int32_t batch, int32_t dim, int32_t seqlen, int32_t dstate, bool varlen,
-                          bool cplx = false) {
-  if (cplx || dstate <= MSS_MAX_DSTATE) return bwd_layout(batch, dim, seqlen, dstate, varlen, cplx);
+                          bool cplx = false, bool split = true) {
+  if (cplx || dstate <= MSS_MAX_DSTATE) return bwd_layout(batch, dim, seqlen, dstate, varlen, cplx, split);
   const int G = state_groups(dstate);
-  const BwdLayout hi = bwd_layout(batch, dim, seqlen, (dstate + G - 1) / G, varlen);
-  const BwdLayout lo = bwd_layout(batch, dim, seqlen, dstate / G, varlen);
+  const BwdLayout hi = bwd_layout(batch, dim, seqlen, (dstate + G - 1) / G, varlen, false, split);
+  const BwdLayout lo = bwd_layout(batch, dim, seqlen, dstate / G, varlen, false, split);
   return hi.total >= lo.total ? hi : lo;
 }
 
@@ -278,6 +288,10 @@ mss::BwdParams pack_bwd(const mss_bwd_args* a, const BwdLayout& l, char* ws) {
   p.waves = l.waves;
   p.chan_per_block = l.chan_per_block;
   p.n_blocks_d = l.n_blocks_d;
+  p.n_split = l.n_split;
+  p.chunks_per_split = l.chunks_per_split;
+  p.n_msg = l.n_msg;
+  p.chunks_per_msg = l.chunks_per_msg;
   p.u = a->u;
   p.delta = a->delta;
   p.A = a->A;
@@ -306,6 +320,7 @@ mss::BwdParams pack_bwd(const mss_bwd_args* a, const BwdLayout& l, char* ws) {
   p.part_dA = reinterpret_cast<float*>(ws + l.off_dA);
   p.part_dD = reinterpret_cast<float*>(ws + l.off_dD);
   p.part_dbias = reinterpret_cast<float*>(ws + l.off_db);
+  p.split_msg = reinterpret_cast<float*>(ws + l.off_msg);
   return p;
 }
 
@@ -315,7 +330,10 @@ int run_bwd(const mss_bwd_args* a, int phases, hipStream_t stream, bool cplx = f
   // State groups hand the du/ddelta/ddelta_bias sums from one group to the next, so the two
   // phases cannot be split across calls.
   if (grouped && phases != kPhaseBoth) return MSS_ERR_UNSUPPORTED;
-  const BwdLayout l = bwd_layout_call(a->batch, a->dim, a->seqlen, a->dstate, varlen, cplx);
+  BwdLayout l = bwd_layout_call(a->batch, a->dim, a->seqlen, a->dstate, varlen, cplx);
+  // A caller's workspace too small for the time-split plan runs the whole-row one.
+  const bool split = a->workspace == nullptr || a->workspace_bytes >= l.total;
+  if (!split) l = bwd_layout_call(a->batch, a->dim, a->seqlen, a->dstate, varlen, cplx, false);
   char* ws = static_cast<char*>(a->workspace);
   bool owned = false;
   if (ws == nullptr) {
@@ -349,7 +367,7 @@ int run_bwd(const mss_bwd_args* a, int phases, hipStream_t stream, bool cplx = f
     const int N = a->dstate;
     for (int g = 0; g < state_groups(N) && e == hipSuccess; ++g) {
       const int n0 = group_begin(N, g), ng = group_begin(N, g + 1) - n0;
-      mss::BwdParams p = pack_bwd(a, bwd_layout(a->batch, a->dim, a->seqlen, ng, varlen), ws);
+      mss::BwdParams p = pack_bwd(a, bwd_layout(a->batch, a->dim, a->seqlen, ng, varlen, false, split), ws);
       const size_t bc_off = static_cast<size_t>(n0) * p.bc_sn * sizeof(float);
       p.dstate = ng;
       p.A = a->A + n0;
@@ -512,7 +530,8 @@ int mss_bwd(const mss_bwd_args* args, void* stream) {
 int mss_bwd_noalloc(const mss_bwd_args* args, void* stream) {
   const int s = validate_bwd(args);
   if (s != MSS_OK) return s;
-  const BwdLayout l = bwd_layout_call(args->batch, args->dim, args->seqlen, args->dstate, args->seq_lens != nullptr);
+  const BwdLayout l = bwd_layout_call(args->batch, args->dim, args->seqlen, args->dstate, args->seq_lens != nullptr,
+                                      false, false);
   if (l.total > kScratchBytes) return MSS_ERR_SCRATCH_LIMIT;
   void* ws = nullptr;
   const int t = scratch_of_current_device(&ws);
@@ -1210,13 +1229,14 @@ int mss_scan_bwd_ws(void* stream, int32_t batch, int32_t length, int32_t dim, in
     return MSS_ERR_INVALID_ARGUMENT;
   // The carry rebuild runs one grid slice per 2048-step block (grid.z).
   if ((length + MSS_REF_CHUNK - 1) / MSS_REF_CHUNK > 65535) return MSS_ERR_UNSUPPORTED;
+  const size_t carry_bytes = scan_bwd_carry_bytes(batch, length, dim, dstate);
+  // (the smallest workspace mss_bwd runs with: without its time splits)
   if (workspace == nullptr || !aligned16(workspace) ||
-      workspace_bytes < mss_scan_bwd_workspace_bytes(batch, length, dim, dstate))
+      workspace_bytes < carry_bytes + bwd_layout_call(batch, dim, length, dstate, false, false, false).total)
     return MSS_ERR_WORKSPACE;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
   float* carries = reinterpret_cast<float*>(ws);
-  const size_t carry_bytes = scan_bwd_carry_bytes(batch, length, dim, dstate);
   // The backward re-runs each 8-step segment from the state entering it; the reference
   // residual holds the state at 2048-step block ends only, so each block's recurrence is
   // re-run from it first (one state pass, blocks in parallel).

@@ -506,9 +506,15 @@ struct FwdParams {
 // z is not tiny, so the real-A forward keeps y itself (y_pre) only where |z| < kZTiny.
 constexpr float kZTiny = 1e-20f;
 
-// Backward launch shape: waves per workgroup and channels per workgroup.
+// Backward launch shape: waves per workgroup, channels per workgroup, and the time splits of a
+// row (each `chunks_per_split` chunks of kPartChunk steps, the last one possibly fewer; 1: the
+// row is one workgroup's).
 struct BwdPlan {
   int waves, chan_per_block;
+  int n_split = 1, chunks_per_split = 0;
+  // Time-split rows: the adjoint maps cover `chunks_per_msg` chunks each (a divisor of
+  // chunks_per_split), `n_msg` of them from the second split's first chunk on.
+  int n_msg = 0, chunks_per_msg = 0;
 };
 
 struct BwdParams {
@@ -519,6 +525,7 @@ struct BwdParams {
   int waves;           // waves per backward workgroup (12 or 16)
   int chan_per_block;  // channels one workgroup walks (multiple of the wave count)
   int n_blocks_d;      // ceil(dim / chan_per_block)
+  int n_split, chunks_per_split, n_msg, chunks_per_msg;  // time splits of a row (BwdPlan)
   long long io_sb, io_sd;  // row strides of u/delta/z/y_pre/dout/du/ddelta/dz
   long long bc_sb, bc_sn;  // row strides of B/C and dB/dC
   const void* u;
@@ -550,9 +557,13 @@ struct BwdParams {
   // workspace partials
   float* part_dBC;   // [n_blocks_d][part_stride]; block = [batch][2][dstate][L] (+ padding)
   size_t part_stride;  // floats per channel block, a multiple of 64
-  float* part_dA;    // [batch][dim][dstate]
-  float* part_dD;    // [batch][dim]
-  float* part_dbias; // [batch][dim]
+  float* part_dA;    // [n_split][batch][dim][dstate]
+  float* part_dD;    // [n_split][batch][dim]
+  float* part_dbias; // [n_split][batch][dim]
+  // n_split > 1: the adjoint map (P, Q) of every run of chunks_per_msg chunks right of the first
+  // split, which sends the message m from its right on to its left as P m + Q:
+  // [n_msg][batch][dim][dstate][2]
+  float* split_msg;
 };
 
 }  // namespace mss

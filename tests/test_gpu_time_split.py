@@ -1,0 +1,44 @@
+"""Scans whose rows are split in time because their channels alone would leave the GPU idle:
+every output and gradient against the float64 oracle, at the edges of the split plans."""
+import pytest
+import torch
+
+from mamba_amd import _lib
+from test_gpu_parity import check_fused, fused_case, log, oracle_fused, run_fused, tol
+from test_zz_no_alloc import GRADS, _backward, _forward, _inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("b,d,l,n,lens,dtype,zoh", [
+    (1, 5, 513, 16, None, "f32", False),       # two chunks, the second of one step
+    (8, 192, 2051, 16, None, "f32", False),    # two splits of three chunks (the second: two and a bit)
+    (8, 192, 8190, 4, None, "bf16", False),    # several chunks to an adjoint map
+    (1, 70, 4096, 11, None, "bf16", True),     # eight splits of one whole chunk, two accumulator copies
+    (3, 100, 4100, 16, [4100, 1, 2560], "f32", False),  # rows ending before, at and inside a split
+    (3, 100, 4100, 8, [0, 4099, 513], "bf16", True),
+])
+def test_time_split_scan(b, d, l, n, lens, dtype, zoh):
+    log(f"case time split b={b} d={d} l={l} n={n} lens={lens} {dtype} zoh={zoh}")
+    x, dout, dlast = fused_case(2000 + l + n, b, d, l, n, dtype, lens=lens, zoh=zoh)
+    ts, out, last = run_fused(x, dout, dlast, dtype, zoh)
+    fw, g = oracle_fused(x, dout, dlast, zoh)
+    check_fused(ts, out, last, fw, g, *tol(dtype))
+
+
+@pytest.mark.parametrize("n", [16, 20])
+def test_backward_in_a_smaller_workspace(n):
+    """A workspace that holds the whole-row plan but not the time-split one: the whole-row
+    plan runs. Both take the same per-step arithmetic, so the results differ by the order of
+    a row's sums only (float32; at most 8 chunks: 1e-5 of the largest value)."""
+    lib = _lib.register_hip_kernel()
+    b, d, l = 2, 40, 4000
+    x, dout, dlast = _inputs(5, b, d, l, n)
+    carries, y_pre, out = _forward(lib, x, b, d, l, n)
+    full = int(lib.mss_bwd_workspace_bytes(_lib.BwdArgs(batch=b, dim=d, seqlen=l, dstate=n)))
+    res = [_backward(lib, lib.mss_bwd, x, carries, y_pre, out, dout, dlast, b, d, l, n,
+                     workspace=torch.empty(size, dtype=torch.uint8, device="cuda")) for size in (full, full - 256)]
+    for k in GRADS:
+        err = (res[0][k] - res[1][k]).abs().max() / res[0][k].abs().max()
+        log(f"  {k}: {err:.1e}")
+        assert err < 1e-5, k
