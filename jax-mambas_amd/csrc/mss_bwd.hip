@@ -120,22 +120,15 @@ __device__ __forceinline__ void stage_chunk(const bc_t* __restrict__ Bb, const b
       __builtin_amdgcn_global_load_lds((gbl_void_t)src, (lds_void_t)(&dst[n][which][s0]), 16, 0, 0);
     }
   } else {
-    for (int f = tid; f < N * 2 * 64 * kT; f += kW * 64) {
-      const int rowi = f / (64 * kT);
+    const bool fast = t0 + 64 * kT <= L;
+    for (int f = tid; f < N * 2 * kSlots; f += kW * 64) {
+      const int rowi = f / kSlots;
       const int n = rowi >> 1;
       const int which = rowi & 1;
-      const int e = f - rowi * 64 * kT;
-      const int i = e / kT;
-      const int r = e % kT;
-      const int sl = kQ * i + ((r / kE) ^ slot_swz<kQ>(i));
-      const int t = t0 + e;
-      bc_t v;
-      if (t < L) {
-        v = ((which ? Cb : Bb) + n * sn)[t];
-      } else {
-        store_as(&v, 0.f);
-      }
-      reinterpret_cast<bc_t*>(&dst[n][which][0])[sl * kE + (r % kE)] = v;
+      const int s = f - rowi * kSlots;
+      const int i = s / kQ;
+      const int q = (s % kQ) ^ slot_swz<kQ>(i);
+      dst[n][which][s] = load_slot((which ? Cb : Bb) + n * sn, t0 + i * kT + q * kE, L, fast);
     }
   }
 }
@@ -144,7 +137,13 @@ __device__ __forceinline__ void stage_chunk(const bc_t* __restrict__ Bb, const b
 // more than kMaxN states (A, the state buffers and the carries read with the strides of the
 // full tensors, p.a_ld / p.state_ld / p.carry_cs; dz only where p.dz is given); 2 = a later
 // group (as 1, and du/ddelta add to the values already in their buffers).
-template <int kW, bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup = 0>
+//
+// kWhole: L is a multiple of the chunk and the B/C rows can be copied to LDS directly, so no
+// lane ever meets the row's end (those paths' registers spill the 16-wave kernel). Measured on
+// MI355X (B=8 D=2048 L=4096 bf16): 871 us with every row loaded and unpacked by itself, so that
+// five memory latencies followed one another, 798 with the rows fetched together; the general
+// instance 887 there. B=3 D=1000 L=2051 bf16: 225 us with element-wise accesses, 144.
+template <int kW, bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup, bool kWhole>
 __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
   constexpr bool kAcc = kGroup == 2;
   constexpr int kT = kBwdT;
@@ -178,8 +177,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
   const long long carry_cs = kGroup ? p.carry_cs : static_cast<long long>(N) * p.n_seg;
   const bool has_dz = kGroup ? p.dz != nullptr : true;  // (z given: dz given, ungrouped)
   const int len = p.seq_lens ? min(max(p.seq_lens[b], 0), L) : L;
-  const bool vec_io = p.vec_io != 0;
-  const bool dma = p.vec_bc != 0;
+  const bool dma = kWhole || p.vec_bc != 0;
   const bc_t* __restrict__ Bb = static_cast<const bc_t*>(p.B) + b * p.bc_sb;
   const bc_t* __restrict__ Cb = static_cast<const bc_t*>(p.C) + b * p.bc_sb;
 
@@ -240,9 +238,9 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
   for (int c = c_end - 1; c >= c_lo; --c) {
     const int t0 = c * kChunk;
     const int tl = t0 + seg * kT;  // first step of this lane's segment
-    const bool fast = vec_io && (t0 + kChunk <= L);  // wave-uniform
+    const bool fast = kWhole || t0 + kChunk <= L;  // wave-uniform
     const int seg_idx = t0 / kT + seg;               // index into a carries row
-    const bool seg_ok = seg_idx < p.n_seg;
+    const bool seg_ok = kWhole || seg_idx < p.n_seg;
 
     if (c >= n_live) {
       // Whole chunk past this row's length: zero gradients; the adjoint message passes
@@ -293,16 +291,25 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       {
         // Unconditional, so no per-step value needs a copy for the inactive path: a wave past
         // the last channel reads the clamped channel's row and never stores or accumulates.
-        load_seg<kT>(static_cast<const io_t*>(p.delta) + row, tl, L, fast, dlt);
-        load_seg<kT>(static_cast<const io_t*>(p.u) + row, tl, L, fast, uu);
-        load_seg<kT>(static_cast<const io_t*>(p.dout) + row, tl, L, fast, g);
+        // All rows are fetched before the first is used: one memory latency.
+        Seg<kT, io_t> sd, su, sg, sz_, so;
+        fetch(sd, static_cast<const io_t*>(p.delta) + row, tl, L, kWhole);
+        fetch(su, static_cast<const io_t*>(p.u) + row, tl, L, kWhole);
+        fetch(sg, static_cast<const io_t*>(p.dout) + row, tl, L, kWhole);
+        if constexpr (kHasZ) {
+          fetch(sz_, static_cast<const io_t*>(p.z) + row, tl, L, kWhole);
+          fetch(so, static_cast<const io_t*>(p.out) + row, tl, L, kWhole);
+        }
+        finish(sd, tl, L, fast, dlt);
+        finish(su, tl, L, fast, uu);
+        finish(sg, tl, L, fast, g);
         if constexpr (kHasZ) {
           // g = dout * silu(z); dz = dout * y * sigmoid(z) * (1 + z * (1 - sigmoid(z))). With the
           // forward's out = y z sigmoid(z): dz = dout * out * (1 / z + 1 - sigmoid(z)), and where
           // |z| < kZTiny (out / z imprecise) y itself, which the forward kept there.
           float zr[kT], yp[kT];
-          load_seg<kT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zr);
-          load_seg<kT>(static_cast<const io_t*>(p.out) + row, tl, L, fast, yp);
+          finish(sz_, tl, L, fast, zr);
+          finish(so, tl, L, fast, yp);
           const io_t* __restrict__ ykept = static_cast<const io_t*>(p.y_pre) + row;
 #pragma unroll
           for (int j = 0; j < kT; ++j) {
@@ -451,7 +458,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       // ---- per-step gradients of the row
       if constexpr (!kZOH) {
         // Euler needs u only from here on: reload it rather than hold it across the loop.
-        load_seg<kT>(static_cast<const io_t*>(p.u) + row, tl, L, fast, uu);
+        load_seg<kT>(static_cast<const io_t*>(p.u) + row, tl, L, fast, uu, kWhole);
       }
       float dD_acc = 0.f, db_acc = 0.f;
       float duv[kT], ddv[kT];
@@ -480,10 +487,10 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       }
       if constexpr (kAcc) {
         float prev[kT];
-        load_seg<kT>(static_cast<const io_t*>(p.du) + row, tl, L, fast, prev);
+        load_seg<kT>(static_cast<const io_t*>(p.du) + row, tl, L, fast, prev, kWhole);
 #pragma unroll
         for (int j = 0; j < kT; ++j) duv[j] += prev[j];
-        load_seg<kT>(static_cast<const io_t*>(p.ddelta) + row, tl, L, fast, prev);
+        load_seg<kT>(static_cast<const io_t*>(p.ddelta) + row, tl, L, fast, prev, kWhole);
 #pragma unroll
         for (int j = 0; j < kT; ++j) ddv[j] += prev[j];
       }
@@ -504,7 +511,6 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
     if (c > c_lo) stage_chunk<kT, kW, bc_t>(Bb, Cb, N, t0 - kChunk, L, p.bc_sn, dma, stage, tid);
     const size_t nl = static_cast<size_t>(N) * L;
     float* part = p.part_dBC + static_cast<size_t>(blk) * p.part_stride + static_cast<size_t>(b) * 2 * nl;
-    const bool vec_part = (L % 4) == 0;
     for (int task = tid; task < 2 * N * 128; task += kW * 64) {
       // Row (which, n); acc lane ln (segment 63 - ln); steps 4qq..4qq+3 of the segment.
       const int rowi = task >> 7;
@@ -525,14 +531,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       }
       const int t = t0 + (63 - ln) * kT + 4 * qq;
       float* dst = part + which * nl + static_cast<size_t>(n) * L + t;
-      if (vec_part && t + 4 <= L) {
-        const f32x4 x = {v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<f32x4*>(dst) = x;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (t + e < L) dst[e] = v[e];
-      }
+      store_seg<4>(dst - t, t, L, kWhole, v);
     }
     wait_vmem_all();
     __syncthreads();
@@ -594,19 +593,22 @@ __global__ __launch_bounds__(kMsgW * 64) void bwd_msg_kernel(BwdParams p) {
   for (int c = c_hi - 1; c >= c_lo; --c) {
     const int t0 = c * kChunk;
     const int tl = t0 + seg * kT;
-    const bool inside = t0 + kChunk <= L;  // wave-uniform
-    const bool fast = p.vec_io && inside;
-    const bool fast_c = p.vec_bc && inside;
+    const bool fast = t0 + kChunk <= L;  // wave-uniform
     float dlt[kT], g[kT], cv[kT];
-    load_seg<kT>(static_cast<const io_t*>(p.delta) + row, tl, L, fast, dlt);
-    load_seg<kT>(static_cast<const io_t*>(p.dout) + row, tl, L, fast, g);
+    Seg<kT, io_t> sd, sg, sz_;
+    Seg<kT, bc_t> sc;
+    fetch(sd, static_cast<const io_t*>(p.delta) + row, tl, L);
+    fetch(sg, static_cast<const io_t*>(p.dout) + row, tl, L);
+    if constexpr (kHasZ) fetch(sz_, static_cast<const io_t*>(p.z) + row, tl, L);
+    fetch(sc, Cb, tl, L);
+    finish(sd, tl, L, fast, dlt);
+    finish(sg, tl, L, fast, g);
     if constexpr (kHasZ) {
       float zr[kT];
-      load_seg<kT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zr);
+      finish(sz_, tl, L, fast, zr);
 #pragma unroll
       for (int j = 0; j < kT; ++j) g[j] *= zr[j] * sigmoid(zr[j]);
     }
-    load_seg<kT>(Cb, tl, L, fast_c, cv);
 #pragma unroll
     for (int j = 0; j < kT; ++j) dlt[j] += bias;
     if (p.delta_softplus) {
@@ -625,8 +627,8 @@ __global__ __launch_bounds__(kMsgW * 64) void bwd_msg_kernel(BwdParams p) {
     for (int n = 0; n < N; ++n) {
       const float a2 = s_a2[w][n];
       const float q_in = s_q[w][n];
-      float cn[kT];
-      load_seg<kT>(Cb + min(n + 1, N - 1) * p.bc_sn, tl, L, fast_c, cn);
+      finish(sc, tl, L, fast, cv);
+      fetch(sc, Cb + min(n + 1, N - 1) * p.bc_sn, tl, L);
       float lam = 0.f;
 #pragma unroll
       for (int j = kT - 1; j >= 0; --j)
@@ -634,8 +636,6 @@ __global__ __launch_bounds__(kMsgW * 64) void bwd_msg_kernel(BwdParams p) {
       float P = fast_exp2(a2 * ssum);
       wave_scan_affine_fwd(P, lam);  // lane 63 (the chunk's first segment): the whole chunk
       if (lane == 63) s_q[w][n] = __builtin_fmaf(P, q_in, lam);
-#pragma unroll
-      for (int j = 0; j < kT; ++j) cv[j] = cn[j];
     }
   }
   if (lane < N) {
@@ -649,7 +649,7 @@ __global__ __launch_bounds__(kMsgW * 64) void bwd_msg_kernel(BwdParams p) {
 //   blocks [0, n_bc_blocks): dB/dC[b][n][t] = sum over channel blocks of the partials
 //     ([block][b][B|C][n][t], block stride `stride` floats). The block's row is
 //     blockIdx / x_blocks = (b, which, n); threads walk the row's steps, 4 at a time (16-byte
-//     loads) when kVec (L a multiple of 4), keeping kDepth blocks' loads in flight (8 when
+//     loads; the row's last L % 4 steps one by one), keeping kDepth blocks' loads in flight (8 when
 //     there are 64 or more channel blocks: c2's 64 blocks reduce in 14.7 us instead of 17.6
 //     on MI355X; with 32 blocks depth 8 was slower). The sum runs over blocks in order
 //     either way, so both depths give the same bits. With
@@ -658,7 +658,7 @@ __global__ __launch_bounds__(kMsgW * 64) void bwd_msg_kernel(BwdParams p) {
 //   the remaining blocks: dA[d][n] = sum_b part_dA[b][d][n] over the `batch` (times the time
 //     splits) rows of partials (dA rows a_ld apart); dD[d], dbias[d] likewise (dbias added to its current value when acc_bias: a state group of a
 //     wider scan).
-template <bool kVec, typename bc_t, int kDepth>
+template <typename bc_t, int kDepth>
 __global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ part, int n_blk,
                                                      size_t stride, int L, int N, int x_blocks,
                                                      int n_bc_blocks, long long sb, long long sn,
@@ -697,52 +697,62 @@ __global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ p
   const int n = rem - which * N;
   const float* src_row = part + static_cast<size_t>(r) * L;
   bc_t* dst = (which ? dC : dB) + bb * sb + n * sn;
-  constexpr int kE = kVec ? 4 : 1;
-  const int nvec = (L + kE - 1) / kE;
-  // Elements (of kE steps) holding partials; live_part_end is a multiple of 4 or L.
-  const int nlive = seq_lens ? (live_part_end(min(max(seq_lens[bb], 0), L), L) + kE - 1) / kE : nvec;
+  const int nvec = (L + 3) / 4;
+  // Quads holding partials; live_part_end is a multiple of 4 or L.
+  const int nlive = seq_lens ? (live_part_end(min(max(seq_lens[bb], 0), L), L) + 3) / 4 : nvec;
   for (int v = xb * blockDim.x + threadIdx.x; v < nvec; v += x_blocks * blockDim.x) {
-    if (v >= nlive) {
-#pragma unroll
-      for (int e = 0; e < kE; ++e) store_as(dst + kE * v + e, 0.f);
-      continue;
-    }
-    if constexpr (kVec) {
-      const f32x4* src = reinterpret_cast<const f32x4*>(src_row) + v;
-      const size_t svec = stride / 4;
-      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    const float* src = src_row + 4 * v;
+    if (v < nlive && 4 * v + 4 <= L) {
       int k = 0;
       for (; k + kDepth <= n_blk; k += kDepth) {
         f32x4 a[kDepth];
 #pragma unroll
-        for (int q = 0; q < kDepth; ++q) a[q] = src[static_cast<size_t>(k + q) * svec];
+        for (int q = 0; q < kDepth; ++q)
+          a[q] = *reinterpret_cast<const f32x4_any*>(src + static_cast<size_t>(k + q) * stride);
 #pragma unroll
-        for (int q = 0; q < kDepth; ++q) s += a[q];
+        for (int q = 0; q < kDepth; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[e] += a[q][e];
       }
-      for (; k < n_blk; ++k) s += src[static_cast<size_t>(k) * svec];
-      store_as(dst + 4 * v + 0, s.x);
-      store_as(dst + 4 * v + 1, s.y);
-      store_as(dst + 4 * v + 2, s.z);
-      store_as(dst + 4 * v + 3, s.w);
-    } else {
-      float s = 0.f;
-      for (int k = 0; k < n_blk; ++k) s += src_row[static_cast<size_t>(k) * stride + v];
-      store_as(dst + v, s);
+      for (; k < n_blk; ++k) {
+        const f32x4 a = *reinterpret_cast<const f32x4_any*>(src + static_cast<size_t>(k) * stride);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += a[e];
+      }
+    } else if (v < nlive) {
+      // The row's last steps: clamped indexes, so that no load waits for a branch.
+#pragma unroll 2
+      for (int k = 0; k < n_blk; ++k) {
+        const float* at = src + static_cast<size_t>(k) * stride;
+#pragma unroll
+        for (int e = 0; e < 3; ++e) s[e] += at[min(e, L - 1 - 4 * v)];
+      }
     }
+    store_seg<4>(dst, 4 * v, L, false, s);
   }
+}
+
+template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup, bool kWhole>
+static hipError_t launch_bwd_w(const BwdParams& p, hipStream_t stream) {
+  dim3 grid(p.n_blocks_d, p.batch, p.n_split);
+  if (p.waves == 16) {
+    if (!bwd_waves_fit(16, p.dstate) || p.chan_per_block % 16 != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((bwd_kernel<16, kZOH, kHasZ, io_t, bc_t, kGroup, kWhole>), grid, dim3(16 * 64), 0, stream, p);
+  } else {
+    if (p.waves != 12 || p.chan_per_block % 12 != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((bwd_kernel<12, kZOH, kHasZ, io_t, bc_t, kGroup, kWhole>), grid, dim3(12 * 64), 0, stream, p);
+  }
+  return hipGetLastError();
 }
 
 template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup>
 static hipError_t launch_bwd_a(const BwdParams& p, hipStream_t stream) {
-  dim3 grid(p.n_blocks_d, p.batch, p.n_split);
-  if (p.waves == 16) {
-    if (!bwd_waves_fit(16, p.dstate) || p.chan_per_block % 16 != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((bwd_kernel<16, kZOH, kHasZ, io_t, bc_t, kGroup>), grid, dim3(16 * 64), 0, stream, p);
-  } else {
-    if (p.waves != 12 || p.chan_per_block % 12 != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((bwd_kernel<12, kZOH, kHasZ, io_t, bc_t, kGroup>), grid, dim3(12 * 64), 0, stream, p);
+  if constexpr (kGroup == 0 && sizeof(io_t) == sizeof(bc_t)) {
+    if (p.vec_bc && p.seqlen % kBwdChunk == 0)
+      return launch_bwd_w<kZOH, kHasZ, io_t, bc_t, kGroup, true>(p, stream);
   }
-  return hipGetLastError();
+  return launch_bwd_w<kZOH, kHasZ, io_t, bc_t, kGroup, false>(p, stream);
 }
 
 template <bool kZOH, bool kHasZ, typename io_t, typename bc_t>
@@ -864,24 +874,23 @@ hipError_t launch_bwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16
 hipError_t launch_bwd_reduce(const BwdParams& p, int bc_bf16, int a_width, int a_ld, int acc_bias,
                              void* dA, void* dB, void* dC, float* dD, float* dbias, hipStream_t stream) {
   const int L = p.seqlen;
-  const bool vec = (L % 4) == 0;  // partial rows are 16-byte aligned (block stride: 64 floats)
-  const int nvec = vec ? L / 4 : L;
+  const int nvec = (L + 3) / 4;
   const int x_blocks = (nvec + 255) / 256;
   const int n_bc_blocks = x_blocks * p.batch * 2 * p.dstate;
   const int small = p.dim * a_width + 2 * p.dim;
   const dim3 grid(n_bc_blocks + (small + 255) / 256);
   const bool deep = p.n_blocks_d >= 64;
-#define MSS_REDUCE(VEC, T)                                                                       \
-  hipLaunchKernelGGL((deep ? reduce_kernel<VEC, T, 8> : reduce_kernel<VEC, T, 4>), grid, dim3(256), \
+#define MSS_REDUCE(T)                                                                       \
+  hipLaunchKernelGGL((deep ? reduce_kernel<T, 8> : reduce_kernel<T, 4>), grid, dim3(256), \
                      0, stream, p.part_dBC, p.n_blocks_d,                                          \
                      p.part_stride, L, p.dstate, x_blocks, n_bc_blocks, p.bc_sb, p.bc_sn,          \
                      static_cast<T*>(dB), static_cast<T*>(dC), p.part_dA, p.part_dD, p.part_dbias,  \
                      p.batch * p.n_split, p.dim, a_width, a_ld, acc_bias, static_cast<float*>(dA), dD, dbias, \
                      p.seq_lens)
   if (bc_bf16) {
-    if (vec) MSS_REDUCE(true, bf16_t); else MSS_REDUCE(false, bf16_t);
+    MSS_REDUCE(bf16_t);
   } else {
-    if (vec) MSS_REDUCE(true, float); else MSS_REDUCE(false, float);
+    MSS_REDUCE(float);
   }
 #undef MSS_REDUCE
   return hipGetLastError();

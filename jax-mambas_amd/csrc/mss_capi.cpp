@@ -233,8 +233,7 @@ int run_fwd(const mss_fwd_args* a, float* ref_states, hipStream_t stream, bool c
   p.bc_sn = st.bc_sn;
   const size_t io_e = dtype_size(a->io_dtype), bc_e = dtype_size(a->bc_dtype);
   const size_t bc_row = static_cast<size_t>(a->seqlen) * bc_e;
-  p.vec_io = strides_aligned(st.io_sb, st.io_sd, io_e) && aligned16(a->u) && aligned16(a->delta) &&
-             aligned16(a->z) && aligned16(a->out) && aligned16(a->y_pre);
+  p.vec_z = strides_aligned(st.io_sb, st.io_sd, io_e) && aligned16(a->z);
   // B/C staging also needs L to be a multiple of the 16-byte slot width.
   p.vec_bc = (bc_row % 16 == 0) && strides_aligned(st.bc_sb, st.bc_sn, bc_e) && aligned16(a->B) &&
              aligned16(a->C);
@@ -277,11 +276,8 @@ mss::BwdParams pack_bwd(const mss_bwd_args* a, const BwdLayout& l, char* ws) {
   p.io_sd = st.io_sd;
   p.bc_sb = st.bc_sb;
   p.bc_sn = st.bc_sn;
-  const size_t io_e = dtype_size(a->io_dtype), bc_e = dtype_size(a->bc_dtype);
+  const size_t bc_e = dtype_size(a->bc_dtype);
   const size_t bc_row = static_cast<size_t>(a->seqlen) * bc_e;
-  p.vec_io = strides_aligned(st.io_sb, st.io_sd, io_e) && aligned16(a->u) && aligned16(a->delta) &&
-             aligned16(a->z) && aligned16(a->dout) && aligned16(a->du) && aligned16(a->ddelta) &&
-             aligned16(a->dz) && aligned16(a->y_pre) && aligned16(a->out);
   p.vec_bc = (bc_row % 16 == 0) && strides_aligned(st.bc_sb, st.bc_sn, bc_e) && aligned16(a->B) &&
              aligned16(a->C);
   p.n_seg = n_seg_of(a->seqlen);
@@ -1245,9 +1241,6 @@ int mss_scan_bwd_ws(void* stream, int32_t batch, int32_t length, int32_t dim, in
   p.dim = dim;
   p.seqlen = length;
   p.dstate = dstate;
-  const size_t row = static_cast<size_t>(length) * sizeof(float);
-  p.vec_io = (row % 16 == 0) && aligned16(u) && aligned16(deltas);
-  p.vec_bc = (row % 16 == 0) && aligned16(B);
   p.n_seg = n_seg_of(length);
   p.n_ref = (length + MSS_REF_CHUNK - 1) / MSS_REF_CHUNK;
   p.u = u;

@@ -170,71 +170,136 @@ __device__ __forceinline__ float sigmoid(float x) {
 
 // ---------------------------------------------------------------------------------
 // Segment loads/stores. `row` points at element 0 of a [..][L] row; the segment is
-// elements [t, t+N). `fast` must be wave-uniform: true when 16-byte vector access is
-// legal for the row and the whole wave's chunk lies inside [0, L); otherwise elements at
-// or beyond `L` read as 0 and are not written.
-template <int N>
-__device__ __forceinline__ void load_seg(const float* __restrict__ row, int t, int L, bool fast,
-                                         float (&v)[N]) {
-  if (fast) {
-    const f32x4* p = reinterpret_cast<const f32x4*>(row + t);
+// elements [t, t+N). `fast` must be wave-uniform: true when the whole wave's chunk lies inside
+// [0, L). Elements at or beyond `L` read as 0 and are not written. Rows need only their
+// elements' alignment: the 16-byte accesses of gfx950 take any address.
+//
+// A load is two calls: fetch() only issues it, finish() turns what arrived into floats, so that
+// a wave's several rows are fetched together and waited for once. A segment that crosses the
+// row's end is fetched as the row's last N elements and moved into place by finish(): the same
+// one load per 16 bytes for every lane, whatever L is (rows shorter than N: element by element).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+
+template <int N, typename T>
+struct Seg {  // the segment's bytes as 32-bit words
+  static constexpr int kWords = N * static_cast<int>(sizeof(T)) / 4;
+  uint32_t w[kWords];
+};
+
+template <int kWords>
+__device__ __forceinline__ void load_words(const float* __restrict__ src, uint32_t (&w)[kWords]) {
+  const f32x4_any* p = reinterpret_cast<const f32x4_any*>(src);
 #pragma unroll
-    for (int q = 0; q < N / 4; ++q) {
-      const f32x4 x = p[q];
-      v[4 * q + 0] = x.x;
-      v[4 * q + 1] = x.y;
-      v[4 * q + 2] = x.z;
-      v[4 * q + 3] = x.w;
-    }
-  } else {
+  for (int q = 0; q < kWords / 4; ++q) {
+    const f32x4 x = p[q];
+    w[4 * q + 0] = __float_as_uint(x.x);
+    w[4 * q + 1] = __float_as_uint(x.y);
+    w[4 * q + 2] = __float_as_uint(x.z);
+    w[4 * q + 3] = __float_as_uint(x.w);
+  }
+}
+template <int kWords>
+__device__ __forceinline__ void load_words(const bf16_t* __restrict__ src, uint32_t (&w)[kWords]) {
+  const u32x4_any* p = reinterpret_cast<const u32x4_any*>(src);
 #pragma unroll
-    for (int j = 0; j < N; ++j) v[j] = (t + j < L) ? row[t + j] : 0.f;
+  for (int q = 0; q < kWords / 4; ++q) {
+    const u32x4 x = p[q];
+    w[4 * q + 0] = x.x;
+    w[4 * q + 1] = x.y;
+    w[4 * q + 2] = x.z;
+    w[4 * q + 3] = x.w;
   }
 }
 
-template <int N>
-__device__ __forceinline__ void load_seg(const bf16_t* __restrict__ row, int t, int L, bool fast,
-                                         float (&v)[N]) {
-  if (fast) {
-    const u32x4* p = reinterpret_cast<const u32x4*>(row + t);
+// whole: known at compile time to lie inside the row.
+template <int N, typename T>
+__device__ __forceinline__ void fetch(Seg<N, T>& s, const T* __restrict__ row, int t, int L, bool whole = false) {
+  if (whole) {
+    load_words(row + t, s.w);
+  } else if (L >= N) {  // uniform
+    load_words(row + min(t, L - N), s.w);
+  } else {
 #pragma unroll
-    for (int q = 0; q < N / 8; ++q) {
-      const u32x4 x = p[q];
-      const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+    for (int k = 0; k < Seg<N, T>::kWords; ++k) s.w[k] = 0;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[8 * q + 2 * k + 0] = __uint_as_float(w[k] << 16);
-        v[8 * q + 2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
+    for (int j = 0; j < N; ++j) {
+      if (t + j < L) {
+        if constexpr (sizeof(T) == 4)
+          s.w[j] = __float_as_uint(row[t + j]);
+        else
+          s.w[j / 2] |= static_cast<uint32_t>(row[t + j].bits) << (16 * (j & 1));
       }
     }
-  } else {
-#pragma unroll
-    for (int j = 0; j < N; ++j) v[j] = (t + j < L) ? to_f32(row[t + j]) : 0.f;
   }
 }
 
-template <int N>
-__device__ __forceinline__ void store_seg(float* __restrict__ row, int t, int L, bool fast,
-                                          const float (&v)[N]) {
-  if (fast) {
-    f32x4* p = reinterpret_cast<f32x4*>(row + t);
+// The segment's words moved down by the elements its fetch started before t (zeros from the top).
+template <int N, typename T>
+__device__ __forceinline__ void shift_to(Seg<N, T>& s, int t, int L) {
+  constexpr int kWords = Seg<N, T>::kWords;
+  const int by = L >= N ? max(0, t - (L - N)) : 0;
+  if constexpr (sizeof(T) == 2) {
 #pragma unroll
-    for (int q = 0; q < N / 4; ++q) {
-      const f32x4 x = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-      p[q] = x;
+    for (int k = 0; k < kWords; ++k) {
+      const uint32_t hi = k + 1 < kWords ? s.w[k + 1] : 0u;
+      s.w[k] = (by & 1) ? (s.w[k] >> 16) | (hi << 16) : s.w[k];
     }
+  }
+  constexpr int kPer = 4 / static_cast<int>(sizeof(T));  // elements per word
+#pragma unroll
+  for (int m = 1; m < kWords; m *= 2) {
+#pragma unroll
+    for (int k = 0; k < kWords; ++k) {
+      const uint32_t up = k + m < kWords ? s.w[k + m] : 0u;
+      s.w[k] = (by & (m * kPer)) ? up : s.w[k];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kWords; ++k) s.w[k] = by >= N ? 0u : s.w[k];
+}
+
+template <int N, typename T>
+__device__ __forceinline__ void finish(Seg<N, T>& s, int t, int L, bool fast, float (&v)[N]) {
+  if (!fast) shift_to(s, t, L);
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] = __uint_as_float(s.w[j]);
   } else {
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-      if (t + j < L) row[t + j] = v[j];
+    for (int k = 0; k < N / 2; ++k) {
+      v[2 * k + 0] = __uint_as_float(s.w[k] << 16);
+      v[2 * k + 1] = __uint_as_float(s.w[k] & 0xffff0000u);
+    }
+  }
+}
+
+template <int N, typename T>
+__device__ __forceinline__ void load_seg(const T* __restrict__ row, int t, int L, bool fast, float (&v)[N],
+                                         bool whole = false) {
+  Seg<N, T> s;
+  fetch(s, row, t, L, whole);
+  finish(s, t, L, fast, v);
+}
+
+template <int N>
+__device__ __forceinline__ void store_vec(float* __restrict__ dst, const float (&v)[N]) {
+  f32x4_any* p = reinterpret_cast<f32x4_any*>(dst);
+#pragma unroll
+  for (int q = 0; q < N / 4; ++q) {
+    const f32x4 x = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    p[q] = x;
   }
 }
 
 template <int N>
-__device__ __forceinline__ void store_seg(bf16_t* __restrict__ row, int t, int L, bool fast,
-                                          const float (&v)[N]) {
-  if (fast) {
-    u32x4* p = reinterpret_cast<u32x4*>(row + t);
+__device__ __forceinline__ void store_vec(bf16_t* __restrict__ dst, const float (&v)[N]) {
+  if constexpr (N == 4) {
+    const u32x2_any x = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    *reinterpret_cast<u32x2_any*>(dst) = x;
+  } else {
+    u32x4_any* p = reinterpret_cast<u32x4_any*>(dst);
 #pragma unroll
     for (int q = 0; q < N / 8; ++q) {
       uint32_t w[4];
@@ -243,6 +308,13 @@ __device__ __forceinline__ void store_seg(bf16_t* __restrict__ row, int t, int L
       const u32x4 x = {w[0], w[1], w[2], w[3]};
       p[q] = x;
     }
+  }
+}
+
+template <int N, typename T>
+__device__ __forceinline__ void store_seg(T* __restrict__ row, int t, int L, bool fast, const float (&v)[N]) {
+  if (fast || t + N <= L) {
+    store_vec<N>(row + t, v);
   } else {
 #pragma unroll
     for (int j = 0; j < N; ++j)
@@ -270,6 +342,15 @@ template <typename bc_t>
 struct BcStage {
   static constexpr int kElemsPerSlot = 16 / static_cast<int>(sizeof(bc_t));
 };
+
+// The 16-byte slot of a row's elements [e, e + kElemsPerSlot), zero from L on; any alignment.
+template <typename T>
+__device__ __forceinline__ uint4 load_slot(const T* __restrict__ row, int e, int L, bool fast) {
+  Seg<BcStage<T>::kElemsPerSlot, T> s;
+  fetch(s, row, e, L);
+  if (!fast) shift_to(s, e, L);
+  return make_uint4(s.w[0], s.w[1], s.w[2], s.w[3]);
+}
 
 // Read lane `lane`'s kT staged values of one row (fp32 or bf16 in LDS) as floats.
 template <int kT, typename bc_t>
@@ -479,8 +560,8 @@ struct ConvParams {
 struct FwdParams {
   int batch, dim, seqlen, dstate;
   int delta_softplus;
-  int vec_io;  // 16-byte vector access legal for u/delta/z/out rows
-  int vec_bc;  // ... for B/C rows
+  int vec_z;   // z rows are 16-byte aligned (direct-to-LDS copies)
+  int vec_bc;  // B/C rows are, and L is a multiple of 16 bytes of them
   int n_seg;  // ceil(L / kSegSteps): carries row length
   int n_ref;    // ceil(L / 2048)
   long long io_sb, io_sd;  // row strides (elements) of u/delta/z/out/y_pre: batch, channel
@@ -520,7 +601,7 @@ struct BwdPlan {
 struct BwdParams {
   int batch, dim, seqlen, dstate;
   int delta_softplus;
-  int vec_io, vec_bc;
+  int vec_bc;  // B/C rows are 16-byte aligned and L a multiple of 16 bytes of them (direct-to-LDS copies)
   int n_seg;
   int waves;           // waves per backward workgroup (12 or 16)
   int chan_per_block;  // channels one workgroup walks (multiple of the wave count)

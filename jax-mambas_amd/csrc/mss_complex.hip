@@ -110,7 +110,7 @@ __device__ __forceinline__ void wave_scan_caffine(float& pr, float& pi, float& h
 // ---------------------------------------------------------------------------------
 // Forward. Workgroup = kCFwdW channels of one batch row; no LDS, no block barriers. The
 // running state of state n (entering the current chunk) is kept by lane n as (run_r, run_i).
-template <bool kZOH, typename io_t, typename bc_t>
+template <bool kZOH, typename io_t, typename bc_t, bool kWhole>
 __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -140,8 +140,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
   for (int c = 0; c < n_chunks; ++c) {
     const int t0 = c * kCChunk;
     const int tl = t0 + lane * kCT;
-    const bool fast = p.vec_io && t0 + kCChunk <= L;
-    const bool fast_bc = p.vec_bc && t0 + kCChunk <= L;
+    const bool fast = kWhole || t0 + kCChunk <= L;
     float y[kCT];
     if (c >= n_live) {
       // The whole chunk is past this row's length: the state is frozen, the output zero
@@ -153,8 +152,11 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
     }
     float dlt[kCT], uu[kCT];
     float ssum = 0.f;
-    load_seg<kCT>(dl_row, tl, L, fast, dlt);
-    load_seg<kCT>(u_row, tl, L, fast, uu);
+    Seg<kCT, io_t> sd, su;
+    fetch(sd, dl_row, tl, L, kWhole);
+    fetch(su, u_row, tl, L, kWhole);
+    finish(sd, tl, L, fast, dlt);
+    finish(su, tl, L, fast, uu);
 #pragma unroll
     for (int j = 0; j < kCT; ++j) {
       const bool valid = tl + j < len;
@@ -166,21 +168,18 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
       ssum += dlt[j];
     }
     // B and C rows of the next state are loaded one state ahead.
-    float bnx[kCT], cnx[kCT];
-    load_seg<kCT>(Bb, tl, L, fast_bc, bnx);
-    load_seg<kCT>(Cb, tl, L, fast_bc, cnx);
+    Seg<kCT, bc_t> sbn, scn;
+    fetch(sbn, Bb, tl, L, kWhole);
+    fetch(scn, Cb, tl, L, kWhole);
     for (int n = 0; n < N; ++n) {
       const CoefA cf = load_coef(p.A, static_cast<size_t>(d) * N + n);
       float ar[kCT], ai[kCT], br[kCT], bi[kCT];
       float bv[kCT], cv[kCT];
-#pragma unroll
-      for (int j = 0; j < kCT; ++j) {
-        bv[j] = bnx[j];
-        cv[j] = cnx[j];
-      }
+      finish(sbn, tl, L, fast, bv);
+      finish(scn, tl, L, fast, cv);
       if (n + 1 < N) {
-        load_seg<kCT>(Bb + (n + 1) * p.bc_sn, tl, L, fast_bc, bnx);
-        load_seg<kCT>(Cb + (n + 1) * p.bc_sn, tl, L, fast_bc, cnx);
+        fetch(sbn, Bb + (n + 1) * p.bc_sn, tl, L, kWhole);
+        fetch(scn, Cb + (n + 1) * p.bc_sn, tl, L, kWhole);
       }
       float hr = 0.f, hi = 0.f;
       {
@@ -220,7 +219,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
         xr = rr;
         xi = ri;
       }
-      if (p.carries && tl < L) {
+      if (p.carries && (kWhole || tl < L)) {
         float2* cp = reinterpret_cast<float2*>(p.carries) + (chan * N + n) * p.n_seg + tl / kCT;
         *cp = make_float2(xr, xi);
       }
@@ -246,7 +245,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
         store_seg<kCT>(static_cast<io_t*>(p.y_pre) + row, tl, L, fast, yp);
       }
       float zv[kCT];
-      load_seg<kCT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zv);
+      load_seg<kCT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zv, kWhole);
 #pragma unroll
       for (int j = 0; j < kCT; ++j) y[j] *= zv[j] * sigmoid(zv[j]);
     }
@@ -273,7 +272,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
 // counted that iteration done in LDS (no workgroup barrier per iteration). After every
 // chunk the rows (copies summed in order) go to this workgroup's partial rows; a second
 // kernel sums the partials over workgroups in a fixed order.
-template <bool kZOH, bool kHasZ, typename io_t, typename bc_t>
+template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, bool kWhole>
 __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
   constexpr int W = kCBwdW;
   __shared__ __attribute__((aligned(16))) float s_acc[kCAccRows][2][kCChunk];
@@ -329,8 +328,7 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
   for (int c = n_chunks - 1; c >= 0; --c) {
     const int t0 = c * kCChunk;
     const int ts = t0 + seg * kCT;
-    const bool fast = p.vec_io && t0 + kCChunk <= L;
-    const bool fast_bc = p.vec_bc && t0 + kCChunk <= L;
+    const bool fast = kWhole || t0 + kCChunk <= L;
     const bool live = c < n_live;  // workgroup-uniform
     for (int r = 0; r < rounds; ++r) {
       const int k = r * W + w;
@@ -356,9 +354,17 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
       const float Dv = p.D ? p.D[dd] : 0.f;
       const float bias = p.delta_bias ? p.delta_bias[dd] : 0.f;
       float xraw[kCT], dlt[kCT], uu[kCT], g[kCT];
-      load_seg<kCT>(static_cast<const io_t*>(p.delta) + row, ts, L, fast, xraw);
-      load_seg<kCT>(static_cast<const io_t*>(p.u) + row, ts, L, fast, uu);
-      load_seg<kCT>(static_cast<const io_t*>(p.dout) + row, ts, L, fast, g);
+      Seg<kCT, io_t> sd, su, sg, sz_, sy;
+      fetch(sd, static_cast<const io_t*>(p.delta) + row, ts, L, kWhole);
+      fetch(su, static_cast<const io_t*>(p.u) + row, ts, L, kWhole);
+      fetch(sg, static_cast<const io_t*>(p.dout) + row, ts, L, kWhole);
+      if constexpr (kHasZ) {
+        fetch(sz_, static_cast<const io_t*>(p.z) + row, ts, L, kWhole);
+        fetch(sy, static_cast<const io_t*>(p.y_pre) + row, ts, L, kWhole);
+      }
+      finish(sd, ts, L, fast, xraw);
+      finish(su, ts, L, fast, uu);
+      finish(sg, ts, L, fast, g);
       float ssum = 0.f;
 #pragma unroll
       for (int j = 0; j < kCT; ++j) {
@@ -372,8 +378,8 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
       }
       if constexpr (kHasZ) {
         float zv[kCT], yp[kCT], dz[kCT];
-        load_seg<kCT>(static_cast<const io_t*>(p.z) + row, ts, L, fast, zv);
-        load_seg<kCT>(static_cast<const io_t*>(p.y_pre) + row, ts, L, fast, yp);
+        finish(sz_, ts, L, fast, zv);
+        finish(sy, ts, L, fast, yp);
 #pragma unroll
         for (int j = 0; j < kCT; ++j) {
           const float sz = sigmoid(zv[j]);
@@ -395,13 +401,13 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
       constexpr bool kAhead = !kZOH;
       const float2* __restrict__ carry_seg = reinterpret_cast<const float2*>(p.carries) +
                                              chan * N * p.n_seg + ts / kCT;
-      float bnx[kCT], cnx[kCT];
+      Seg<kCT, bc_t> sbn, scn;
       float2 hnx = make_float2(0.f, 0.f);
       if (kAhead && active) {
         const int n0 = w % N;
-        load_seg<kCT>(Bb + n0 * p.bc_sn, ts, L, fast_bc, bnx);
-        load_seg<kCT>(Cb + n0 * p.bc_sn, ts, L, fast_bc, cnx);
-        if (ts < L) hnx = carry_seg[static_cast<size_t>(n0) * p.n_seg];
+        fetch(sbn, Bb + n0 * p.bc_sn, ts, L, kWhole);
+        fetch(scn, Cb + n0 * p.bc_sn, ts, L, kWhole);
+        if (kWhole || ts < L) hnx = carry_seg[static_cast<size_t>(n0) * p.n_seg];
       }
       for (int it = 0; it < N; ++it) {
         const int n = (it + w) % N;
@@ -411,23 +417,20 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
           float bv[kCT], cv[kCT];
           float hinr, hini;
           if constexpr (kAhead) {
-#pragma unroll
-            for (int j = 0; j < kCT; ++j) {
-              bv[j] = bnx[j];
-              cv[j] = cnx[j];
-            }
+            finish(sbn, ts, L, fast, bv);
+            finish(scn, ts, L, fast, cv);
             hinr = hnx.x;
             hini = hnx.y;
             if (it + 1 < N) {
               const int nn = (it + 1 + w) % N;
-              load_seg<kCT>(Bb + nn * p.bc_sn, ts, L, fast_bc, bnx);
-              load_seg<kCT>(Cb + nn * p.bc_sn, ts, L, fast_bc, cnx);
-              if (ts < L) hnx = carry_seg[static_cast<size_t>(nn) * p.n_seg];
+              fetch(sbn, Bb + nn * p.bc_sn, ts, L, kWhole);
+              fetch(scn, Cb + nn * p.bc_sn, ts, L, kWhole);
+              if (kWhole || ts < L) hnx = carry_seg[static_cast<size_t>(nn) * p.n_seg];
             }
           } else {
-            load_seg<kCT>(Bb + n * p.bc_sn, ts, L, fast_bc, bv);
-            load_seg<kCT>(Cb + n * p.bc_sn, ts, L, fast_bc, cv);
-            const float2 h0 = ts < L ? carry_seg[static_cast<size_t>(n) * p.n_seg] : make_float2(0.f, 0.f);
+            load_seg<kCT>(Bb + n * p.bc_sn, ts, L, fast, bv, kWhole);
+            load_seg<kCT>(Cb + n * p.bc_sn, ts, L, fast, cv, kWhole);
+            const float2 h0 = kWhole || ts < L ? carry_seg[static_cast<size_t>(n) * p.n_seg] : make_float2(0.f, 0.f);
             hinr = h0.x;
             hini = h0.y;
           }
@@ -712,7 +715,13 @@ hipError_t launch_cssm_step(const StepParams& p, bool zoh, bool io_bf16, bool bc
 template <bool kZOH, typename io_t, typename bc_t>
 static hipError_t launch_cfwd_t(const FwdParams& p, hipStream_t stream) {
   dim3 grid((p.dim + kCFwdW - 1) / kCFwdW, p.batch);
-  hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t>), grid, dim3(kCFwdW * 64), 0, stream, p);
+  if constexpr (sizeof(io_t) == sizeof(bc_t)) {
+    if (p.seqlen % kCChunk == 0) {
+      hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, true>), grid, dim3(kCFwdW * 64), 0, stream, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, false>), grid, dim3(kCFwdW * 64), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -743,7 +752,13 @@ int cbwd_chan_per_block(int batch, int dim) {
 template <bool kZOH, bool kHasZ, typename io_t, typename bc_t>
 static hipError_t launch_cbwd_t(const BwdParams& p, hipStream_t stream) {
   dim3 grid(p.n_blocks_d, p.batch);
-  hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t>), grid, dim3(kCBwdW * 64), 0, stream, p);
+  if constexpr (sizeof(io_t) == sizeof(bc_t)) {
+    if (p.seqlen % kCChunk == 0) {
+      hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t, true>), grid, dim3(kCBwdW * 64), 0, stream, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t, false>), grid, dim3(kCBwdW * 64), 0, stream, p);
   return hipGetLastError();
 }
 

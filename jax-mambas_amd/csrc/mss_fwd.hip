@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kRebuildW * 64) void carry_rebuild_kernel(FwdParams
   const int c_end = min((L + kChunk - 1) / kChunk, (blk + 1) * kChunksPerBlock);
   for (int c = blk * kChunksPerBlock; c < c_end; ++c) {
     const int tl = c * kChunk + lane * kT;
-    const bool fast = p.vec_io && c * kChunk + kChunk <= L;
+    const bool fast = c * kChunk + kChunk <= L;
     float dlt[kT], dlu[kT];
     load_seg<kT>(dl_row, tl, L, fast, dlt);
     load_seg<kT>(u_row, tl, L, fast, dlu);
@@ -80,15 +80,14 @@ __global__ __launch_bounds__(kRebuildW * 64) void carry_rebuild_kernel(FwdParams
       ssum += dlt[j];
     }
     const int seg_idx = tl / kT;
-    const bool fast_b = fast && p.vec_bc;
     // B rows one state ahead: the next state's load is in flight while this one computes.
     float bv[kT];
-    load_seg<kT>(Bb, tl, L, fast_b, bv);
+    load_seg<kT>(Bb, tl, L, fast, bv);
     for (int n = 0; n < N; ++n) {
       const float a2 = s_a2[w][n];
       const float run = s_run[w][n];
       float bn[kT];
-      if (n + 1 < N) load_seg<kT>(Bb + static_cast<size_t>(n + 1) * L, tl, L, fast_b, bn);
+      if (n + 1 < N) load_seg<kT>(Bb + static_cast<size_t>(n + 1) * L, tl, L, fast, bn);
       float H = 0.f;
 #pragma unroll
       for (int j = 0; j < kT; ++j) H = __builtin_fmaf(fast_exp2(dlt[j] * a2), H, dlu[j] * bv[j]);

@@ -64,31 +64,25 @@ __device__ __forceinline__ void stage_round(const bc_t* __restrict__ Bb, const b
       __builtin_amdgcn_global_load_lds((gbl_void_t)src, (lds_void_t)(&dst[k][which][s0]), 16, 0, 0);
     }
   } else {
-    for (int f = tid; f < nb * 2 * 64 * kT; f += kW * 64) {
-      const int rowi = f / (64 * kT);
+    const bool fast = t0 + 64 * kT <= L;
+    for (int f = tid; f < total; f += kW * 64) {
+      const int rowi = f / kSlots;
       const int k = rowi >> 1;
       const int which = rowi & 1;
-      const int e = f - rowi * 64 * kT;
-      const int i = e / kT;
-      const int r = e % kT;
-      const int q = r / kE;
-      const int sl = kQ * i + (q ^ slot_swz<kQ>(i));
-      const int t = t0 + e;
-      const bc_t* src = (which ? Cb : Bb) + (n0 + k) * sn;
-      bc_t v;
-      if (t < L) {
-        v = src[t];
-      } else {
-        store_as(&v, 0.f);
-      }
-      reinterpret_cast<bc_t*>(&dst[k][which][0])[sl * kE + (r % kE)] = v;
+      const int s = f - rowi * kSlots;
+      const int i = s / kQ;
+      const int q = (s % kQ) ^ slot_swz<kQ>(i);
+      dst[k][which][s] = load_slot((which ? Cb : Bb) + (n0 + k) * sn, t0 + i * kT + q * kE, L, fast);
     }
   }
 }
 
 // kMaxS: the per-wave state tables' size (kMaxN, or kMaxNWide for float32 scans with more
-// states).
-template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS = kMaxN>
+// states). kWhole: L is a multiple of the chunk and the B/C rows can be copied to LDS directly,
+// so no lane ever meets the row's end (the paths that handle it spill registers: B=8 D=2560
+// L=4096 float32 with lengths 306 us, the general instance 351). The general instance takes
+// B=3 D=1000 L=2051 bf16 in 92 us; element-wise accesses to such rows took 146.
+template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS, bool kWhole>
 __global__ __launch_bounds__(kW * 64) __attribute__((amdgpu_waves_per_eu(kOcc, kOcc)))
 void fwd_kernel(FwdParams p) {
   constexpr int kChunk = 64 * kT;
@@ -137,8 +131,7 @@ void fwd_kernel(FwdParams p) {
   }
   const float Dv = p.D ? p.D[d] : 0.f;
   const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
-  const bool vec_io = p.vec_io != 0;
-  const bool dma = p.vec_bc != 0;
+  const bool dma = kWhole || p.vec_bc != 0;
   float dsum_total = 0.f;  // sum of delta over all finished steps (reference residual)
 
   const int n_chunks = (L + kChunk - 1) / kChunk;
@@ -157,7 +150,7 @@ void fwd_kernel(FwdParams p) {
   for (int c = 0; c < n_chunks; ++c) {
     const int t0 = c * kChunk;
     const int tl = t0 + lane * kT;
-    const bool fast = vec_io && (t0 + kChunk <= L);  // wave-uniform
+    const bool fast = kWhole || t0 + kChunk <= L;  // wave-uniform
     // Reference residual slot written at this chunk's end (2048-step boundary or end of
     // the sequence), -1 if none.
     const int chunk_end = t0 + kChunk;
@@ -188,12 +181,13 @@ void fwd_kernel(FwdParams p) {
 
     float dlt[kT], dlu[kT], y[kT];
     float ssum = 0.f;
-    // z through LDS for whole vectorisable chunks (wave-uniform); the first round barrier's
+    // z through LDS for whole chunks of aligned rows (wave-uniform); the first round barrier's
     // wait covers the copies.
-    const bool z_lds = kZLds && active && fast && p.z != nullptr && p.out != nullptr;
+    const bool z_lds = kZLds && active && fast && p.vec_z && p.z != nullptr && p.out != nullptr;
     if (active) {
-      load_seg<kT>(dl_row, tl, L, fast, dlt);
-      load_seg<kT>(u_row, tl, L, fast, y);
+      Seg<kT, io_t> sd, su;
+      fetch(sd, dl_row, tl, L, kWhole);
+      fetch(su, u_row, tl, L, kWhole);
       if (kZLds && z_lds) {
         const io_t* zsrc = static_cast<const io_t*>(p.z) + row + tl;
 #pragma unroll
@@ -201,6 +195,8 @@ void fwd_kernel(FwdParams p) {
           __builtin_amdgcn_global_load_lds((gbl_void_t)(zsrc + q * (16 / static_cast<int>(sizeof(io_t)))),
                                            (lds_void_t)(&s_z[w][q * 64]), 16, 0, 0);
       }
+      finish(sd, tl, L, fast, dlt);
+      finish(su, tl, L, fast, y);
 #pragma unroll
       for (int j = 0; j < kT; ++j) {
         const bool valid = tl + j < len;
@@ -262,7 +258,7 @@ void fwd_kernel(FwdParams p) {
             float* crow = p.carries + (chan * N + n) * p.n_seg + tl / kSegSteps;
 #pragma unroll
             for (int q = 0; q < kT / kSegSteps; ++q)
-              if (tl / kSegSteps + q < p.n_seg) crow[q] = hseg[q];
+              if (kWhole || tl / kSegSteps + q < p.n_seg) crow[q] = hseg[q];
           }
         }
         const float run_new = readlane(hend, 63);
@@ -316,7 +312,7 @@ void fwd_kernel(FwdParams p) {
             }
           }
         } else {
-          load_seg<kT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zv);
+          load_seg<kT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zv, kWhole);
         }
         if (p.y_pre) {
           // The backward takes y sigma(z) from out / z; y itself is kept only where z is too
@@ -339,7 +335,13 @@ void fwd_kernel(FwdParams p) {
 template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS = kMaxN>
 static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   dim3 grid((p.dim + kW - 1) / kW, p.batch);
-  hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS>), grid, dim3(kW * 64), 0, stream, p);
+  if constexpr (kMaxS == kMaxN && sizeof(io_t) == sizeof(bc_t)) {
+    if (p.vec_bc && p.seqlen % (64 * kT) == 0) {
+      hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, true>), grid, dim3(kW * 64), 0, stream, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, false>), grid, dim3(kW * 64), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -362,9 +364,11 @@ static hipError_t launch_fwd_z(const FwdParams& p, hipStream_t stream) {
   // B=8 D=1536 L=2048 167 vs 175 us wide vs narrow).
   constexpr long long kNarrowSlots = 256LL * MSS_FWD_OCC_NARROW * 4 / MSS_FWD_W;
   const long long groups = static_cast<long long>(p.batch) * ((p.dim + MSS_FWD_W - 1) / MSS_FWD_W);
-  if (sizeof(io_t) == 4 || groups <= kNarrowSlots)
-    return launch_fwd_t<MSS_FWD_T_NARROW, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_NARROW, kZOH, io_t, bc_t>(p, stream);
-  return launch_fwd_t<MSS_FWD_T_WIDE, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_WIDE, kZOH, io_t, bc_t>(p, stream);
+  if constexpr (sizeof(io_t) == 2) {
+    if (groups > kNarrowSlots)
+      return launch_fwd_t<MSS_FWD_T_WIDE, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_WIDE, kZOH, io_t, bc_t>(p, stream);
+  }
+  return launch_fwd_t<MSS_FWD_T_NARROW, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_NARROW, kZOH, io_t, bc_t>(p, stream);
 }
 
 }  // namespace mss
