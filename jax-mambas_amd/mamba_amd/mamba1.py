@@ -411,7 +411,7 @@ class _MambaMixer(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w_in, w_z, conv_w, conv_b, w_x, w_dt, A, D, dt_bias, w_xz_act, w_x_act, w_dt_act,
-                batch, seq_lens, zoh, w_xz_t=None):
+                batch, seq_lens, zoh, w_xz_t=None, keep=True):
         lib = _lib.register_hip_kernel()
         di, T = w_in.shape[0], x.shape[1]
         r = w_dt.shape[1]
@@ -435,15 +435,17 @@ class _MambaMixer(torch.autograd.Function):
         sdt = torch.complex64 if cplx else torch.float32
         rv = (lambda t: torch.view_as_real(t).data_ptr()) if cplx else (lambda t: t.data_ptr())
         y = torch.empty(di, T, dtype=act, device=dev)
-        y_pre = torch.empty(di, T, dtype=act, device=dev)
         last = torch.empty(batch, di, n, dtype=sdt, device=dev)
-        carries = torch.empty(batch, di, n, n_seg, dtype=sdt, device=dev)
+        y_pre = carries = None  # the backward's residuals
+        if keep:
+            y_pre = torch.empty(di, T, dtype=act, device=dev)
+            carries = torch.empty(batch, di, n, n_seg, dtype=sdt, device=dev)
         fa = _lib.FwdArgs(batch=batch, dim=di, seqlen=L, dstate=n,
                           discretization=_lib.MSS_ZOH if zoh else _lib.MSS_EULER, delta_softplus=1,
                           io_dtype=io, bc_dtype=io, u=u.data_ptr(), delta=dt.data_ptr(), A=rv(A),
                           B=x_dbl[r].data_ptr(), C=x_dbl[r + n].data_ptr(), D=_ptr(D), z=z.data_ptr(),
                           delta_bias=dt_bias.data_ptr(), seq_lens=_ptr(seq_lens), out=y.data_ptr(),
-                          last_state=rv(last), carries=rv(carries), y_pre=y_pre.data_ptr(), strides=st)
+                          last_state=rv(last), carries=rv(carries) if keep else None, y_pre=_ptr(y_pre), strides=st)
         _lib.check((lib.mss_cfwd if cplx else lib.mss_fwd)(fa, stream), "scan forward")
         ctx.save_for_backward(x, xz, u, x_dbl, dt, carries, y_pre, A, D, dt_bias, conv_w, conv_b,
                               w_xz_act, w_x_act, w_dt_act, seq_lens, w_xz_t, y)
@@ -504,7 +506,7 @@ class _MambaMixer(torch.autograd.Function):
         dw_xz = _wgrad_mm(dxz, x)
         dx = torch.mm(w_xz_t if w_xz_t is not None else w_xz_act.t(), dxz)
         return (dx, dw_xz[:di], dw_xz[di:], dconv_w, dconv_b, dw_x, dw_dt, dA, dD, dbias,
-                None, None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None)
 
 
 class MambaBlock(nn.Module):
@@ -551,7 +553,7 @@ class MambaBlock(nn.Module):
             x, self.in_proj, self.z_proj, self.conv_weight, self.conv_bias, s6.x_proj, s6.dt_proj, A,
             None if s6.D is None else s6.D.float(), s6.dt_bias.float(), w_xz,
             weights.act(s6.x_proj, act_dtype), weights.act(s6.dt_proj, act_dtype), batch, seq_lens,
-            s6.discretization == "zoh", w_xz_t)
+            s6.discretization == "zoh", w_xz_t, torch.is_grad_enabled())
         if not torch.is_grad_enabled():  # inference: keep the decode caches of this prompt
             xin = xz[:self.in_proj.shape[0]]
             k = self.conv_weight.shape[1]
