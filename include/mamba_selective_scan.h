@@ -164,6 +164,12 @@ size_t mss_bwd_workspace_bytes(const mss_bwd_args* args);
 int mss_bwd_plan(const mss_bwd_args* args, int32_t* waves, int32_t* chan_per_block);
 
 int mss_fwd(const mss_fwd_args* args, void* stream);
+
+/* mss_fwd with a workspace, in which few channels with long rows are split in time (the same
+ * results up to the rounding of the state handed from split to split). The workspace holds
+ * mss_fwd_workspace_bytes(args) bytes, 16-byte aligned; 0 bytes: none is needed or read. */
+size_t mss_fwd_workspace_bytes(const mss_fwd_args* args);
+int mss_fwd_ws(const mss_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
 int mss_bwd(const mss_bwd_args* args, void* stream);
 
 /* mss_bwd without any allocation, for callers that cannot allocate device memory (code

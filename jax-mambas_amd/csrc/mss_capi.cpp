@@ -27,6 +27,7 @@ hipError_t launch_bwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16
                            hipStream_t stream);
 hipError_t launch_bwd_reduce(const BwdParams& p, int bc_bf16, int a_width, int a_ld, int acc_bias,
                              void* dA, void* dB, void* dC, float* dD, float* dbias, hipStream_t stream);
+FwdPlan fwd_plan(int batch, int dim, int seqlen, int dstate);
 BwdPlan bwd_plan(int batch, int dim, int seqlen, int dstate, int varlen, bool split);
 hipError_t launch_cfwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
 hipError_t launch_cbwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
@@ -218,8 +219,21 @@ int validate_bwd(const mss_bwd_args* a, bool cplx = false) {
   return resolve_strides(a->strides, a->batch, a->dim, a->seqlen, a->dstate, &st);
 }
 
-int run_fwd(const mss_fwd_args* a, float* ref_states, hipStream_t stream, bool cplx = false) {
+size_t fwd_workspace_bytes(const mss_fwd_args* a, const mss::FwdPlan& plan) {
+  return static_cast<size_t>(plan.n_split - 1) * a->batch * a->dim * a->dstate * 2 * sizeof(float);
+}
+
+// ws: room for the plan's split maps, or null (rows whole).
+int run_fwd(const mss_fwd_args* a, float* ref_states, hipStream_t stream, bool cplx = false, void* ws = nullptr) {
   mss::FwdParams p{};
+  p.n_split = 1;
+  p.chunks_per_split = (a->seqlen + mss::kPartChunk - 1) / mss::kPartChunk;
+  if (ws != nullptr) {
+    const mss::FwdPlan plan = mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate);
+    p.n_split = plan.n_split;
+    p.chunks_per_split = plan.chunks_per_split;
+    p.split_map = static_cast<float*>(ws);
+  }
   p.batch = a->batch;
   p.dim = a->dim;
   p.seqlen = a->seqlen;
@@ -515,6 +529,21 @@ int mss_fwd(const mss_fwd_args* args, void* stream) {
   const int s = validate_fwd(args);
   if (s != MSS_OK) return s;
   return run_fwd(args, nullptr, static_cast<hipStream_t>(stream));
+}
+
+size_t mss_fwd_workspace_bytes(const mss_fwd_args* a) {
+  if (a == nullptr ||
+      check_dims(a->batch, a->dim, a->seqlen, a->dstate, max_dstate_for(a->io_dtype, a->bc_dtype, false)) != MSS_OK)
+    return 0;
+  return fwd_workspace_bytes(a, mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate));
+}
+
+int mss_fwd_ws(const mss_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream) {
+  const int s = validate_fwd(args);
+  if (s != MSS_OK) return s;
+  const size_t need = mss_fwd_workspace_bytes(args);
+  if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) return MSS_ERR_WORKSPACE;
+  return run_fwd(args, nullptr, static_cast<hipStream_t>(stream), false, need > 0 ? workspace : nullptr);
 }
 
 int mss_bwd(const mss_bwd_args* args, void* stream) {

@@ -581,6 +581,16 @@ struct FwdParams {
   float* carries;  // [B][D][N][n_seg]: state before each kSegSteps-step segment
   float* ref_states;
   void* y_pre;
+  // Time splits of a row (FwdPlan), 1 without a workspace: `chunks_per_split` chunks of
+  // kPartChunk steps each, and the (P, H) maps h -> P h + H of every split but the last,
+  // [n_split - 1][batch][dim][dstate][2]
+  int n_split, chunks_per_split;
+  float* split_map;
+};
+
+// Forward launch shape of a call with a workspace.
+struct FwdPlan {
+  int n_split = 1, chunks_per_split = 0;
 };
 
 // The silu(z) gate's backward needs y sigma(z); out = y z sigma(z) gives it as out / z wherever

@@ -30,7 +30,12 @@
 #define MSS_FWD_OCC_NARROW 6
 #endif
 
+
 namespace mss {
+
+// Resident workgroups of the narrow shape: 256 CUs * kOcc waves per SIMD * 4 SIMDs / kW.
+constexpr long long kFwdNarrowSlots = 256LL * MSS_FWD_OCC_NARROW * 4 / MSS_FWD_W;
+constexpr int kFwdG = 4;  // waves that share a channel where the channels alone leave it idle
 
 // Stage elements [t0, t0 + 64*kT) of `nrows` rows (B rows of states n0.., then C rows)
 // into dst[row][slot] (64*kT elements of bc_t per row), spread over all threads.
@@ -82,7 +87,10 @@ __device__ __forceinline__ void stage_round(const bc_t* __restrict__ Bb, const b
 // so no lane ever meets the row's end (the paths that handle it spill registers: B=8 D=2560
 // L=4096 float32 with lengths 306 us, the general instance 351). The general instance takes
 // B=3 D=1000 L=2051 bf16 in 92 us; element-wise accesses to such rows took 146.
-template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS, bool kWhole>
+// kG: waves that share a channel, each taking every kG-th state of a staging round; their partial
+// outputs are added in order through LDS at the end of a chunk. 1 where the channels alone fill
+// the GPU (the waves of a channel repeat its delta and u loads and the softplus).
+template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS, bool kWhole, int kG>
 __global__ __launch_bounds__(kW * 64) __attribute__((amdgpu_waves_per_eu(kOcc, kOcc)))
 void fwd_kernel(FwdParams p) {
   constexpr int kChunk = 64 * kT;
@@ -103,12 +111,16 @@ void fwd_kernel(FwdParams p) {
   constexpr bool kZLds = kT == 16;
   constexpr int kZq = kT * static_cast<int>(sizeof(io_t)) / 16;
   __shared__ uint4 s_z[kW][kZLds ? kZq * 64 : 1];
+  static_assert(kG == 1 || (kT == kSegSteps && kNB % kG == 0 && kT % kG == 0), "state groups share rounds evenly");
+  __shared__ float s_y[kG > 1 ? kW : 1][kG > 1 ? kT : 1][kG > 1 ? 65 : 1];  // partial outputs [wave][step][lane]
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = row_longest_first(p.seq_lens, p.batch, p.seqlen, blockIdx.y);
-  const int d_raw = blockIdx.x * kW + w;
+  const int d_raw = blockIdx.x * (kW / kG) + w / kG;
+  const int grp = w % kG;
+  auto own = [&](int n) { return (n % kNB) % kG == grp; };  // the states this wave runs
   const bool active = d_raw < p.dim;
   const int d = active ? d_raw : p.dim - 1;
   const int L = p.seqlen;
@@ -123,8 +135,23 @@ void fwd_kernel(FwdParams p) {
   const bc_t* __restrict__ Bb = static_cast<const bc_t*>(p.B) + b * p.bc_sb;
   const bc_t* __restrict__ Cb = static_cast<const bc_t*>(p.C) + b * p.bc_sb;
 
+  const int n_chunks = (L + kChunk - 1) / kChunk;
+  const int n_active_chunks = (len + kChunk - 1) / kChunk;
+  // Chunks [c_lo, c_end) of the row are this workgroup's.
+  const int c_lo = kG > 1 ? blockIdx.z * p.chunks_per_split : 0;
+  const int c_end = kG > 1 ? min(n_chunks, c_lo + p.chunks_per_split) : n_chunks;
+
   for (int n = lane; n < N; n += 64) {
-    s_run[w][n] = p.x0 ? p.x0[chan * N + n] : 0.f;
+    float h0 = p.x0 ? p.x0[chan * N + n] : 0.f;
+    if constexpr (kG > 1) {
+      // the state through the splits to the left (those past the row's length keep it)
+      const size_t m_ld = static_cast<size_t>(p.batch) * p.dim * N * 2;
+      const float* map = p.split_map + (chan * N + n) * 2;
+      const int m_end = min(static_cast<int>(blockIdx.z), (n_active_chunks + p.chunks_per_split - 1) / p.chunks_per_split);
+#pragma unroll 4
+      for (int m = 0; m < m_end; ++m) h0 = __builtin_fmaf(map[m * m_ld], h0, map[m * m_ld + 1]);
+    }
+    s_run[w][n] = h0;
     const float an = p.A[static_cast<size_t>(d) * N + n];
     s_a[w][n] = an;
     s_a2[w][n] = an * kLog2e;
@@ -134,8 +161,6 @@ void fwd_kernel(FwdParams p) {
   const bool dma = kWhole || p.vec_bc != 0;
   float dsum_total = 0.f;  // sum of delta over all finished steps (reference residual)
 
-  const int n_chunks = (L + kChunk - 1) / kChunk;
-  const int n_active_chunks = (len + kChunk - 1) / kChunk;
   // Rounds of kNB states per chunk, padded to an even count so round g of every chunk
   // uses buffer g & 1.
   const int rounds = ((N + kNB - 1) / kNB + 1) & ~1;
@@ -145,9 +170,10 @@ void fwd_kernel(FwdParams p) {
     const int nb = min(kNB, N - n0);
     if (nb > 0) stage_round<kT, kW, kNB, bc_t>(Bb, Cb, n0, nb, c * kChunk, L, p.bc_sn, dma, buf, tid);
   };
-  if (n_active_chunks > 0) issue_round(0, stage0);
+  const int c_live = min(n_active_chunks, c_end);
+  if (c_live > c_lo) issue_round(c_lo * rounds, stage0);
 
-  for (int c = 0; c < n_chunks; ++c) {
+  for (int c = c_lo; c < c_end; ++c) {
     const int t0 = c * kChunk;
     const int tl = t0 + lane * kT;
     const bool fast = kWhole || t0 + kChunk <= L;  // wave-uniform
@@ -165,16 +191,18 @@ void fwd_kernel(FwdParams p) {
         float zero[kT];
 #pragma unroll
         for (int j = 0; j < kT; ++j) zero[j] = 0.f;
-        if (p.out) store_seg<kT>(out_row, tl, L, fast, zero);
+        if (p.out && grp == 0) store_seg<kT>(out_row, tl, L, fast, zero);
         if (p.ref_states && lane == 63 && ref_idx >= 0) {
           for (int n = 0; n < N; ++n) {
+            if (!own(n)) continue;
             float* rs = p.ref_states + ((chan * p.n_ref + ref_idx) * N + n) * 2;
             rs[0] = fast_exp2(s_a2[w][n] * dsum_total);
             rs[1] = s_run[w][n];
           }
         }
         if (p.last && c == n_chunks - 1)
-          for (int n = lane; n < N; n += 64) p.last[chan * N + n] = s_run[w][n];
+          for (int n = lane; n < N; n += 64)
+            if (own(n)) p.last[chan * N + n] = s_run[w][n];
       }
       continue;
     }
@@ -206,7 +234,7 @@ void fwd_kernel(FwdParams p) {
         const float uu = valid ? y[j] : 0.f;
         dlt[j] = dv;
         dlu[j] = kZOH ? uu : dv * uu;  // ZOH keeps u; Euler keeps delta*u
-        y[j] = Dv * uu;
+        y[j] = grp == 0 ? Dv * uu : 0.f;
         ssum += dv;
       }
     } else {
@@ -218,7 +246,7 @@ void fwd_kernel(FwdParams p) {
     auto compute_round = [&](int g, uint4 (*buf)[2][kRowSlots]) {
       const int n0 = g * kNB;
       const int nb = min(kNB, N - n0);
-      for (int k = 0; k < nb; ++k) {
+      for (int k = grp; k < nb; k += kG) {
         const int n = n0 + k;
         const float a2 = s_a2[w][n];
         const float run = s_run[w][n];  // read early: its wait would otherwise follow the scan
@@ -272,7 +300,7 @@ void fwd_kernel(FwdParams p) {
         if (p.last && c == n_chunks - 1 && lane == 63) p.last[chan * N + n] = hend;
       }
     };
-    const int last_round = n_active_chunks * rounds;
+    const int last_round = c_live * rounds;
     for (int g = 0; g < rounds; g += 2) {
       const int r = c * rounds + g;
       wait_vmem_all();   // this thread's copies for round r have landed in LDS
@@ -285,7 +313,36 @@ void fwd_kernel(FwdParams p) {
       if (active) compute_round(g + 1, stage1);
     }
 
-    if (active && p.out) {
+    if constexpr (kG > 1) {
+      // The waves of a channel finish kT / kG steps a lane each: steps [grp, grp + 1) * 64 * kV of
+      // the chunk.
+      constexpr int kV = kT / kG;
+      const int tc = (grp * 64 + lane) * kV;  // first step within the chunk
+      const int t = t0 + tc;
+      float zv[kV];
+      if (active && p.z) {
+#pragma unroll
+        for (int e = 0; e < kV; ++e)
+          zv[e] = (kWhole || t + e < L) ? to_f32((static_cast<const io_t*>(p.z) + row)[t + e]) : 0.f;
+      }
+#pragma unroll
+      for (int j = 0; j < kT; ++j) s_y[w][j][lane] = y[j];
+      __syncthreads();  // (the next chunk's writes come after its round barriers)
+      if (active && p.out) {
+#pragma unroll
+        for (int e = 0; e < kV; ++e) {
+          float v = 0.f;
+#pragma unroll
+          for (int q = 0; q < kG; ++q) v += s_y[w - grp + q][(tc + e) % kT][(tc + e) / kT];
+          if (p.z) {
+            if (p.y_pre && t + e < len && __builtin_fabsf(zv[e]) < kZTiny)
+              store_as(static_cast<io_t*>(p.y_pre) + row + t + e, v);
+            v *= zv[e] * sigmoid(zv[e]);
+          }
+          if (kWhole || t + e < L) store_as(out_row + t + e, t + e < len ? v : 0.f);
+        }
+      }
+    } else if (active && p.out) {
       if (p.z) {
         float zv[kT];
         if (kZLds && z_lds) {
@@ -332,16 +389,110 @@ void fwd_kernel(FwdParams p) {
   }
 }
 
-template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS = kMaxN>
+// The maps of a time-split forward (FwdParams::split_map): for every (channel, state) and every
+// split but the last, (P, H) with P the product of the split's a_bar and H its end state from
+// zero. kMapG waves share a (channel, split), each taking every kMapG-th state; lane = 8 steps.
+// B rows straight from memory, the next state's fetched while this one computes. It runs only
+// where most of the GPU would idle, so its time is its own latency: short chains, few states a
+// wave.
+constexpr int kMapW = 8;
+constexpr int kMapG = 4;
+
+template <bool kZOH, typename io_t, typename bc_t>
+__global__ __launch_bounds__(kMapW * 64) void fwd_map_kernel(FwdParams p) {
+  constexpr int kT = kSegSteps;
+  constexpr int kChunk = 64 * kT;
+  __shared__ float s_h[kMapW][kMaxN];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.y;
+  const int d = blockIdx.x * (kMapW / kMapG) + w / kMapG;
+  const int grp = w % kMapG;
+  if (d >= p.dim || grp >= p.dstate) return;  // no barrier in this kernel: idle waves may leave
+  const int L = p.seqlen;
+  const int N = p.dstate;
+  const int len = p.seq_lens ? min(max(p.seq_lens[b], 0), L) : L;
+  const int c_lo = blockIdx.z * p.chunks_per_split;
+  const int c_end = min((len + kChunk - 1) / kChunk, c_lo + p.chunks_per_split);
+  if (c_lo >= c_end) return;  // no valid step: fwd_kernel skips the split
+  const size_t chan = static_cast<size_t>(b) * p.dim + d;
+  const long long row = b * p.io_sb + d * p.io_sd;
+  const bc_t* __restrict__ Bb = static_cast<const bc_t*>(p.B) + b * p.bc_sb;
+  const float* __restrict__ Ad = p.A + static_cast<size_t>(d) * N;
+  const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
+  if (lane < N) s_h[w][lane] = 0.f;
+  float dsum = 0.f;  // sum of delta over the split
+  for (int c = c_lo; c < c_end; ++c) {
+    const int t0 = c * kChunk;
+    const int tl = t0 + lane * kT;
+    const bool fast = t0 + kChunk <= L;  // wave-uniform
+    float dlt[kT], dlu[kT], bv[kT];
+    Seg<kT, io_t> sd, su;
+    Seg<kT, bc_t> sb;
+    fetch(sd, static_cast<const io_t*>(p.delta) + row, tl, L);
+    fetch(su, static_cast<const io_t*>(p.u) + row, tl, L);
+    fetch(sb, Bb + grp * p.bc_sn, tl, L);
+    finish(sd, tl, L, fast, dlt);
+    finish(su, tl, L, fast, dlu);
+    float ssum = 0.f;
+#pragma unroll
+    for (int j = 0; j < kT; ++j) {
+      const bool valid = tl + j < len;
+      const float x = dlt[j] + bias;
+      const float dv = p.delta_softplus ? softplus(x) : x;
+      const float uu = valid ? dlu[j] : 0.f;
+      dlt[j] = valid ? dv : 0.f;
+      dlu[j] = kZOH ? uu : dlt[j] * uu;
+      ssum += dlt[j];
+    }
+    dsum += wave_sum(ssum);
+    for (int n = grp; n < N; n += kMapG) {
+      const float An = Ad[n];
+      const float a2 = An * kLog2e;
+      const float h_in = s_h[w][n];
+      finish(sb, tl, L, fast, bv);
+      fetch(sb, Bb + min(n + kMapG, N - 1) * p.bc_sn, tl, L);
+      float H = 0.f;
+#pragma unroll
+      for (int j = 0; j < kT; ++j) {
+        const float bu = kZOH ? (expm1f(dlt[j] * An) * fast_rcp(An)) * bv[j] * dlu[j] : dlu[j] * bv[j];
+        H = __builtin_fmaf(fast_exp2(dlt[j] * a2), H, bu);
+      }
+      float P = fast_exp2(a2 * ssum);
+      wave_scan_affine_fwd(P, H);  // lane 63: the whole chunk
+      if (lane == 63) s_h[w][n] = __builtin_fmaf(P, h_in, H);
+    }
+  }
+  for (int n = lane; n < N; n += 64) {
+    if (n % kMapG != grp) continue;
+    float* map = p.split_map + ((static_cast<size_t>(blockIdx.z) * p.batch * p.dim + chan) * N + n) * 2;
+    map[0] = fast_exp2(Ad[n] * kLog2e * dsum);
+    map[1] = s_h[w][n];
+  }
+}
+
+template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS = kMaxN, int kG = 1>
 static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
-  dim3 grid((p.dim + kW - 1) / kW, p.batch);
+  constexpr int kChan = kW / kG;  // channels of a workgroup
+  const dim3 grid((p.dim + kChan - 1) / kChan, p.batch, kG > 1 ? p.n_split : 1);
+  if constexpr (kG > 1) {
+    if (p.n_split > 1) {
+      constexpr int kMapChan = kMapW / kMapG;
+      const dim3 maps((p.dim + kMapChan - 1) / kMapChan, p.batch, p.n_split - 1);
+      hipLaunchKernelGGL((fwd_map_kernel<kZOH, io_t, bc_t>), maps, dim3(kMapW * 64), 0, stream, p);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
+  }
   if constexpr (kMaxS == kMaxN && sizeof(io_t) == sizeof(bc_t)) {
     if (p.vec_bc && p.seqlen % (64 * kT) == 0) {
-      hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, true>), grid, dim3(kW * 64), 0, stream, p);
+      hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, true, kG>), grid, dim3(kW * 64), 0,
+                         stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, false>), grid, dim3(kW * 64), 0, stream, p);
+  hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, false, kG>), grid, dim3(kW * 64), 0,
+                     stream, p);
   return hipGetLastError();
 }
 
@@ -357,17 +508,20 @@ static hipError_t launch_fwd_z(const FwdParams& p, hipStream_t stream) {
       return hipErrorInvalidValue;
     }
   }
-  // Resident workgroups of the narrow shape: 256 CUs * kOcc waves per SIMD * 4 SIMDs / kW.
   // Float32 rows take the narrow shape at every grid size (measured on MI355X: B=16 D=2560
   // L=8192 with variable lengths 1.69 -> 1.39 ms, B=8 D=2048 L=4096 0.54 -> 0.48 ms); bf16
   // rows take it only when the grid fits one pass of it (B=8 D=2048 L=4096 428 vs 436 us,
-  // B=8 D=1536 L=2048 167 vs 175 us wide vs narrow).
-  constexpr long long kNarrowSlots = 256LL * MSS_FWD_OCC_NARROW * 4 / MSS_FWD_W;
+  // B=8 D=1536 L=2048 167 vs 175 us wide vs narrow). Four waves share a channel where one each
+  // would fill half a pass or less: B=1 D=1536 L=16384 bf16 333 -> 275 us (two waves: 311; eight
+  // over rounds of eight states: 364), B=1 D=256 L=8192 float32 133 -> 66 (108; 52).
   const long long groups = static_cast<long long>(p.batch) * ((p.dim + MSS_FWD_W - 1) / MSS_FWD_W);
   if constexpr (sizeof(io_t) == 2) {
-    if (groups > kNarrowSlots)
+    if (groups > kFwdNarrowSlots)
       return launch_fwd_t<MSS_FWD_T_WIDE, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_WIDE, kZOH, io_t, bc_t>(p, stream);
   }
+  if (2 * groups <= kFwdNarrowSlots)
+    return launch_fwd_t<MSS_FWD_T_NARROW, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_NARROW, kZOH, io_t, bc_t, kMaxN, kFwdG>(
+        p, stream);
   return launch_fwd_t<MSS_FWD_T_NARROW, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_NARROW, kZOH, io_t, bc_t>(p, stream);
 }
 

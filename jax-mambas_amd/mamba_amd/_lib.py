@@ -37,6 +37,8 @@ EXPORTED_SYMBOLS = (
     "mss_bwd_workspace_bytes",
     "mss_bwd_plan",
     "mss_fwd",
+    "mss_fwd_workspace_bytes",
+    "mss_fwd_ws",
     "mss_bwd",
     "mss_bwd_noalloc",
     "mss_bwd_scan",
@@ -211,6 +213,10 @@ def register_hip_kernel(library_path=None):
     lib = ctypes.CDLL(str(path))
     lib.mss_fwd.argtypes = [ctypes.POINTER(FwdArgs), _p]
     lib.mss_fwd.restype = ctypes.c_int
+    lib.mss_fwd_workspace_bytes.argtypes = [ctypes.POINTER(FwdArgs)]
+    lib.mss_fwd_workspace_bytes.restype = ctypes.c_size_t
+    lib.mss_fwd_ws.argtypes = [ctypes.POINTER(FwdArgs), _p, ctypes.c_size_t, _p]
+    lib.mss_fwd_ws.restype = ctypes.c_int
     lib.mss_bwd.argtypes = [ctypes.POINTER(BwdArgs), _p]
     lib.mss_bwd.restype = ctypes.c_int
     for name in ("mss_bwd_noalloc", "mss_bwd_scan", "mss_bwd_reduce", "mss_cbwd"):

@@ -33,7 +33,7 @@ from .decode import (causal_conv1d_update, gemv, gemv_conv_update, gemv_state_up
                      selective_state_update)
 from .lm_ops import GradHolder, add_rmsnorm, embed_cm
 from .proj import proj, proj_fits, wgrad, wgrad_fits
-from .selective_scan_hip import _io_tag, _ptr, _stream, selective_scan_fn
+from .selective_scan_hip import _io_tag, _ptr, _stream, launch_fwd, selective_scan_fn
 
 __all__ = ["S6", "MambaBlock", "MambaLM", "RMSNormCM", "ShadowWeights", "GraphedTrainStep"]
 
@@ -446,7 +446,7 @@ class _MambaMixer(torch.autograd.Function):
                           B=x_dbl[r].data_ptr(), C=x_dbl[r + n].data_ptr(), D=_ptr(D), z=z.data_ptr(),
                           delta_bias=dt_bias.data_ptr(), seq_lens=_ptr(seq_lens), out=y.data_ptr(),
                           last_state=rv(last), carries=rv(carries) if keep else None, y_pre=_ptr(y_pre), strides=st)
-        _lib.check((lib.mss_cfwd if cplx else lib.mss_fwd)(fa, stream), "scan forward")
+        launch_fwd(lib, fa, x, cplx)
         ctx.save_for_backward(x, xz, u, x_dbl, dt, carries, y_pre, A, D, dt_bias, conv_w, conv_b,
                               w_xz_act, w_x_act, w_dt_act, seq_lens, w_xz_t, y)
         ctx.batch, ctx.zoh, ctx.dims = batch, zoh, (di, r, n, L)

@@ -210,6 +210,16 @@ def _rv(t):
     return torch.view_as_real(t).data_ptr() if t.is_complex() else t.data_ptr()
 
 
+def launch_fwd(lib, args, u, cplx):
+    """mss_fwd_ws with the workspace its plan asks for (mss_cfwd for a complex A)."""
+    if cplx:
+        _lib.check(lib.mss_cfwd(args, _stream(u)), "mss_cfwd")
+        return
+    ws_bytes = int(lib.mss_fwd_workspace_bytes(args))
+    ws = torch.empty(ws_bytes, device=u.device, dtype=torch.uint8) if ws_bytes else None
+    _lib.check(lib.mss_fwd_ws(args, _ptr(ws), ws_bytes, _stream(u)), "mss_fwd_ws")
+
+
 @torch.library.custom_op("mamba_amd::selective_scan_fwd", mutates_args=(), device_types="cuda")
 def _scan_fwd_op(u: torch.Tensor, delta: torch.Tensor, A: torch.Tensor, B: torch.Tensor, C: torch.Tensor,
                  D: Optional[torch.Tensor], z: Optional[torch.Tensor], delta_bias: Optional[torch.Tensor],
@@ -235,8 +245,7 @@ def _scan_fwd(u, delta, A, B, C, D, z, delta_bias, initial_state, seq_lens, delt
         out=_ptr(out), last_state=_rv(last), carries=_rv(carries), y_pre=_ptr(y_pre) if z is not None else None,
         strides=_strides(u, io_layout, B, bc_layout),
     )
-    fn, name = (lib.mss_cfwd, "mss_cfwd") if A.is_complex() else (lib.mss_fwd, "mss_fwd")
-    _lib.check(fn(args, _stream(u)), name)
+    launch_fwd(lib, args, u, A.is_complex())
     return out, last, carries, y_pre
 
 

@@ -4,7 +4,8 @@ import pytest
 import torch
 
 from mamba_amd import _lib
-from test_gpu_parity import check_fused, fused_case, log, oracle_fused, run_fused, tol
+from mamba_amd.selective_scan_hip import selective_scan_fn
+from test_gpu_parity import check_fused, close, fused_case, log, oracle_fused, run_fused, tol
 from test_zz_no_alloc import GRADS, _backward, _forward, _inputs
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +43,42 @@ def test_backward_in_a_smaller_workspace(n):
         err = (res[0][k] - res[1][k]).abs().max() / res[0][k].abs().max()
         log(f"  {k}: {err:.1e}")
         assert err < 1e-5, k
+
+
+@pytest.mark.parametrize("n", [1, 3, 16])
+@pytest.mark.parametrize("grad", [False, True])
+def test_state_groups_of_a_forward(n, grad):
+    """Four waves to a channel: fewer states than waves, a last round that is not full, steps that
+    end inside a wave's share of the outputs; without gradients (no residuals) the same values."""
+    from oracle import scan64c
+    log(f"case state groups N={n} grad={grad}")
+    x, dout, dlast = fused_case(2600 + n, 2, 9, 1290, n, lens=[1290, 515])
+    if grad:
+        ts, out, last = run_fused(x, dout, dlast, "f32", False)
+        check_fused(ts, out, last, *oracle_fused(x, dout, dlast, False))
+        return
+    with torch.no_grad():
+        t = {k: torch.as_tensor(v).cuda() for k, v in x.items()}
+        out, last = selective_scan_fn(**t, delta_softplus=True, return_last_state=True)
+    fw = scan64c.forward(x["u"], x["delta"], x["A"], x["B"], x["C"], **{k: x[k] for k in x if k not in "uABC" and k != "delta"},
+                         delta_softplus=True)
+    close("out", out, fw["out"])
+    close("last_state", last, fw["last_state"])
+
+
+def test_forward_workspace():
+    """mss_fwd_ws refuses a workspace smaller than its plan's before any launch; mss_fwd, which has
+    none, keeps the rows whole and gives the same values up to rounding."""
+    lib = _lib.register_hip_kernel()
+    b, d, l, n = 1, 64, 4100, 16
+    x, _, _ = _inputs(9, b, d, l, n)
+    carries, _, out = _forward(lib, x, b, d, l, n)
+    split = selective_scan_fn(**x, delta_softplus=True)
+    assert (split - out).abs().max() < 1e-5 * out.abs().max()
+    p = lambda t: t.data_ptr()
+    fa = _lib.FwdArgs(batch=b, dim=d, seqlen=l, dstate=n, u=p(x["u"]), delta=p(x["delta"]), A=p(x["A"]), B=p(x["B"]),
+                      C=p(x["C"]), out=p(out))
+    need = int(lib.mss_fwd_workspace_bytes(fa))
+    assert need > 0
+    assert lib.mss_fwd_ws(fa, p(carries), need - 1, None) == _lib.MSS_ERR_WORKSPACE
+    assert lib.mss_fwd_ws(fa, None, need, None) == _lib.MSS_ERR_WORKSPACE
