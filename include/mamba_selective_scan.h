@@ -165,6 +165,18 @@ int mss_bwd_plan(const mss_bwd_args* args, int32_t* waves, int32_t* chan_per_blo
 
 int mss_fwd(const mss_fwd_args* args, void* stream);
 
+/* Up to MSS_MAX_TRANSPOSES float32 tensors [batch][rows][cols] copied to [batch][cols][rows] in one
+ * launch: the reference API's (B, L, D) tensors to the scan's channel-major rows (the reference
+ * gets that layout from XLA, mamba/selective_scan_cuda.py:135-147). No source may overlap a
+ * destination. */
+#define MSS_MAX_TRANSPOSES 4
+typedef struct mss_transpose_entry {
+  const float* src;
+  float* dst;
+  int32_t batch, rows, cols, reserved; /* reserved: 0 */
+} mss_transpose_entry;
+int mss_transpose(const mss_transpose_entry* entries, int32_t n, void* stream);
+
 /* mss_fwd with a workspace, in which few channels with long rows are split in time (the same
  * results up to the rounding of the state handed from split to split). The workspace holds
  * mss_fwd_workspace_bytes(args) bytes, 16-byte aligned; 0 bytes: none is needed or read. */

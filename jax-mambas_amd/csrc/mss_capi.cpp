@@ -50,6 +50,7 @@ hipError_t launch_gemv(const GemvParams& p, hipStream_t stream);
 hipError_t launch_proj(const ProjParams& p, hipStream_t stream);
 hipError_t launch_wgrad(const WgradParams& p, hipStream_t stream);
 hipError_t launch_shadow_refresh(const ShadowParams& p, hipStream_t stream);
+hipError_t launch_transpose(const TransposeParams& p, hipStream_t stream);
 hipError_t launch_adamw(const AdamWParams& p, hipStream_t stream);
 hipError_t launch_embed_cm(const EmbedParams& p, hipStream_t stream);
 hipError_t launch_embed_cm_backward(const EmbedParams& p, hipStream_t stream);
@@ -1188,6 +1189,35 @@ int mss_gemv_scan_step(const mss_gemv_args* g, const mss_step_args* a, void* str
   p.epi = 2;
   p.zoh = a->discretization == MSS_ZOH;
   return run_gemv(p, stream);
+}
+
+int mss_transpose(const mss_transpose_entry* entries, int32_t n, void* stream) {
+  static_assert(mss::kMaxTransposes == MSS_MAX_TRANSPOSES, "header and kernel disagree");
+  if (entries == nullptr || n < 1 || n > MSS_MAX_TRANSPOSES) return MSS_ERR_INVALID_ARGUMENT;
+  mss::TransposeParams p{};
+  long long tiles = 0;
+  for (int i = 0; i < n; ++i) {
+    const mss_transpose_entry& e = entries[i];
+    if (!e.src || !e.dst || e.batch <= 0 || e.rows <= 0 || e.cols <= 0 || e.reserved != 0) return MSS_ERR_INVALID_ARGUMENT;
+    p.e[i].src = e.src;
+    p.e[i].dst = e.dst;
+    p.e[i].rows = e.rows;
+    p.e[i].cols = e.cols;
+    p.e[i].tiles = (e.rows + 63LL) / 64 * ((e.cols + 63LL) / 64) * e.batch;
+    if (p.e[i].tiles >= (1LL << 31)) return MSS_ERR_UNSUPPORTED;
+    tiles += p.e[i].tiles;
+  }
+  for (int i = 0; i < n; ++i)
+    for (int j = 0; j < n; ++j) {
+      const size_t si = sizeof(float) * entries[i].batch * entries[i].rows * entries[i].cols;
+      const size_t sj = sizeof(float) * entries[j].batch * entries[j].rows * entries[j].cols;
+      if (overlaps(entries[i].dst, si, entries[j].src, sj) || (i != j && overlaps(entries[i].dst, si, entries[j].dst, sj)))
+        return MSS_ERR_INVALID_ARGUMENT;
+    }
+  if (tiles >= (1LL << 31)) return MSS_ERR_UNSUPPORTED;
+  p.n = n;
+  const hipError_t e = mss::launch_transpose(p, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? MSS_OK : hip_fail(e, "launching transposes");
 }
 
 int mss_scan_fwd_repeat(void* stream, int32_t discretization, int32_t repeats, int32_t batch,

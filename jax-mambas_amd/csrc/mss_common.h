@@ -495,6 +495,19 @@ struct EmbedParams {
   float* dE;                        // [V][D], accumulated
 };
 
+// Tensors transposed by one launch (mss_transpose): [batch][rows][cols] to [batch][cols][rows].
+constexpr int kMaxTransposes = 4;
+struct TransposeEntry {
+  const float* src;
+  float* dst;
+  int rows, cols;
+  long long tiles;  // 64 x 64 tiles of all batches
+};
+struct TransposeParams {
+  TransposeEntry e[kMaxTransposes];
+  int n;
+};
+
 struct StepParams {
   int batch, dim, dstate, delta_softplus;
   long long io_sb, io_sd, bc_sb, bc_sn;

@@ -37,6 +37,7 @@ EXPORTED_SYMBOLS = (
     "mss_bwd_workspace_bytes",
     "mss_bwd_plan",
     "mss_fwd",
+    "mss_transpose",
     "mss_fwd_workspace_bytes",
     "mss_fwd_ws",
     "mss_bwd",
@@ -170,6 +171,10 @@ class ShadowEntry(ctypes.Structure):
                 ("tile0", ctypes.c_int64)]
 
 
+class TransposeEntry(ctypes.Structure):
+    _fields_ = [("src", _p), ("dst", _p), ("batch", _i32), ("rows", _i32), ("cols", _i32), ("reserved", _i32)]
+
+
 class AdamWEntry(ctypes.Structure):
     _fields_ = [("param", _p), ("grad", _p), ("exp_avg", _p), ("exp_avg_sq", _p), ("step", _p), ("shadow", _p),
                 ("shadow_t", _p), ("rows", _i32), ("cols", _i32), ("ld_t", ctypes.c_int64), ("numel", ctypes.c_int64)]
@@ -213,6 +218,8 @@ def register_hip_kernel(library_path=None):
     lib = ctypes.CDLL(str(path))
     lib.mss_fwd.argtypes = [ctypes.POINTER(FwdArgs), _p]
     lib.mss_fwd.restype = ctypes.c_int
+    lib.mss_transpose.argtypes = [ctypes.POINTER(TransposeEntry), _i32, _p]
+    lib.mss_transpose.restype = ctypes.c_int
     lib.mss_fwd_workspace_bytes.argtypes = [ctypes.POINTER(FwdArgs)]
     lib.mss_fwd_workspace_bytes.restype = ctypes.c_size_t
     lib.mss_fwd_ws.argtypes = [ctypes.POINTER(FwdArgs), _p, ctypes.c_size_t, _p]

@@ -162,6 +162,24 @@ def _conform(t, layout):
     return out
 
 
+def _transposed(xs):
+    """Contiguous float32 GPU tensors (b, r, c), at most four, as contiguous (b, c, r): one launch."""
+    out = [torch.empty(x.shape[0], x.shape[2], x.shape[1], dtype=x.dtype, device=x.device) for x in xs]
+    entries = (_lib.TransposeEntry * len(xs))(*(
+        _lib.TransposeEntry(src=x.data_ptr(), dst=o.data_ptr(), batch=x.shape[0], rows=x.shape[1], cols=x.shape[2])
+        for x, o in zip(xs, out)))
+    _lib.check(register_hip_kernel().mss_transpose(entries, len(xs), _stream(xs[0])), "mss_transpose")
+    return out
+
+
+def _conform_grad(t, layout):
+    """_conform for a gradient tensor (no autograd): a channel-last one by the transpose kernel."""
+    if (layout == "brl" and t.dtype == torch.float32 and t.numel() and not _strides_match(t, layout)
+            and t.transpose(1, 2).is_contiguous()):
+        return _transposed([t.transpose(1, 2)])[0]
+    return _conform(t, layout)
+
+
 def _row_strides(t, layout):
     """(batch stride, row stride) the kernels use for tensors in this layout."""
     s = _dense_strides(t.shape, layout)
@@ -287,7 +305,7 @@ def _scan_bwd(u, delta, A, B, C, D, z, delta_bias, initial_state, seq_lens, carr
               delta_softplus, zoh):
     lib = register_hip_kernel()
     io_layout, bc_layout = _layouts(u, B)
-    delta, z, dout = _conform(delta, io_layout), _conform(z, io_layout), _conform(dout.to(u.dtype), io_layout)
+    delta, z, dout = _conform(delta, io_layout), _conform(z, io_layout), _conform_grad(dout.to(u.dtype), io_layout)
     C = _conform(C, bc_layout)
     y_pre = _conform(y_pre, io_layout) if z is not None else None
     out = _conform(out, io_layout) if z is not None and out is not None else None
@@ -393,6 +411,35 @@ def _scan(*inputs):
 torch.library.register_autograd("mamba_amd::selective_scan_fwd", _scan_backward, setup_context=_scan_setup_context)
 
 
+class _ToRows(torch.autograd.Function):
+    """_transposed with its gradient, the transposed view of what comes back."""
+
+    @staticmethod
+    def forward(ctx, *xs):
+        ctx.set_materialize_grads(False)
+        return tuple(_transposed(xs))
+
+    @staticmethod
+    def backward(ctx, *gs):
+        return tuple(None if g is None else g.transpose(1, 2) for g in gs)
+
+
+def _to_rows(*xs):
+    """(b, l, d) float32 tensors as contiguous (b, d, l) ones: views where their memory already
+    is, the others copied together."""
+    rows = [x.transpose(1, 2) for x in xs]
+    todo = [i for i, r in enumerate(rows) if not r.is_contiguous()]
+    if not todo:
+        return rows
+    src = [xs[i] for i in todo]
+    if not (_plain_eager(*src) and all(x.is_contiguous() and x.numel() for x in src)):
+        return [r.contiguous() for r in rows]
+    grad = torch.is_grad_enabled() and any(x.requires_grad for x in src)
+    for i, r in zip(todo, _ToRows.apply(*src) if grad else _transposed(src)):
+        rows[i] = r
+    return rows
+
+
 def _validate_complex(A, initial_state):
     if A.dtype != torch.complex64:
         raise TypeError(f"a complex A must be complex64, got {A.dtype}")
@@ -467,8 +514,8 @@ def selective_scan(A, deltas, Bs, Cs, u, initial_x=None, *, use_euler_barB_appro
     register_hip_kernel()
     # Channel-major physical layout at the kernel boundary (the reference gets the same
     # layout from XLA input_layouts=(0,2,1), mamba/selective_scan_cuda.py:135-147).
-    t = lambda x: x.transpose(1, 2).contiguous()
+    u_rows, delta_rows, B_rows, C_rows = _to_rows(u, deltas, Bs, Cs)
     out, last = _scan(
-        t(u), t(deltas), A.contiguous(), t(Bs), t(Cs), None, None, None, initial_x.contiguous(), None,
+        u_rows, delta_rows, A.contiguous(), B_rows, C_rows, None, None, None, initial_x.contiguous(), None,
         False, not use_euler_barB_approx)
     return out.transpose(1, 2), last
