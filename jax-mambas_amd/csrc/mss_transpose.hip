@@ -5,7 +5,7 @@
 // Bound by HBM: one read and one write of every element. A workgroup moves a 64 x 64 tile through
 // LDS (rows 65 floats wide, so both directions touch 64 different banks): 256-byte pieces of the
 // source rows in, 256-byte pieces of the destination rows out, each thread's 16 loads in flight
-// together. Measured on MI355X for the four inputs of a scan (two of 8 MB, two of 0.5 MB): @T4@ us
+// together. Measured on MI355X for the four inputs of a scan (two of 8 MB, two of 0.5 MB): 8.7 us
 // against 31 as torch's four strided copies.
 #include "mss_common.h"
 
