@@ -33,11 +33,11 @@ hipError_t launch_cfwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hi
 hipError_t launch_cbwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
 int cbwd_chan_per_block(int batch, int dim);
 hipError_t launch_cssm_step(const StepParams& p, bool zoh, bool io_bf16, bool bc_bf16, hipStream_t stream);
-hipError_t launch_conv(const ConvParams& p, bool bwd, bool vec, bool silu, bool io_bf16,
+hipError_t launch_conv(const ConvParams& p, bool bwd, bool silu, bool io_bf16,
                        hipStream_t stream);
 hipError_t launch_conv_reduce(const ConvParams& p, int n_tiles, float* dw, float* dbias,
                               hipStream_t stream);
-int conv_tile_steps(int vec, int io_bf16);
+int conv_tile_steps(int io_bf16);
 hipError_t launch_norm_fwd(const NormParams& p, bool io_bf16, hipStream_t stream);
 hipError_t launch_norm_bwd(const NormParams& p, bool io_bf16, float* dw, hipStream_t stream);
 int norm_blocks(int tokens);
@@ -456,7 +456,6 @@ int validate_conv(const mss_conv_args* a, bool bwd) {
 
 struct ConvSetup {
   mss::ConvParams p{};
-  bool vec = false;
   int n_tiles = 0;
   size_t ws_bytes = 0;
 };
@@ -478,10 +477,7 @@ ConvSetup conv_setup(const mss_conv_args* a) {
   c.p.y = a->y;
   c.p.dy = a->dy;
   c.p.dx = a->dx;
-  const size_t esz = dtype_size(a->io_dtype);
-  c.vec = strides_aligned(st.io_sb, st.io_sd, esz) && aligned16(a->x) && aligned16(a->y) &&
-          aligned16(a->dy) && aligned16(a->dx);
-  const int tile = mss::conv_tile_steps(c.vec, a->io_dtype == MSS_BF16);
+  const int tile = mss::conv_tile_steps(a->io_dtype == MSS_BF16);
   c.n_tiles = (a->seqlen + tile - 1) / tile;
   c.ws_bytes = static_cast<size_t>(a->dim) * a->batch * c.n_tiles * (a->width + 1) * sizeof(float);
   return c;
@@ -604,10 +600,10 @@ int mss_cbwd(const mss_bwd_args* args, void* stream) {
 }
 
 size_t mss_conv_bwd_workspace_bytes(const mss_conv_args* a) {
-  // Shapes only: sized for the scalar path, which has the most step tiles.
+  // Shapes only, whatever the type: a slot for every 256 steps (a call uses one for 1024 or 2048).
   if (a == nullptr || a->batch <= 0 || a->dim <= 0 || a->seqlen <= 0 || a->width < 1 || a->width > 4)
     return 0;
-  const int tile = mss::conv_tile_steps(0, 0);
+  const int tile = 256;
   const size_t tiles = (static_cast<size_t>(a->seqlen) + tile - 1) / tile;
   return static_cast<size_t>(a->dim) * a->batch * tiles * (a->width + 1) * sizeof(float);
 }
@@ -616,7 +612,7 @@ int mss_conv_fwd(const mss_conv_args* args, void* stream) {
   const int s = validate_conv(args, false);
   if (s != MSS_OK) return s;
   ConvSetup c = conv_setup(args);
-  const hipError_t e = mss::launch_conv(c.p, false, c.vec, args->activation == 1,
+  const hipError_t e = mss::launch_conv(c.p, false, args->activation == 1,
                                         args->io_dtype == MSS_BF16, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? MSS_OK : hip_fail(e, "launching conv1d forward");
 }
@@ -636,7 +632,7 @@ int mss_conv_bwd(const mss_conv_args* args, void* stream) {
     return MSS_ERR_WORKSPACE;
   }
   c.p.part = reinterpret_cast<float*>(ws);
-  hipError_t e = mss::launch_conv(c.p, true, c.vec, args->activation == 1, args->io_dtype == MSS_BF16, st);
+  hipError_t e = mss::launch_conv(c.p, true, args->activation == 1, args->io_dtype == MSS_BF16, st);
   if (e == hipSuccess) e = mss::launch_conv_reduce(c.p, c.n_tiles, args->dweight, args->dbias, st);
   if (owned) {
     const hipError_t f = hipFreeAsync(ws, st);

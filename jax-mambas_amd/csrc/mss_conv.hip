@@ -8,9 +8,12 @@
 //   pre[t] = bias[d] + sum_{k<K} w[d][k] * x[t - (K-1) + k]      (x[t<0] = 0)
 //   y[t]   = act(pre[t]),  y[t] = 0 for t >= seq_lens[b]
 //
-// Mapping: one thread = kE consecutive steps of one row (a 16-byte vector when rows are
-// aligned, else kE = 1); grid (step tiles, channels, batch). On the vector path the K-1
-// halo steps around a thread's vector come from its neighbours through LDS.
+// Mapping: one thread = kE consecutive steps of one row, a 16-byte vector at any alignment
+// (Seg in mss_common.h); grid (step tiles, channels, batch). The K-1 halo steps around a
+// thread's vector come from its neighbours through LDS. Bound by HBM. Rows without 16-byte
+// alignment used to go one step to a thread, every thread reading its own halos: measured on
+// MI355X (bf16, 1536 channels, B=8 L=2047) forward 73 us, backward 191; so: 23 and 35
+// (17 and 31 at L=2048).
 // Backward recomputes pre from x (no residual), forms g = dy * act'(pre), and writes
 //   dx[t] = sum_k w[k] * g[t + (K-1) - k],   and per-block partials of
 //   dw[k] = sum_t g[t] * x[t - (K-1) + k],   dbias = sum_t g[t]
@@ -28,55 +31,19 @@ __device__ __forceinline__ float silu_grad(float p) {
   return s * (1.f + p * (1.f - s));
 }
 
-template <int kE, typename io_t>
-__device__ __forceinline__ void load_vec(const io_t* __restrict__ p, float (&v)[kE]) {
-  if constexpr (kE == 1) {
-    v[0] = to_f32(p[0]);
-  } else if constexpr (sizeof(io_t) == 4) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(p);
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-  } else {
-    const u32x4 a = *reinterpret_cast<const u32x4*>(p);
-    const unsigned w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = __uint_as_float(w[i] << 16);
-      v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-    }
-  }
-}
-
-template <int kE, typename io_t>
-__device__ __forceinline__ void store_vec(io_t* __restrict__ p, const float (&v)[kE]) {
-  if constexpr (kE == 1) {
-    store_as(p, v[0]);
-  } else if constexpr (sizeof(io_t) == 4) {
-    f32x4 a = {v[0], v[1], v[2], v[3]};
-    *reinterpret_cast<f32x4*>(p) = a;
-  } else {
-    u32x4 a;
-    unsigned w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-    a.x = w[0]; a.y = w[1]; a.z = w[2]; a.w = w[3];
-    *reinterpret_cast<u32x4*>(p) = a;
-  }
-}
-
 // Scalar read of row element t (0 outside [0, L)).
 template <typename io_t>
 __device__ __forceinline__ float at(const io_t* __restrict__ row, int t, int L) {
   return (t >= 0 && t < L) ? to_f32(row[t]) : 0.f;
 }
 
-// Vector path (kE >= K-1): the K-1 steps before a thread's vector are the previous
-// thread's last ones and, in the backward, the K-1 gradient terms after it are the next
-// thread's first ones; they are exchanged through LDS, so only the first (last) thread of a
-// workgroup reads its halo from global memory. Scalar path (kE = 1): halos are read.
+// The K-1 steps before a thread's vector (kE >= K-1) are the previous thread's last ones and, in
+// the backward, the K-1 gradient terms after it are the next thread's first ones; they are
+// exchanged through LDS, so only the first (last) thread of a workgroup reads its halo from
+// global memory.
 template <int kK, int kE>
 struct ConvShare {
-  static constexpr bool kOn = kE > 1 && kK > 1;
+  static constexpr bool kOn = kK > 1;
   static constexpr int kRows = kOn ? kConvThreads : 1;
   static constexpr int kH = kK > 1 ? kK - 1 : 1;
 };
@@ -91,7 +58,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_fwd_kernel(ConvParams p) {
   const int tid = threadIdx.x;
   const int t0 = (blockIdx.x * kConvThreads + tid) * kE;
   const bool live = t0 < L;
-  if (!Sh::kOn && !live) return;  // no barrier on the scalar path
+  if (!Sh::kOn && !live) return;  // (no barrier without halos)
   const long long row = b * p.sb + d * p.sd;
   const io_t* __restrict__ xr = static_cast<const io_t*>(p.x) + row;
   io_t* __restrict__ yr = static_cast<io_t*>(p.y) + row;
@@ -103,13 +70,8 @@ __global__ __launch_bounds__(kConvThreads) void conv_fwd_kernel(ConvParams p) {
 
   float xe[kE + kK - 1];  // x[t0 - (K-1) .. t0 + kE)
   float v[kE];
-  const bool full = kE > 1 && t0 + kE <= L;
-  if (full) {
-    load_vec<kE>(xr + t0, v);
-  } else {
-#pragma unroll
-    for (int j = 0; j < kE; ++j) v[j] = at(xr, t0 + j, L);
-  }
+  const bool full = t0 + kE <= L;
+  load_seg<kE>(xr, t0, L, full, v);
   if constexpr (Sh::kOn) {
 #pragma unroll
     for (int k = 0; k < kK - 1; ++k) s_tail[tid][k] = v[kE - (kK - 1) + k];
@@ -132,13 +94,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_fwd_kernel(ConvParams p) {
     for (int k = 0; k < kK; ++k) pre = __builtin_fmaf(w[k], xe[j + k], pre);
     out[j] = (t0 + j < len) ? (kSilu ? pre * sigmoid(pre) : pre) : 0.f;
   }
-  if (full) {
-    store_vec<kE>(yr + t0, out);
-  } else {
-#pragma unroll
-    for (int j = 0; j < kE; ++j)
-      if (t0 + j < L) store_as(yr + t0 + j, out[j]);
-  }
+  store_seg<kE>(yr, t0, L, full, out);
 }
 
 template <int kK, int kE, bool kSilu, typename io_t>
@@ -172,24 +128,21 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvParams p) {
   constexpr int kG = kE + kK - 1;
   float xe[kX];
   float ge[kG];
-  const bool full = kE > 1 && t0 + kE <= L;
+  const bool full = t0 + kE <= L;
   float v[kE], dv[kE];
-  if (full) {
-    load_vec<kE>(xr + t0, v);
-    load_vec<kE>(gr + t0, dv);
-  } else {
-#pragma unroll
-    for (int j = 0; j < kE; ++j) {
-      v[j] = at(xr, t0 + j, L);
-      dv[j] = at(gr, t0 + j, L);
-    }
+  {
+    Seg<kE, io_t> sx, sg;
+    fetch(sx, xr, t0, L);
+    fetch(sg, gr, t0, L);
+    finish(sx, t0, L, full, v);
+    finish(sg, t0, L, full, dv);
   }
 #pragma unroll
   for (int j = 0; j < kE; ++j) {
     xe[kK - 1 + j] = v[j];
     ge[j] = dv[j];
   }
-  // The last thread of the workgroup (or every thread on the scalar path) reads the halo
+  // The last thread of the workgroup (or every thread without halos) reads what comes
   // after its vector; the others take the next thread's gradient terms below.
   const bool own_after = !Sh::kOn || tid == kConvThreads - 1;
   if constexpr (Sh::kOn) {
@@ -241,13 +194,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvParams p) {
       for (int k = 0; k < kK; ++k) dw[k] = __builtin_fmaf(ge[j], xe[j + k], dw[k]);
       dw[kK] += ge[j];
     }
-    if (full) {
-      store_vec<kE>(dxr + t0, dx);
-    } else {
-#pragma unroll
-      for (int j = 0; j < kE; ++j)
-        if (t0 + j < L) store_as(dxr + t0 + j, dx[j]);
-    }
+    store_seg<kE>(dxr, t0, L, full, dx);
   }
   // block sums of dw / dbias -> partial slot (d, b, blockIdx.x)
 #pragma unroll
@@ -284,43 +231,39 @@ __global__ __launch_bounds__(256) void conv_reduce_kernel(const float* __restric
   }
 }
 
-int conv_tile_steps(int vec, int io_bf16) { return kConvThreads * (vec ? (io_bf16 ? 8 : 4) : 1); }
+int conv_tile_steps(int io_bf16) { return kConvThreads * (io_bf16 ? 8 : 4); }
 
 template <int kK, bool kSilu, typename io_t>
-static hipError_t launch_conv_t(const ConvParams& p, bool bwd, bool vec, hipStream_t stream) {
+static hipError_t launch_conv_t(const ConvParams& p, bool bwd, hipStream_t stream) {
   constexpr int kV = sizeof(io_t) == 2 ? 8 : 4;
-  const int per = vec ? kV : 1;
-  const dim3 grid((p.seqlen + kConvThreads * per - 1) / (kConvThreads * per), p.dim, p.batch);
-  if (bwd) {
-    if (vec) hipLaunchKernelGGL((conv_bwd_kernel<kK, kV, kSilu, io_t>), grid, dim3(kConvThreads), 0, stream, p);
-    else hipLaunchKernelGGL((conv_bwd_kernel<kK, 1, kSilu, io_t>), grid, dim3(kConvThreads), 0, stream, p);
-  } else {
-    if (vec) hipLaunchKernelGGL((conv_fwd_kernel<kK, kV, kSilu, io_t>), grid, dim3(kConvThreads), 0, stream, p);
-    else hipLaunchKernelGGL((conv_fwd_kernel<kK, 1, kSilu, io_t>), grid, dim3(kConvThreads), 0, stream, p);
-  }
+  const dim3 grid((p.seqlen + kConvThreads * kV - 1) / (kConvThreads * kV), p.dim, p.batch);
+  if (bwd)
+    hipLaunchKernelGGL((conv_bwd_kernel<kK, kV, kSilu, io_t>), grid, dim3(kConvThreads), 0, stream, p);
+  else
+    hipLaunchKernelGGL((conv_fwd_kernel<kK, kV, kSilu, io_t>), grid, dim3(kConvThreads), 0, stream, p);
   return hipGetLastError();
 }
 
 template <int kK, typename io_t>
-static hipError_t launch_conv_k(const ConvParams& p, bool bwd, bool vec, bool silu, hipStream_t stream) {
-  return silu ? launch_conv_t<kK, true, io_t>(p, bwd, vec, stream)
-              : launch_conv_t<kK, false, io_t>(p, bwd, vec, stream);
+static hipError_t launch_conv_k(const ConvParams& p, bool bwd, bool silu, hipStream_t stream) {
+  return silu ? launch_conv_t<kK, true, io_t>(p, bwd, stream)
+              : launch_conv_t<kK, false, io_t>(p, bwd, stream);
 }
 
 template <typename io_t>
-static hipError_t launch_conv_io(const ConvParams& p, bool bwd, bool vec, bool silu, hipStream_t stream) {
+static hipError_t launch_conv_io(const ConvParams& p, bool bwd, bool silu, hipStream_t stream) {
   switch (p.width) {
-    case 1: return launch_conv_k<1, io_t>(p, bwd, vec, silu, stream);
-    case 2: return launch_conv_k<2, io_t>(p, bwd, vec, silu, stream);
-    case 3: return launch_conv_k<3, io_t>(p, bwd, vec, silu, stream);
-    default: return launch_conv_k<4, io_t>(p, bwd, vec, silu, stream);
+    case 1: return launch_conv_k<1, io_t>(p, bwd, silu, stream);
+    case 2: return launch_conv_k<2, io_t>(p, bwd, silu, stream);
+    case 3: return launch_conv_k<3, io_t>(p, bwd, silu, stream);
+    default: return launch_conv_k<4, io_t>(p, bwd, silu, stream);
   }
 }
 
-hipError_t launch_conv(const ConvParams& p, bool bwd, bool vec, bool silu, bool io_bf16,
+hipError_t launch_conv(const ConvParams& p, bool bwd, bool silu, bool io_bf16,
                        hipStream_t stream) {
-  return io_bf16 ? launch_conv_io<bf16_t>(p, bwd, vec, silu, stream)
-                 : launch_conv_io<float>(p, bwd, vec, silu, stream);
+  return io_bf16 ? launch_conv_io<bf16_t>(p, bwd, silu, stream)
+                 : launch_conv_io<float>(p, bwd, silu, stream);
 }
 
 hipError_t launch_conv_reduce(const ConvParams& p, int n_tiles, float* dw, float* dbias,

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from mamba_amd.selective_scan_hip import selective_scan_fn
+from test_conv import run_case as conv_case
 from test_gpu_parity import check_fused, dev, fused_case, log, oracle_fused, run_fused, tol
 
 pytestmark = pytest.mark.gpu
@@ -57,3 +58,10 @@ def test_misaligned_tensors(l, dtype, which):
         err = float((a - m).norm() / a.norm())
         log(f"  output {i}: {err:.1e}")
         assert err < (1e-6 if dtype == "f32" else 1e-4), i
+
+
+@pytest.mark.parametrize("layout", ["brl", "rbl"])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("l", [2, 5, 9, 2047, 2050, 4097])
+def test_conv_at_any_alignment(l, dtype, layout):
+    conv_case(3, 5, l, 4, dtype, layout=layout, lens=[l, l - 1, l // 2], seed=l)
