@@ -225,6 +225,9 @@ int mss_bwd_reduce(const mss_bwd_args* args, void* stream);
  * from mss_cbwd_workspace_bytes. dB/dC sums inside one workgroup use a fixed order. */
 size_t mss_cbwd_workspace_bytes(const mss_bwd_args* args);
 int mss_cfwd(const mss_fwd_args* args, void* stream);
+/* mss_cfwd with a workspace, as mss_fwd_ws. */
+size_t mss_cfwd_workspace_bytes(const mss_fwd_args* args);
+int mss_cfwd_ws(const mss_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
 int mss_cbwd(const mss_bwd_args* args, void* stream);
 
 /* --- Causal depthwise conv1d + activation (the Mamba-1 block's short convolution). ---

@@ -31,7 +31,8 @@ FwdPlan fwd_plan(int batch, int dim, int seqlen, int dstate);
 BwdPlan bwd_plan(int batch, int dim, int seqlen, int dstate, int varlen, bool split);
 hipError_t launch_cfwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
 hipError_t launch_cbwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
-int cbwd_chan_per_block(int batch, int dim);
+BwdPlan cbwd_plan(int batch, int dim, int seqlen, bool split);
+FwdPlan cfwd_plan(int batch, int dim, int seqlen);
 hipError_t launch_cssm_step(const StepParams& p, bool zoh, bool io_bf16, bool bc_bf16, hipStream_t stream);
 hipError_t launch_conv(const ConvParams& p, bool bwd, bool silu, bool io_bf16,
                        hipStream_t stream);
@@ -157,18 +158,14 @@ struct BwdLayout {
 BwdLayout bwd_layout(int32_t batch, int32_t dim, int32_t seqlen, int32_t dstate, bool varlen,
                      bool cplx = false, bool split = true) {
   BwdLayout l;
-  l.chunks_per_split = (seqlen + mss::kPartChunk - 1) / mss::kPartChunk;
-  if (cplx) {
-    l.chan_per_block = mss::cbwd_chan_per_block(batch, dim);
-  } else {
-    const mss::BwdPlan plan = mss::bwd_plan(batch, dim, seqlen, dstate, varlen ? 1 : 0, split);
-    l.waves = plan.waves;
-    l.chan_per_block = plan.chan_per_block;
-    l.n_split = plan.n_split;
-    l.chunks_per_split = plan.chunks_per_split;
-    l.n_msg = plan.n_msg;
-    l.chunks_per_msg = std::max(1, plan.chunks_per_msg);
-  }
+  const mss::BwdPlan plan = cplx ? mss::cbwd_plan(batch, dim, seqlen, split)
+                                 : mss::bwd_plan(batch, dim, seqlen, dstate, varlen ? 1 : 0, split);
+  l.waves = plan.waves;
+  l.chan_per_block = plan.chan_per_block;
+  l.n_split = plan.n_split;
+  l.chunks_per_split = plan.chunks_per_split;
+  l.n_msg = plan.n_msg;
+  l.chunks_per_msg = std::max(1, plan.chunks_per_msg);
   l.n_blocks_d = (dim + l.chan_per_block - 1) / l.chan_per_block;
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
   l.part_stride = (static_cast<size_t>(batch) * 2 * dstate * seqlen + 63) / 64 * 64;
@@ -178,7 +175,7 @@ BwdLayout bwd_layout(int32_t batch, int32_t dim, int32_t seqlen, int32_t dstate,
   l.off_dD = l.off_dA + up(l.n_split * chans * dstate * (cplx ? 2 : 1) * sizeof(float));
   l.off_db = l.off_dD + up(l.n_split * chans * sizeof(float));
   l.off_msg = l.off_db + up(l.n_split * chans * sizeof(float));
-  l.total = l.off_msg + up(l.n_msg * chans * dstate * 2 * sizeof(float));
+  l.total = l.off_msg + up(l.n_msg * chans * dstate * (cplx ? 4 : 2) * sizeof(float));
   return l;
 }
 
@@ -220,8 +217,14 @@ int validate_bwd(const mss_bwd_args* a, bool cplx = false) {
   return resolve_strides(a->strides, a->batch, a->dim, a->seqlen, a->dstate, &st);
 }
 
-size_t fwd_workspace_bytes(const mss_fwd_args* a, const mss::FwdPlan& plan) {
-  return static_cast<size_t>(plan.n_split - 1) * a->batch * a->dim * a->dstate * 2 * sizeof(float);
+mss::FwdPlan fwd_plan_of(const mss_fwd_args* a, bool cplx) {
+  return cplx ? mss::cfwd_plan(a->batch, a->dim, a->seqlen) : mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate);
+}
+
+// Room for the split maps of a call whose sizes are valid.
+size_t fwd_workspace_bytes(const mss_fwd_args* a, bool cplx) {
+  return static_cast<size_t>(fwd_plan_of(a, cplx).n_split - 1) * a->batch * a->dim * a->dstate * (cplx ? 4 : 2) *
+         sizeof(float);
 }
 
 // ws: room for the plan's split maps, or null (rows whole).
@@ -230,7 +233,7 @@ int run_fwd(const mss_fwd_args* a, float* ref_states, hipStream_t stream, bool c
   p.n_split = 1;
   p.chunks_per_split = (a->seqlen + mss::kPartChunk - 1) / mss::kPartChunk;
   if (ws != nullptr) {
-    const mss::FwdPlan plan = mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate);
+    const mss::FwdPlan plan = fwd_plan_of(a, cplx);
     p.n_split = plan.n_split;
     p.chunks_per_split = plan.chunks_per_split;
     p.split_map = static_cast<float*>(ws);
@@ -532,13 +535,18 @@ size_t mss_fwd_workspace_bytes(const mss_fwd_args* a) {
   if (a == nullptr ||
       check_dims(a->batch, a->dim, a->seqlen, a->dstate, max_dstate_for(a->io_dtype, a->bc_dtype, false)) != MSS_OK)
     return 0;
-  return fwd_workspace_bytes(a, mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate));
+  return fwd_workspace_bytes(a, false);
+}
+
+size_t mss_cfwd_workspace_bytes(const mss_fwd_args* a) {
+  if (a == nullptr || check_dims(a->batch, a->dim, a->seqlen, a->dstate) != MSS_OK) return 0;
+  return fwd_workspace_bytes(a, true);
 }
 
 int mss_fwd_ws(const mss_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream) {
   const int s = validate_fwd(args);
   if (s != MSS_OK) return s;
-  const size_t need = mss_fwd_workspace_bytes(args);
+  const size_t need = fwd_workspace_bytes(args, false);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) return MSS_ERR_WORKSPACE;
   return run_fwd(args, nullptr, static_cast<hipStream_t>(stream), false, need > 0 ? workspace : nullptr);
 }
@@ -590,6 +598,17 @@ int mss_cfwd(const mss_fwd_args* args, void* stream) {
       !aligned8(args->carries))
     return MSS_ERR_INVALID_ARGUMENT;
   return run_fwd(args, nullptr, static_cast<hipStream_t>(stream), true);
+}
+
+int mss_cfwd_ws(const mss_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream) {
+  const int s = validate_fwd(args, true);
+  if (s != MSS_OK) return s;
+  if (!aligned8(args->A) || !aligned8(args->initial_state) || !aligned8(args->last_state) ||
+      !aligned8(args->carries))
+    return MSS_ERR_INVALID_ARGUMENT;
+  const size_t need = fwd_workspace_bytes(args, true);
+  if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) return MSS_ERR_WORKSPACE;
+  return run_fwd(args, nullptr, static_cast<hipStream_t>(stream), true, need > 0 ? workspace : nullptr);
 }
 
 int mss_cbwd(const mss_bwd_args* args, void* stream) {

@@ -108,15 +108,21 @@ __device__ __forceinline__ void wave_scan_caffine(float& pr, float& pi, float& h
 }
 
 // ---------------------------------------------------------------------------------
-// Forward. Workgroup = kCFwdW channels of one batch row; no LDS, no block barriers. The
-// running state of state n (entering the current chunk) is kept by lane n as (run_r, run_i).
-template <bool kZOH, typename io_t, typename bc_t, bool kWhole>
+// Forward. Workgroup = kCFwdW waves over kCFwdW / kG channels of one batch row; kG = 1: no LDS, no
+// block barriers. The running state of state n (entering the current chunk) is kept by lane n as
+// (run_r, run_i). kG > 1: that many waves share a channel, each taking every kG-th state, their
+// outputs added in order through LDS at the end of a chunk; the row may be split in time as well
+// (FwdParams::split_map, here complex: [n_split - 1][batch][dim][dstate][P re, im, H re, im]).
+template <bool kZOH, typename io_t, typename bc_t, bool kWhole, int kG>
 __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = row_longest_first(p.seq_lens, p.batch, p.seqlen, blockIdx.y);
-  const int d = blockIdx.x * kCFwdW + w;
-  if (d >= p.dim) return;  // wave-uniform; the kernel has no block-level barrier
+  const int d = blockIdx.x * (kCFwdW / kG) + w / kG;
+  const int grp = w % kG;
+  static_assert(kG == 1 || kG == kCFwdW, "a workgroup leaves as one where it has barriers");
+  __shared__ float s_y[kG > 1 ? kG : 1][kG > 1 ? kCT : 1][kG > 1 ? 65 : 1];  // partial outputs [wave][step][lane]
+  if (d >= p.dim) return;
   const int L = p.seqlen;
   const int N = p.dstate;
   const int len = p.seq_lens ? min(max(p.seq_lens[b], 0), L) : L;
@@ -137,7 +143,23 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
   }
   const int n_chunks = (L + kCChunk - 1) / kCChunk;
   const int n_live = (len + kCChunk - 1) / kCChunk;
-  for (int c = 0; c < n_chunks; ++c) {
+  const int c_lo = kG > 1 ? blockIdx.z * p.chunks_per_split : 0;
+  const int c_end = kG > 1 ? min(n_chunks, c_lo + p.chunks_per_split) : n_chunks;
+  if constexpr (kG > 1) {
+    if (lane < N) {  // the state through the splits to the left (those past the length keep it)
+      const float4* map = reinterpret_cast<const float4*>(p.split_map) + chan * N + lane;
+      const size_t m_ld = static_cast<size_t>(p.batch) * p.dim * N;
+      const int m_end = min(static_cast<int>(blockIdx.z), (n_live + p.chunks_per_split - 1) / p.chunks_per_split);
+      for (int m = 0; m < m_end; ++m) {
+        const float4 ph = map[m * m_ld];
+        const float nr = __builtin_fmaf(ph.x, run_r, __builtin_fmaf(-ph.y, run_i, ph.z));
+        const float ni = __builtin_fmaf(ph.x, run_i, __builtin_fmaf(ph.y, run_r, ph.w));
+        run_r = nr;
+        run_i = ni;
+      }
+    }
+  }
+  for (int c = c_lo; c < c_end; ++c) {
     const int t0 = c * kCChunk;
     const int tl = t0 + lane * kCT;
     const bool fast = kWhole || t0 + kCChunk <= L;
@@ -147,7 +169,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
       // (the backward reads no residual here, so y_pre is left unwritten).
 #pragma unroll
       for (int j = 0; j < kCT; ++j) y[j] = 0.f;
-      store_seg<kCT>(out_row, tl, L, fast, y);
+      if (grp == 0) store_seg<kCT>(out_row, tl, L, fast, y);
       continue;
     }
     float dlt[kCT], uu[kCT];
@@ -164,22 +186,24 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
       const float dv = p.delta_softplus ? softplus(x) : x;
       dlt[j] = valid ? dv : 0.f;
       uu[j] = valid ? uu[j] : 0.f;
-      y[j] = Dv * uu[j];
+      y[j] = grp == 0 ? Dv * uu[j] : 0.f;
       ssum += dlt[j];
     }
     // B and C rows of the next state are loaded one state ahead.
     Seg<kCT, bc_t> sbn, scn;
-    fetch(sbn, Bb, tl, L, kWhole);
-    fetch(scn, Cb, tl, L, kWhole);
-    for (int n = 0; n < N; ++n) {
+    if (grp < N) {
+      fetch(sbn, Bb + grp * p.bc_sn, tl, L, kWhole);
+      fetch(scn, Cb + grp * p.bc_sn, tl, L, kWhole);
+    }
+    for (int n = grp; n < N; n += kG) {
       const CoefA cf = load_coef(p.A, static_cast<size_t>(d) * N + n);
       float ar[kCT], ai[kCT], br[kCT], bi[kCT];
       float bv[kCT], cv[kCT];
       finish(sbn, tl, L, fast, bv);
       finish(scn, tl, L, fast, cv);
-      if (n + 1 < N) {
-        fetch(sbn, Bb + (n + 1) * p.bc_sn, tl, L, kWhole);
-        fetch(scn, Cb + (n + 1) * p.bc_sn, tl, L, kWhole);
+      if (n + kG < N) {
+        fetch(sbn, Bb + (n + kG) * p.bc_sn, tl, L, kWhole);
+        fetch(scn, Cb + (n + kG) * p.bc_sn, tl, L, kWhole);
       }
       float hr = 0.f, hi = 0.f;
       {
@@ -237,6 +261,37 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
       run_r = lane == n ? nr : run_r;
       run_i = lane == n ? ni : run_i;
     }
+    if constexpr (kG > 1) {
+      // Each wave finishes kV steps a lane: steps [grp, grp + 1) * 64 * kV of the chunk.
+      constexpr int kV = kCT / kG;
+      const int tc = (grp * 64 + lane) * kV;
+      const int t = t0 + tc;
+      float zv[kV];
+      if (p.z) {
+#pragma unroll
+        for (int e = 0; e < kV; ++e)
+          zv[e] = (kWhole || t + e < L) ? to_f32((static_cast<const io_t*>(p.z) + row)[t + e]) : 0.f;
+      }
+      __syncthreads();  // the previous chunk's partial outputs have been read
+#pragma unroll
+      for (int j = 0; j < kCT; ++j) s_y[grp][j][lane] = y[j];
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < kV; ++e) {
+        float v = 0.f;
+#pragma unroll
+        for (int q = 0; q < kG; ++q) v += s_y[q][(tc + e) % kCT][(tc + e) / kCT];
+        v = t + e < len ? v : 0.f;
+        if (kWhole || t + e < L) {
+          if (p.z) {
+            if (p.y_pre) store_as(static_cast<io_t*>(p.y_pre) + row + t + e, v);
+            v = t + e < len ? v * (zv[e] * sigmoid(zv[e])) : 0.f;
+          }
+          store_as(out_row + t + e, v);
+        }
+      }
+      continue;
+    }
     if (p.z) {
       if (p.y_pre) {
         float yp[kCT];
@@ -253,9 +308,197 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
     for (int j = 0; j < kCT; ++j) y[j] = (tl + j < len) ? y[j] : 0.f;
     store_seg<kCT>(out_row, tl, L, fast, y);
   }
-  if (p.last && lane < N) {
+  if (p.last && lane < N && c_end == n_chunks && lane % kG == grp) {
     p.last[(chan * N + lane) * 2] = run_r;
     p.last[(chan * N + lane) * 2 + 1] = run_i;
+  }
+}
+
+// The maps of a time-split forward: for every (channel, state) and every split but the last, the
+// product of its a_bar and its end state from zero, as fwd_map_kernel does for real states. The
+// product is taken chunk by chunk: one exponential of the whole split's delta would round its
+// angle in turns once, at the split's size.
+constexpr int kCMapW = 8;
+constexpr int kCMapG = 4;  // waves that share a channel
+
+template <bool kZOH, typename io_t, typename bc_t>
+__global__ __launch_bounds__(kCMapW * 64) void cfwd_map_kernel(FwdParams p) {
+  __shared__ float s_ph[kCMapW][kMaxN][4];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.y;
+  const int d = blockIdx.x * (kCMapW / kCMapG) + w / kCMapG;
+  const int grp = w % kCMapG;
+  const int L = p.seqlen;
+  const int N = p.dstate;
+  if (d >= p.dim || grp >= N) return;  // no barrier in this kernel: idle waves may leave
+  const int len = p.seq_lens ? min(max(p.seq_lens[b], 0), L) : L;
+  const int c_lo = blockIdx.z * p.chunks_per_split;
+  const int c_end = min((len + kCChunk - 1) / kCChunk, c_lo + p.chunks_per_split);
+  if (c_lo >= c_end) return;  // no valid step: cfwd_kernel skips the split
+  const size_t chan = static_cast<size_t>(b) * p.dim + d;
+  const long long row = b * p.io_sb + d * p.io_sd;
+  const bc_t* __restrict__ Bb = static_cast<const bc_t*>(p.B) + b * p.bc_sb;
+  const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
+  if (lane < N) {
+    s_ph[w][lane][0] = 1.f;
+    s_ph[w][lane][1] = s_ph[w][lane][2] = s_ph[w][lane][3] = 0.f;
+  }
+  for (int c = c_lo; c < c_end; ++c) {
+    const int t0 = c * kCChunk;
+    const int tl = t0 + lane * kCT;
+    const bool fast = t0 + kCChunk <= L;
+    float dlt[kCT], uu[kCT], bv[kCT];
+    Seg<kCT, io_t> sd, su;
+    Seg<kCT, bc_t> sb;
+    fetch(sd, static_cast<const io_t*>(p.delta) + row, tl, L);
+    fetch(su, static_cast<const io_t*>(p.u) + row, tl, L);
+    fetch(sb, Bb + grp * p.bc_sn, tl, L);
+    finish(sd, tl, L, fast, dlt);
+    finish(su, tl, L, fast, uu);
+    float ssum = 0.f;
+#pragma unroll
+    for (int j = 0; j < kCT; ++j) {
+      const bool valid = tl + j < len;
+      const float x = dlt[j] + bias;
+      const float dv = p.delta_softplus ? softplus(x) : x;
+      dlt[j] = valid ? dv : 0.f;
+      uu[j] = valid ? uu[j] : 0.f;
+      ssum += dlt[j];
+    }
+    for (int n = grp; n < N; n += kCMapG) {
+      const CoefA cf = load_coef(p.A, static_cast<size_t>(d) * N + n);
+      finish(sb, tl, L, fast, bv);
+      fetch(sb, Bb + min(n + kCMapG, N - 1) * p.bc_sn, tl, L);
+      float hr = 0.f, hi = 0.f;
+#pragma unroll
+      for (int j = 0; j < kCT; ++j) {
+        const CExp e = cexp_t(dlt[j], cf);
+        const bool valid = tl + j < len;
+        const float ar = valid ? e.m * e.cy : 1.f, ai = valid ? e.m * e.sy : 0.f;
+        float br, bi;
+        if constexpr (kZOH) {
+          zoh_e(dlt[j], cf, e, br, bi);
+          br *= bv[j] * uu[j];
+          bi *= bv[j] * uu[j];
+        } else {
+          br = dlt[j] * uu[j] * bv[j];
+          bi = 0.f;
+        }
+        const float nr = __builtin_fmaf(ar, hr, __builtin_fmaf(-ai, hi, br));
+        const float ni = __builtin_fmaf(ar, hi, __builtin_fmaf(ai, hr, bi));
+        hr = nr;
+        hi = ni;
+      }
+      const CExp pe = cexp_t(ssum, cf);
+      float pr = pe.m * pe.cy, pi = pe.m * pe.sy;
+      wave_scan_caffine(pr, pi, hr, hi);  // lane 63: the whole chunk
+      if (lane == 63) {
+        float* ph = s_ph[w][n];
+        const float p0 = ph[0], p1 = ph[1], h0 = ph[2], h1 = ph[3];
+        ph[0] = __builtin_fmaf(pr, p0, -pi * p1);
+        ph[1] = __builtin_fmaf(pr, p1, pi * p0);
+        ph[2] = __builtin_fmaf(pr, h0, __builtin_fmaf(-pi, h1, hr));
+        ph[3] = __builtin_fmaf(pr, h1, __builtin_fmaf(pi, h0, hi));
+      }
+    }
+  }
+  if (lane < N && lane % kCMapG == grp) {
+    const float* ph = s_ph[w][lane];
+    reinterpret_cast<float4*>(p.split_map)[(static_cast<size_t>(blockIdx.z) * p.batch * p.dim + chan) * N + lane] =
+        make_float4(ph[0], ph[1], ph[2], ph[3]);
+  }
+}
+
+// The adjoint maps of a time-split backward (BwdParams::split_msg, complex as above): for every
+// (channel, state) and every run of chunks_per_msg chunks right of the first split, the map
+// m -> P m + Q of the adjoint entering from the right to the one the run sends left.
+template <bool kHasZ, typename io_t, typename bc_t>
+__global__ __launch_bounds__(kCMapW * 64) void cbwd_msg_kernel(BwdParams p) {
+  __shared__ float s_pq[kCMapW][kMaxN][4];
+  const int lane = threadIdx.x & 63;
+  const int seg = 63 - lane;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.y;
+  const int d = blockIdx.x * (kCMapW / kCMapG) + w / kCMapG;
+  const int grp = w % kCMapG;
+  const int L = p.seqlen;
+  const int N = p.dstate;
+  if (d >= p.dim || grp >= N) return;  // no barrier in this kernel: idle waves may leave
+  const int len = p.seq_lens ? min(max(p.seq_lens[b], 0), L) : L;
+  const int n_live = (len + kCChunk - 1) / kCChunk;
+  const int c_lo = p.chunks_per_split + blockIdx.z * p.chunks_per_msg;
+  const int c_hi = min(n_live, c_lo + p.chunks_per_msg);
+  if (c_lo >= c_hi) return;  // no valid step: cbwd_kernel skips the run
+  const size_t chan = static_cast<size_t>(b) * p.dim + d;
+  const long long row = b * p.io_sb + d * p.io_sd;
+  const bc_t* __restrict__ Cb = static_cast<const bc_t*>(p.C) + b * p.bc_sb;
+  const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
+  if (lane < N) {
+    s_pq[w][lane][0] = 1.f;
+    s_pq[w][lane][1] = s_pq[w][lane][2] = s_pq[w][lane][3] = 0.f;
+  }
+  for (int c = c_hi - 1; c >= c_lo; --c) {
+    const int t0 = c * kCChunk;
+    const int ts = t0 + seg * kCT;
+    const bool fast = t0 + kCChunk <= L;
+    float dlt[kCT], g[kCT], cv[kCT];
+    Seg<kCT, io_t> sd, sg, sz_;
+    Seg<kCT, bc_t> sc;
+    fetch(sd, static_cast<const io_t*>(p.delta) + row, ts, L);
+    fetch(sg, static_cast<const io_t*>(p.dout) + row, ts, L);
+    if constexpr (kHasZ) fetch(sz_, static_cast<const io_t*>(p.z) + row, ts, L);
+    fetch(sc, Cb + grp * p.bc_sn, ts, L);
+    finish(sd, ts, L, fast, dlt);
+    finish(sg, ts, L, fast, g);
+    if constexpr (kHasZ) {
+      float zv[kCT];
+      finish(sz_, ts, L, fast, zv);
+#pragma unroll
+      for (int j = 0; j < kCT; ++j) g[j] *= zv[j] * sigmoid(zv[j]);
+    }
+    float ssum = 0.f;
+#pragma unroll
+    for (int j = 0; j < kCT; ++j) {
+      const bool valid = ts + j < len;
+      const float x = dlt[j] + bias;
+      const float dv = p.delta_softplus ? softplus(x) : x;
+      dlt[j] = valid ? dv : 0.f;
+      g[j] = valid ? g[j] : 0.f;
+      ssum += dlt[j];
+    }
+    for (int n = grp; n < N; n += kCMapG) {
+      const CoefA cf = load_coef(p.A, static_cast<size_t>(d) * N + n);
+      finish(sc, ts, L, fast, cv);
+      fetch(sc, Cb + min(n + kCMapG, N - 1) * p.bc_sn, ts, L);
+      float qr = 0.f, qi = 0.f;
+#pragma unroll
+      for (int j = kCT - 1; j >= 0; --j) {
+        const CExp e = cexp_t(dlt[j], cf);
+        const bool valid = ts + j < len;
+        const float ar = valid ? e.m * e.cy : 1.f, ai = valid ? e.m * e.sy : 0.f;
+        const float lr = __builtin_fmaf(cv[j], g[j], qr);
+        const float li = qi;
+        qr = __builtin_fmaf(ar, lr, ai * li);
+        qi = __builtin_fmaf(ar, li, -ai * lr);
+      }
+      const CExp pe = cexp_t(ssum, cf);
+      float pr = pe.m * pe.cy, pi = -pe.m * pe.sy;
+      wave_scan_caffine(pr, pi, qr, qi);  // lane 63 (the chunk's first segment): the whole chunk
+      if (lane == 63) {
+        float* pq = s_pq[w][n];
+        const float p0 = pq[0], p1 = pq[1], q0 = pq[2], q1 = pq[3];
+        pq[0] = __builtin_fmaf(pr, p0, -pi * p1);
+        pq[1] = __builtin_fmaf(pr, p1, pi * p0);
+        pq[2] = __builtin_fmaf(pr, q0, __builtin_fmaf(-pi, q1, qr));
+        pq[3] = __builtin_fmaf(pr, q1, __builtin_fmaf(pi, q0, qi));
+      }
+    }
+  }
+  if (lane < N && lane % kCMapG == grp) {
+    const float* pq = s_pq[w][lane];
+    reinterpret_cast<float4*>(p.split_msg)[(static_cast<size_t>(blockIdx.z) * p.batch * p.dim + chan) * N + lane] =
+        make_float4(pq[0], pq[1], pq[2], pq[3]);
   }
 }
 
@@ -296,6 +539,11 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
   const int seg = 63 - lane;
   const bc_t* __restrict__ Bb = static_cast<const bc_t*>(p.B) + b * p.bc_sb;
   const bc_t* __restrict__ Cb = static_cast<const bc_t*>(p.C) + b * p.bc_sb;
+  // Chunks [c_lo, c_end) of the row are this workgroup's.
+  const int n_chunks = (L + kCChunk - 1) / kCChunk;
+  const int n_live = (len + kCChunk - 1) / kCChunk;
+  const int c_lo = blockIdx.z * p.chunks_per_split;
+  const int c_end = min(n_chunks, c_lo + p.chunks_per_split);
 
   for (int i = tid; i < cpb * N; i += W * 64) {
     const int k = i / N, n = i - k * N;
@@ -305,6 +553,19 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
       const size_t o = ((static_cast<size_t>(b) * p.dim + d) * N + n) * 2;
       mr = p.dlast[o];
       mi = p.dlast[o + 1];
+    }
+    if (p.n_split > 1 && d < p.dim) {
+      // the adjoint through the chunks to the right (those past the row's length pass it on)
+      const float4* pq = reinterpret_cast<const float4*>(p.split_msg) + (static_cast<size_t>(b) * p.dim + d) * N + n;
+      const size_t m_ld = static_cast<size_t>(p.batch) * p.dim * N;
+      const int m_end = (n_live - p.chunks_per_split + p.chunks_per_msg - 1) / p.chunks_per_msg;
+      for (int m = m_end - 1; m >= c_lo / p.chunks_per_msg; --m) {
+        const float4 x = pq[m * m_ld];
+        const float nr = __builtin_fmaf(x.x, mr, __builtin_fmaf(-x.y, mi, x.z));
+        const float ni = __builtin_fmaf(x.x, mi, __builtin_fmaf(x.y, mr, x.w));
+        mr = nr;
+        mi = ni;
+      }
     }
     s_mu[k][n][0] = mr;
     s_mu[k][n][1] = mi;
@@ -323,9 +584,7 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
   const int pred_lag = wmod + 1 < copy_waves ? 1 : N - wmod;
   __syncthreads();
 
-  const int n_chunks = (L + kCChunk - 1) / kCChunk;
-  const int n_live = (len + kCChunk - 1) / kCChunk;
-  for (int c = n_chunks - 1; c >= 0; --c) {
+  for (int c = c_end - 1; c >= c_lo; --c) {
     const int t0 = c * kCChunk;
     const int ts = t0 + seg * kCT;
     const bool fast = kWhole || t0 + kCChunk <= L;
@@ -623,9 +882,10 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
     const int d = d0 + k;
     if (d >= p.dim) continue;
     const size_t o = ((static_cast<size_t>(b) * p.dim + d) * N + n) * 2;
-    p.part_dA[o] = s_dA[k][n][0];
-    p.part_dA[o + 1] = s_dA[k][n][1];
-    if (p.dinit) {
+    float* part_dA = p.part_dA + static_cast<size_t>(blockIdx.z) * p.batch * p.dim * N * 2;
+    part_dA[o] = s_dA[k][n][0];
+    part_dA[o + 1] = s_dA[k][n][1];
+    if (p.dinit && c_lo == 0) {
       p.dinit[o] = s_mu[k][n][0];
       p.dinit[o + 1] = s_mu[k][n][1];
     }
@@ -633,8 +893,9 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
   for (int i = tid; i < cpb; i += W * 64) {
     const int d = d0 + i;
     if (d >= p.dim) continue;
-    p.part_dD[static_cast<size_t>(b) * p.dim + d] = s_dD[i];
-    p.part_dbias[static_cast<size_t>(b) * p.dim + d] = s_db[i];
+    const size_t o = (static_cast<size_t>(blockIdx.z) * p.batch + b) * p.dim + d;
+    p.part_dD[o] = s_dD[i];
+    p.part_dbias[o] = s_db[i];
   }
 }
 
@@ -712,17 +973,50 @@ hipError_t launch_cssm_step(const StepParams& p, bool zoh, bool io_bf16, bool bc
 }
 
 // ---------------------------------------------------------------------------------
-template <bool kZOH, typename io_t, typename bc_t>
-static hipError_t launch_cfwd_t(const FwdParams& p, hipStream_t stream) {
-  dim3 grid((p.dim + kCFwdW - 1) / kCFwdW, p.batch);
+// Four waves share a channel where one each would leave three quarters of the GPU's waves (5 per
+// SIMD) idle; rows are split in time where even those leave half idle, as fwd_plan does for real
+// states. Measured on MI355X, B=1 D=400 L=8000 N=16 float32: forward 356 us with a wave to
+// a channel, 165 in three splits (maps 63).
+constexpr int kCFwdSlots = 5 * 4 * kCUs;
+
+static bool cfwd_groups(const FwdParams& p) { return 4LL * p.batch * p.dim <= kCFwdSlots; }
+
+FwdPlan cfwd_plan(int batch, int dim, int seqlen) {
+  const int n_chunks = (seqlen + kCChunk - 1) / kCChunk;
+  FwdPlan plan{1, n_chunks};
+  const long long waves = 4LL * batch * dim;
+  if (2 * waves > kCFwdSlots) return plan;
+  const int s = static_cast<int>(kCFwdSlots / waves < n_chunks ? kCFwdSlots / waves : n_chunks);
+  const int per = (n_chunks + s - 1) / s;
+  if (n_chunks - per < 2) return plan;
+  return FwdPlan{(n_chunks + per - 1) / per, per};
+}
+
+template <bool kZOH, typename io_t, typename bc_t, int kG>
+static hipError_t launch_cfwd_g(const FwdParams& p, hipStream_t stream) {
+  constexpr int kChan = kCFwdW / kG;
+  const dim3 grid((p.dim + kChan - 1) / kChan, p.batch, kG > 1 ? p.n_split : 1);
   if constexpr (sizeof(io_t) == sizeof(bc_t)) {
     if (p.seqlen % kCChunk == 0) {
-      hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, true>), grid, dim3(kCFwdW * 64), 0, stream, p);
+      hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, true, kG>), grid, dim3(kCFwdW * 64), 0, stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, false>), grid, dim3(kCFwdW * 64), 0, stream, p);
+  hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, false, kG>), grid, dim3(kCFwdW * 64), 0, stream, p);
   return hipGetLastError();
+}
+
+template <bool kZOH, typename io_t, typename bc_t>
+static hipError_t launch_cfwd_t(const FwdParams& p, hipStream_t stream) {
+  if (!cfwd_groups(p)) return launch_cfwd_g<kZOH, io_t, bc_t, 1>(p, stream);
+  if (p.n_split > 1) {
+    constexpr int kChan = kCMapW / kCMapG;
+    const dim3 grid((p.dim + kChan - 1) / kChan, p.batch, p.n_split - 1);
+    hipLaunchKernelGGL((cfwd_map_kernel<kZOH, io_t, bc_t>), grid, dim3(kCMapW * 64), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return launch_cfwd_g<kZOH, io_t, bc_t, kCFwdW>(p, stream);
 }
 
 hipError_t launch_cfwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream) {
@@ -738,20 +1032,40 @@ hipError_t launch_cfwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hi
                  : launch_cfwd_t<false, float, float>(p, stream);
 }
 
-int cbwd_chan_per_block(int batch, int dim) {
+BwdPlan cbwd_plan(int batch, int dim, int seqlen, bool split) {
   // One workgroup per CU (registers: 3 waves per SIMD); take the fewest channel rounds K
   // with batch * ceil(dim / (kW*K)) <= 256, at most kCMaxChan channels.
   const long long per_row = (dim + kCBwdW - 1) / kCBwdW;
   long long k = 1;
   while (k < per_row && k * kCBwdW < kCMaxChan &&
-         static_cast<long long>(batch) * ((per_row + k - 1) / k) > 256)
+         static_cast<long long>(batch) * ((per_row + k - 1) / k) > kCUs)
     ++k;
-  return static_cast<int>(k) * kCBwdW;
+  const int n_chunks = (seqlen + kCChunk - 1) / kCChunk;
+  BwdPlan plan{kCBwdW, static_cast<int>(k) * kCBwdW, 1, n_chunks, 0, 1};
+  // Rows split in time where that leaves half the CUs or more idle, as bwd_split_plan does for
+  // real states; a chunk of a round takes about 60 us, its adjoint map an eighth of that. Measured
+  // on MI355X, B=1 D=400 L=8000 N=16 float32: 996 us whole, 271 in six splits
+  // (maps 62).
+  const long long grid = static_cast<long long>(batch) * ((per_row + k - 1) / k);
+  if (split && 2 * grid <= kCUs && n_chunks > 1) {
+    const int s = static_cast<int>(kCUs / grid < n_chunks ? kCUs / grid : n_chunks);
+    plan.chunks_per_split = (n_chunks + s - 1) / s;
+    // Maps as long as they can be with 16 waves (four to a channel) for every CU.
+    const long long map_chunks = static_cast<long long>(batch) * dim * kCMapG * (n_chunks - plan.chunks_per_split);
+    const long long want = map_chunks / (16LL * kCUs) > 1 ? map_chunks / (16LL * kCUs) : 1;
+    const int per_split = static_cast<int>((plan.chunks_per_split + want - 1) / want);
+    plan.chunks_per_msg = (plan.chunks_per_split + per_split - 1) / per_split;
+    plan.chunks_per_split = plan.chunks_per_msg * per_split;
+    plan.n_split = (n_chunks + plan.chunks_per_split - 1) / plan.chunks_per_split;
+    if (plan.n_split > 1)
+      plan.n_msg = (n_chunks - plan.chunks_per_split + plan.chunks_per_msg - 1) / plan.chunks_per_msg;
+  }
+  return plan;
 }
 
 template <bool kZOH, bool kHasZ, typename io_t, typename bc_t>
 static hipError_t launch_cbwd_t(const BwdParams& p, hipStream_t stream) {
-  dim3 grid(p.n_blocks_d, p.batch);
+  dim3 grid(p.n_blocks_d, p.batch, p.n_split);
   if constexpr (sizeof(io_t) == sizeof(bc_t)) {
     if (p.seqlen % kCChunk == 0) {
       hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t, true>), grid, dim3(kCBwdW * 64), 0, stream, p);
@@ -765,6 +1079,14 @@ static hipError_t launch_cbwd_t(const BwdParams& p, hipStream_t stream) {
 template <typename io_t, typename bc_t>
 static hipError_t launch_cbwd_io(const BwdParams& p, int zoh, hipStream_t stream) {
   const bool hz = p.z != nullptr;
+  if (p.n_split > 1) {
+    constexpr int kChan = kCMapW / kCMapG;
+    const dim3 grid((p.dim + kChan - 1) / kChan, p.batch, p.n_msg);
+    hipLaunchKernelGGL((hz ? cbwd_msg_kernel<true, io_t, bc_t> : cbwd_msg_kernel<false, io_t, bc_t>), grid,
+                       dim3(kCMapW * 64), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   if (zoh) return hz ? launch_cbwd_t<true, true, io_t, bc_t>(p, stream)
                      : launch_cbwd_t<true, false, io_t, bc_t>(p, stream);
   return hz ? launch_cbwd_t<false, true, io_t, bc_t>(p, stream)

@@ -40,6 +40,8 @@ EXPORTED_SYMBOLS = (
     "mss_transpose",
     "mss_fwd_workspace_bytes",
     "mss_fwd_ws",
+    "mss_cfwd_workspace_bytes",
+    "mss_cfwd_ws",
     "mss_bwd",
     "mss_bwd_noalloc",
     "mss_bwd_scan",
@@ -220,10 +222,11 @@ def register_hip_kernel(library_path=None):
     lib.mss_fwd.restype = ctypes.c_int
     lib.mss_transpose.argtypes = [ctypes.POINTER(TransposeEntry), _i32, _p]
     lib.mss_transpose.restype = ctypes.c_int
-    lib.mss_fwd_workspace_bytes.argtypes = [ctypes.POINTER(FwdArgs)]
-    lib.mss_fwd_workspace_bytes.restype = ctypes.c_size_t
-    lib.mss_fwd_ws.argtypes = [ctypes.POINTER(FwdArgs), _p, ctypes.c_size_t, _p]
-    lib.mss_fwd_ws.restype = ctypes.c_int
+    for size, call in ((lib.mss_fwd_workspace_bytes, lib.mss_fwd_ws), (lib.mss_cfwd_workspace_bytes, lib.mss_cfwd_ws)):
+        size.argtypes = [ctypes.POINTER(FwdArgs)]
+        size.restype = ctypes.c_size_t
+        call.argtypes = [ctypes.POINTER(FwdArgs), _p, ctypes.c_size_t, _p]
+        call.restype = ctypes.c_int
     lib.mss_bwd.argtypes = [ctypes.POINTER(BwdArgs), _p]
     lib.mss_bwd.restype = ctypes.c_int
     for name in ("mss_bwd_noalloc", "mss_bwd_scan", "mss_bwd_reduce", "mss_cbwd"):

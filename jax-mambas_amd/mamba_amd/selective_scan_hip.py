@@ -229,13 +229,11 @@ def _rv(t):
 
 
 def launch_fwd(lib, args, u, cplx):
-    """mss_fwd_ws with the workspace its plan asks for (mss_cfwd for a complex A)."""
-    if cplx:
-        _lib.check(lib.mss_cfwd(args, _stream(u)), "mss_cfwd")
-        return
-    ws_bytes = int(lib.mss_fwd_workspace_bytes(args))
+    """mss_fwd_ws (mss_cfwd_ws for a complex A) with the workspace its plan asks for."""
+    size, call = (lib.mss_cfwd_workspace_bytes, lib.mss_cfwd_ws) if cplx else (lib.mss_fwd_workspace_bytes, lib.mss_fwd_ws)
+    ws_bytes = int(size(args))
     ws = torch.empty(ws_bytes, device=u.device, dtype=torch.uint8) if ws_bytes else None
-    _lib.check(lib.mss_fwd_ws(args, _ptr(ws), ws_bytes, _stream(u)), "mss_fwd_ws")
+    _lib.check(call(args, _ptr(ws), ws_bytes, _stream(u)), "mss_cfwd_ws" if cplx else "mss_fwd_ws")
 
 
 @torch.library.custom_op("mamba_amd::selective_scan_fwd", mutates_args=(), device_types="cuda")

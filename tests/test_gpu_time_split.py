@@ -6,6 +6,7 @@ import torch
 from mamba_amd import _lib
 from mamba_amd.selective_scan_hip import selective_scan_fn
 from test_gpu_parity import check_fused, close, fused_case, log, oracle_fused, run_fused, tol
+from test_gpu_complex import check as check_complex, complex_case
 from test_zz_no_alloc import GRADS, _backward, _forward, _inputs
 
 pytestmark = pytest.mark.gpu
@@ -82,3 +83,48 @@ def test_forward_workspace():
     assert need > 0
     assert lib.mss_fwd_ws(fa, p(carries), need - 1, None) == _lib.MSS_ERR_WORKSPACE
     assert lib.mss_fwd_ws(fa, None, need, None) == _lib.MSS_ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("b,d,l,n,lens,dtype,zoh", [
+    (1, 40, 4100, 16, None, "f32", False),               # nine chunks, the last of four steps
+    (3, 30, 2600, 5, [2600, 1, 1030], "f32", True),      # rows ending before and inside a split
+    (2, 50, 3072, 3, None, "bf16", False),               # fewer states than waves of a channel
+    (8, 130, 2560, 4, None, "f32", False),               # two splits; several chunks of a channel round
+])
+def test_complex_time_split(b, d, l, n, lens, dtype, zoh):
+    log(f"case complex time split b={b} d={d} l={l} n={n} lens={lens} {dtype} zoh={zoh}")
+    x, dout, dlast = complex_case(4000 + l + n, b, d, l, n, dtype, lens=lens)
+    check_complex(x, dout, dlast, zoh, dtype)
+
+
+def test_complex_backward_in_a_smaller_workspace():
+    """mss_cbwd runs whole rows in a workspace too small for its time splits (sized without them:
+    what the library asked for before a row could be split)."""
+    lib = _lib.register_hip_kernel()
+    b, d, l, n = 1, 24, 1600, 4
+    x, _, _ = complex_case(4100, b, d, l, n, extras=False)
+    t = {k: torch.as_tensor(v).cuda() for k, v in x.items()}
+    dout = torch.randn(b, d, l, device="cuda")
+    out, last, carries, _ = torch.ops.mamba_amd.selective_scan_fwd(t["u"], t["delta"].abs(), t["A"], t["B"], t["C"], None,
+                                                                  None, None, None, None, False, False)
+    p = lambda v: (torch.view_as_real(v) if v.is_complex() else v).data_ptr()
+    res = []
+    up = lambda v: (v + 255) // 256 * 256
+    whole = up((b * 2 * n * l + 63) // 64 * 64 * 4 * 2) + up(b * d * n * 8) + 2 * up(b * d * 4)
+    delta = t["delta"].abs()
+    for size in (None, whole):
+        g = {k: torch.full_like(v, float("nan")) for k, v in dict(u=t["u"], delta=delta, A=t["A"], B=t["B"], C=t["C"]).items()}
+        a = _lib.BwdArgs(batch=b, dim=d, seqlen=l, dstate=n, u=p(t["u"]), delta=p(delta), A=p(t["A"]), B=p(t["B"]),
+                         C=p(t["C"]), carries=p(carries), dout=p(dout), du=p(g["u"]), ddelta=p(g["delta"]), dA=p(g["A"]),
+                         dB=p(g["B"]), dC=p(g["C"]))
+        need = int(lib.mss_cbwd_workspace_bytes(a))
+        assert need > whole
+        ws = torch.empty(size or need, dtype=torch.uint8, device="cuda")
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+        _lib.check(lib.mss_cbwd(a, None), "mss_cbwd")
+        torch.cuda.synchronize()
+        res.append(g)
+    for k in res[0]:
+        x0, x1 = (torch.view_as_real(r[k]) if r[k].is_complex() else r[k] for r in res)
+        assert bool(torch.isfinite(x0).all())
+        assert (x0 - x1).abs().max() < 1e-5 * x0.abs().max(), k
