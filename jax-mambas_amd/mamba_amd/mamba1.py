@@ -557,10 +557,12 @@ class MambaBlock(nn.Module):
         if not torch.is_grad_enabled():  # inference: keep the decode caches of this prompt
             xin = xz[:self.in_proj.shape[0]]
             k = self.conv_weight.shape[1]
-            tail = _rows(xin, batch)[:, :, max(0, xin.shape[1] // batch - (k - 1)):]
-            conv = torch.zeros(batch, xin.shape[0], k - 1, dtype=xin.dtype, device=xin.device)
-            if k > 1:
-                conv[:, :, conv.shape[2] - tail.shape[2]:] = tail
+            length = xin.shape[1] // batch
+            tail = _rows(xin, batch)[:, :, max(0, length - (k - 1)):]
+            if length >= k - 1:  # the whole window: one copy
+                conv = tail.clone(memory_format=torch.contiguous_format)
+            else:
+                conv = F.pad(tail, (k - 1 - length, 0))
             self.cache = {"conv": conv, "ssm": last, "A": A.detach()}
         return h, weights.mm(self.out_proj, y)
 
