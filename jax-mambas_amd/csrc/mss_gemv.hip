@@ -277,57 +277,96 @@ __device__ __forceinline__ void store_xrow(bf16_t* x, const float (&v)[kN]) {
   }
 }
 
+// The stream loads of a thread's features, kFeat of them (K <= 256 kFeat).
+template <int kN, int kFeat>
+struct NormLoads {
+  float v[kFeat][kN], w[kFeat];
+  uint32_t dv[kFeat][(kN + 1) / 2];  // delta's bf16 pairs
+};
+
+template <int kN, int kFeat>
+__device__ __forceinline__ void norm_load(const NormParams& q, int K, NormLoads<kN, kFeat>& o) {
+  const uint16_t* __restrict__ delta = static_cast<const uint16_t*>(q.delta);
+#pragma unroll
+  for (int j = 0; j < kFeat; ++j) {
+    const int f = min(static_cast<int>(threadIdx.x) + 256 * j, K - 1);
+    load_hrow<kN>(q.h + f * kN, o.v[j]);
+    o.w[j] = q.w[f];
+    if (delta) {
+      if constexpr (kN == 8) {
+        const u32x4 x = *reinterpret_cast<const u32x4*>(delta + f * kN);
+        o.dv[j][0] = x.x;
+        o.dv[j][1] = x.y;
+        o.dv[j][2] = x.z;
+        o.dv[j][3] = x.w;
+      } else if constexpr (kN == 4) {
+        const uint2 x = *reinterpret_cast<const uint2*>(delta + f * kN);
+        o.dv[j][0] = x.x;
+        o.dv[j][1] = x.y;
+      } else if constexpr (kN == 2) {
+        o.dv[j][0] = *reinterpret_cast<const uint32_t*>(delta + f * kN);
+      } else {
+        o.dv[j][0] = delta[f];
+      }
+    }
+  }
+}
+
 // X = RMSNorm(h + delta) * w of the kN tokens into LDS: the arithmetic of
 // add_rmsnorm_fwd_rows_kernel (mss_norm.hip) for each token, in the same order (thread t
 // sums its features t, t + 256, .. by fma, the waves by wave_sum, then waves 0..3 in
 // order; x = (hn * rstd) * w rounded to bf16), so X equals that kernel's output bit for
 // bit. Every workgroup computes X (a few KB from the L2); workgroup 0 also stores hn and
-// rstd. The stream loads are issued before any use, behind the weights already in flight.
-template <int kN, bool kTransposed = false>
-__device__ __forceinline__ void norm_prologue(const NormParams& q, int K, bf16_t* X, float (*s_ss)[4]) {
+// rstd. A chain of latencies in front of the products, so it is kept short. Measured on MI355X,
+// the in-projection of a 130M decode step (3072 x 768, 8 tokens), 8.2 us: one root and division
+// a lane and no feature slot past K 7.5, the token sums without a branch between them 7.3, the
+// loads ahead of the weights' 6.5.
+template <int kN, bool kTransposed, int kFeat>
+__device__ __forceinline__ void norm_finish(const NormParams& q, int K, NormLoads<kN, kFeat>& o, bf16_t* X,
+                                            float (*s_ss)[4]) {
   const int tid = threadIdx.x;
-  const bf16_t* __restrict__ delta = static_cast<const bf16_t*>(q.delta);
-  float v[kNormFeat][kN], w[kNormFeat];
-#pragma unroll
-  for (int j = 0; j < kNormFeat; ++j) {
-    const int f = min(tid + 256 * j, K - 1);
-    load_hrow<kN>(q.h + f * kN, v[j]);
-    w[j] = q.w[f];
-  }
+  const bool delta = q.delta != nullptr;
+  auto& v = o.v;
+  auto& w = o.w;
   if (delta) {
-    float dv[kNormFeat][kN];
 #pragma unroll
-    for (int j = 0; j < kNormFeat; ++j) load_xrow<kN>(delta + min(tid + 256 * j, K - 1) * kN, dv[j]);
+    for (int j = 0; j < kFeat; ++j)
 #pragma unroll
-    for (int j = 0; j < kNormFeat; ++j)
-#pragma unroll
-      for (int c = 0; c < kN; ++c) v[j][c] += dv[j][c];
+      for (int c = 0; c < kN; ++c) {
+        const uint32_t pair = o.dv[j][c / 2];
+        v[j][c] += __uint_as_float(c & 1 ? pair & 0xffff0000u : pair << 16);
+      }
   }
   float ss[kN];
 #pragma unroll
   for (int c = 0; c < kN; ++c) ss[c] = 0.f;
 #pragma unroll
-  for (int j = 0; j < kNormFeat; ++j) {
+  for (int j = 0; j < kFeat; ++j) {
     if (tid + 256 * j < K) {
 #pragma unroll
       for (int c = 0; c < kN; ++c) ss[c] = __builtin_fmaf(v[j][c], v[j][c], ss[c]);
     }
   }
 #pragma unroll
-  for (int c = 0; c < kN; ++c) {
-    const float t = wave_sum(ss[c]);
-    if ((tid & 63) == 0) s_ss[c][tid >> 6] = t;
+  for (int c = 0; c < kN; ++c) ss[c] = wave_sum(ss[c]);  // (no branch between: the sums overlap)
+  if ((tid & 63) == 0) {
+#pragma unroll
+    for (int c = 0; c < kN; ++c) s_ss[c][tid >> 6] = ss[c];
   }
   __syncthreads();
+  // One square root and division a lane (for token lane % kN), then every token's from its lane:
+  // kN of each in every thread were a third of the prologue's instructions.
   float r[kN];
-#pragma unroll
-  for (int c = 0; c < kN; ++c) {
+  {
+    const int c = tid % kN;
     const float tot = s_ss[c][0] + s_ss[c][1] + s_ss[c][2] + s_ss[c][3];
-    r[c] = 1.f / __builtin_sqrtf(tot / K + q.eps);
+    const float mine = 1.f / __builtin_sqrtf(tot / K + q.eps);
+#pragma unroll
+    for (int k = 0; k < kN; ++k) r[k] = readlane(mine, k);
   }
   const bool first = blockIdx.x == 0;
 #pragma unroll
-  for (int j = 0; j < kNormFeat; ++j) {
+  for (int j = 0; j < kFeat; ++j) {
     const int f = tid + 256 * j;
     if (f < K) {
       if (first && delta) store_hrow<kN>(q.hn + f * kN, v[j]);
@@ -346,6 +385,13 @@ __device__ __forceinline__ void norm_prologue(const NormParams& q, int K, bf16_t
 #pragma unroll
     for (int c = 0; c < kN; ++c) q.rstd[c] = r[c];
   }
+}
+
+template <int kN, bool kTransposed = false>
+__device__ __forceinline__ void norm_prologue(const NormParams& q, int K, bf16_t* X, float (*s_ss)[4]) {
+  NormLoads<kN, kNormFeat> o;
+  norm_load(q, K, o);
+  norm_finish<kN, kTransposed>(q, K, o, X, s_ss);
 }
 
 // A workgroup of 4 waves stages X (K x N bf16, at most 64 KB) in LDS once; each wave
@@ -572,12 +618,14 @@ __device__ __forceinline__ mfma_bf16x4 bf16x4_of(uint32_t lo, uint32_t hi) {
 }
 
 // kEpi 1: the conv-window step on rows [0, cs.dim) (each lane: its token column, four rows),
-// operands loaded before the X barrier; kNorm: X is the norm prologue's, stored transposed.
+// operands loaded before the X barrier; kNorm > 0: X is the norm prologue's, stored transposed
+// (kNorm features to a thread). The prologue's loads go out before the weights': memory answers
+// in order, so its sums pass while the weights are still on their way.
 // kSplit 1: each wave owns a 16-row tile (4 tiles per workgroup); kSplit 4: the workgroup's
 // 4 waves share one tile, each taking a quarter of the K steps, and the partial tiles are
 // added in wave order through LDS (more, shorter workgroups for the in-projection's 3072
 // rows).
-template <int kN, int kEpi, bool kNorm, int kSplit>
+template <int kN, int kEpi, int kNorm, int kSplit>
 __global__ __launch_bounds__(256) void gemv_mfma_kernel(GemvParams p) {
   constexpr int kPf = kSplit == 1 ? MSS_MFMA_PF_TALL : kMfmaPf;
   static_assert(kEpi == 0 || kEpi == 1, "plain store or conv-window step");
@@ -598,6 +646,11 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(GemvParams p) {
   const int g = lane >> 4;  // k-group of the lane
   const int row = min(r0 + (lane & 15), p.M - 1);
   const bf16_t* __restrict__ wrow = static_cast<const bf16_t*>(p.W) + static_cast<size_t>(row) * p.ldw + g * 16;
+  NormLoads<kN, kNorm ? kNorm : 1> nl;
+  if constexpr (kNorm > 0) {
+    norm_load(p.nm, K, nl);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   u32x4 wq[kPf][2];
 #pragma unroll
   for (int j = 0; j < kPf; ++j) {  // steps past the range re-read the row's last slice
@@ -612,8 +665,8 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(GemvParams p) {
     for (int e = 0; e < 4; ++e) load_conv(p.cs, min(r0 + 4 * g + e, p.M - 1), col, kN, co[e]);
   }
   bf16_t* __restrict__ xt = reinterpret_cast<bf16_t*>(s_xt);
-  if constexpr (kNorm) {
-    norm_prologue<kN, true>(p.nm, K, xt, s_ss);
+  if constexpr (kNorm > 0) {
+    norm_finish<kN, true>(p.nm, K, nl, xt, s_ss);
   } else {
     const bf16_t* __restrict__ X = static_cast<const bf16_t*>(p.X);
     for (int kk = tid; kk < K; kk += 256) {
@@ -705,11 +758,13 @@ static hipError_t launch_gemv_p(const GemvParams& p, hipStream_t stream) {
     if (mfma) {
       if (p.norm && p.K > kNormGemvMaxFeatures) return hipErrorInvalidValue;
       if (kEpi == 0 && p.M >= 4096) {
-        hipLaunchKernelGGL((gemv_mfma_kernel<kN, kEpi, false, 1>), dim3((p.M + 63) / 64), dim3(256), lds, stream, p);
+        hipLaunchKernelGGL((gemv_mfma_kernel<kN, kEpi, 0, 1>), dim3((p.M + 63) / 64), dim3(256), lds, stream, p);
+      } else if (p.norm && p.K <= 3 * 256) {
+        hipLaunchKernelGGL((gemv_mfma_kernel<kN, kEpi, 3, 4>), dim3((p.M + 15) / 16), dim3(256), lds, stream, p);
       } else if (p.norm) {
-        hipLaunchKernelGGL((gemv_mfma_kernel<kN, kEpi, true, 4>), dim3((p.M + 15) / 16), dim3(256), lds, stream, p);
+        hipLaunchKernelGGL((gemv_mfma_kernel<kN, kEpi, kNormFeat, 4>), dim3((p.M + 15) / 16), dim3(256), lds, stream, p);
       } else {
-        hipLaunchKernelGGL((gemv_mfma_kernel<kN, kEpi, false, 4>), dim3((p.M + 15) / 16), dim3(256), lds, stream, p);
+        hipLaunchKernelGGL((gemv_mfma_kernel<kN, kEpi, 0, 4>), dim3((p.M + 15) / 16), dim3(256), lds, stream, p);
       }
       return hipGetLastError();
     }
