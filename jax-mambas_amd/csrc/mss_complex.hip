@@ -974,9 +974,10 @@ hipError_t launch_cssm_step(const StepParams& p, bool zoh, bool io_bf16, bool bc
 
 // ---------------------------------------------------------------------------------
 // Four waves share a channel where one each would leave three quarters of the GPU's waves (5 per
-// SIMD) idle; rows are split in time where even those leave half idle, as fwd_plan does for real
-// states. Measured on MI355X, B=1 D=400 L=8000 N=16 float32: forward 356 us with a wave to
-// a channel, 165 in three splits (maps 63).
+// SIMD) idle; rows are split in time where even those leave four fifths idle (256 channels or
+// fewer), as fwd_plan does for real states. Measured on MI355X, N=16 float32: B=1 D=400 L=8000 356 us
+// with a wave to a channel, 165 with four; whole and split (maps among it) B=1 D=300 L=4096 60 and
+// 57 (four splits), D=600 L=2048 43 and 58, L=8192 173 and 209 (two splits).
 constexpr int kCFwdSlots = 5 * 4 * kCUs;
 
 static bool cfwd_groups(const FwdParams& p) { return 4LL * p.batch * p.dim <= kCFwdSlots; }
@@ -985,7 +986,7 @@ FwdPlan cfwd_plan(int batch, int dim, int seqlen) {
   const int n_chunks = (seqlen + kCChunk - 1) / kCChunk;
   FwdPlan plan{1, n_chunks};
   const long long waves = 4LL * batch * dim;
-  if (2 * waves > kCFwdSlots) return plan;
+  if (5 * waves > kCFwdSlots) return plan;
   const int s = static_cast<int>(kCFwdSlots / waves < n_chunks ? kCFwdSlots / waves : n_chunks);
   const int per = (n_chunks + s - 1) / s;
   if (n_chunks - per < 2) return plan;
@@ -1045,7 +1046,7 @@ BwdPlan cbwd_plan(int batch, int dim, int seqlen, bool split) {
   // Rows split in time where that leaves half the CUs or more idle, as bwd_split_plan does for
   // real states; a chunk of a round takes about 60 us, its adjoint map an eighth of that. Measured
   // on MI355X, B=1 D=400 L=8000 N=16 float32: 996 us whole, 271 in six splits
-  // (maps 62).
+  // (maps 62); D=1536 L=2048 241 and 166 in two.
   const long long grid = static_cast<long long>(batch) * ((per_row + k - 1) / k);
   if (split && 2 * grid <= kCUs && n_chunks > 1) {
     const int s = static_cast<int>(kCUs / grid < n_chunks ? kCUs / grid : n_chunks);

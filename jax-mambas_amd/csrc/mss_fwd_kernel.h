@@ -511,15 +511,16 @@ static hipError_t launch_fwd_z(const FwdParams& p, hipStream_t stream) {
   // Float32 rows take the narrow shape at every grid size (measured on MI355X: B=16 D=2560
   // L=8192 with variable lengths 1.69 -> 1.39 ms, B=8 D=2048 L=4096 0.54 -> 0.48 ms); bf16
   // rows take it only when the grid fits one pass of it (B=8 D=2048 L=4096 428 vs 436 us,
-  // B=8 D=1536 L=2048 167 vs 175 us wide vs narrow). Four waves share a channel where one each
-  // would fill half a pass or less: B=1 D=1536 L=16384 bf16 333 -> 275 us (two waves: 311; eight
-  // over rounds of eight states: 364), B=1 D=256 L=8192 float32 133 -> 66 (108; 52).
+  // B=8 D=1536 L=2048 167 vs 175 us wide vs narrow). Four waves share a channel where that
+  // still fits one pass: B=1 D=1536 L=16384 bf16 333 -> 275 us (two waves: 311; eight over rounds
+  // of eight states: 364), B=1 D=256 L=8192 float32 133 -> 66 (108; 52). Over two passes they
+  // lose: a B=3 D=1000 L=2051 bf16 training call takes 249 us with one wave, 268 with four.
   const long long groups = static_cast<long long>(p.batch) * ((p.dim + MSS_FWD_W - 1) / MSS_FWD_W);
   if constexpr (sizeof(io_t) == 2) {
     if (groups > kFwdNarrowSlots)
       return launch_fwd_t<MSS_FWD_T_WIDE, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_WIDE, kZOH, io_t, bc_t>(p, stream);
   }
-  if (2 * groups <= kFwdNarrowSlots)
+  if (kFwdG * groups <= kFwdNarrowSlots)
     return launch_fwd_t<MSS_FWD_T_NARROW, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_NARROW, kZOH, io_t, bc_t, kMaxN, kFwdG>(
         p, stream);
   return launch_fwd_t<MSS_FWD_T_NARROW, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_NARROW, kZOH, io_t, bc_t>(p, stream);

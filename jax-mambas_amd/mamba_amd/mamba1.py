@@ -270,6 +270,8 @@ class ShadowWeights:
         shadow for the input gradient, when kept)."""
         if x.dtype == torch.float32 or not self.by_id:
             return w.to(x.dtype) @ x
+        if not torch.is_grad_enabled():
+            return self.by_id[id(w)] @ x
         return _WeightMM.apply(x, w, self.by_id[id(w)], self.stacked_t(w))
 
     def head(self, x, e, holder=None):
