@@ -153,8 +153,10 @@ struct BwdLayout {
 };
 
 // cplx: the complex-A backward (its own channel blocking; dA partials are complex).
-// split: false keeps each row whole where the plan would split it in time (the smallest
-// workspace the call runs with).
+// split: false keeps each row whole where the plan would split it in time. Neither plan's
+// workspace is always the smaller: the time-split one holds adjoint maps, but may walk more
+// channels a workgroup and so write fewer dB/dC partials (B=1 D=256 L=8192 N=16: 17.6 MB
+// split, 23.1 whole).
 BwdLayout bwd_layout(int32_t batch, int32_t dim, int32_t seqlen, int32_t dstate, bool varlen,
                      bool cplx = false, bool split = true) {
   BwdLayout l;
@@ -189,6 +191,18 @@ BwdLayout bwd_layout_call(int32_t batch, int32_t dim, int32_t seqlen, int32_t ds
   const BwdLayout hi = bwd_layout(batch, dim, seqlen, (dstate + G - 1) / G, varlen, false, split);
   const BwdLayout lo = bwd_layout(batch, dim, seqlen, dstate / G, varlen, false, split);
   return hi.total >= lo.total ? hi : lo;
+}
+
+// The plan a call runs in `available` bytes: the time-split one (`split`) where it fits, else the
+// whole-row one. False: neither fits.
+bool bwd_layout_in(size_t available, int32_t batch, int32_t dim, int32_t seqlen, int32_t dstate, bool varlen,
+                   bool cplx, BwdLayout* l, bool* split) {
+  *split = true;
+  *l = bwd_layout_call(batch, dim, seqlen, dstate, varlen, cplx);
+  if (l->total <= available) return true;
+  *split = false;
+  *l = bwd_layout_call(batch, dim, seqlen, dstate, varlen, cplx, false);
+  return l->total <= available;
 }
 
 int validate_fwd(const mss_fwd_args* a, bool cplx = false) {
@@ -344,10 +358,10 @@ int run_bwd(const mss_bwd_args* a, int phases, hipStream_t stream, bool cplx = f
   // State groups hand the du/ddelta/ddelta_bias sums from one group to the next, so the two
   // phases cannot be split across calls.
   if (grouped && phases != kPhaseBoth) return MSS_ERR_UNSUPPORTED;
-  BwdLayout l = bwd_layout_call(a->batch, a->dim, a->seqlen, a->dstate, varlen, cplx);
-  // A caller's workspace too small for the time-split plan runs the whole-row one.
-  const bool split = a->workspace == nullptr || a->workspace_bytes >= l.total;
-  if (!split) l = bwd_layout_call(a->batch, a->dim, a->seqlen, a->dstate, varlen, cplx, false);
+  BwdLayout l;
+  bool split;
+  const bool fits = bwd_layout_in(a->workspace == nullptr ? SIZE_MAX : a->workspace_bytes, a->batch, a->dim, a->seqlen,
+                                  a->dstate, varlen, cplx, &l, &split);
   char* ws = static_cast<char*>(a->workspace);
   bool owned = false;
   if (ws == nullptr) {
@@ -356,7 +370,7 @@ int run_bwd(const mss_bwd_args* a, int phases, hipStream_t stream, bool cplx = f
     const hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&ws), l.total, stream);
     if (e != hipSuccess) return hip_fail(e, "allocating backward workspace");
     owned = true;
-  } else if (a->workspace_bytes < l.total || !aligned16(ws)) {
+  } else if (!fits || !aligned16(ws)) {
     return MSS_ERR_WORKSPACE;
   }
   const int zoh = a->discretization == MSS_ZOH;
@@ -1300,9 +1314,11 @@ int mss_scan_bwd_ws(void* stream, int32_t batch, int32_t length, int32_t dim, in
   // The carry rebuild runs one grid slice per 2048-step block (grid.z).
   if ((length + MSS_REF_CHUNK - 1) / MSS_REF_CHUNK > 65535) return MSS_ERR_UNSUPPORTED;
   const size_t carry_bytes = scan_bwd_carry_bytes(batch, length, dim, dstate);
-  // (the smallest workspace mss_bwd runs with: without its time splits)
-  if (workspace == nullptr || !aligned16(workspace) ||
-      workspace_bytes < carry_bytes + bwd_layout_call(batch, dim, length, dstate, false, false, false).total)
+  BwdLayout l;
+  bool split;
+  // (before the carry rebuild's launch: run_bwd's own check comes after it)
+  if (workspace == nullptr || !aligned16(workspace) || workspace_bytes < carry_bytes ||
+      !bwd_layout_in(workspace_bytes - carry_bytes, batch, dim, length, dstate, false, false, &l, &split))
     return MSS_ERR_WORKSPACE;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);

@@ -296,6 +296,20 @@ def test_reference_backward_workspace(lib):
     assert lib.mss_scan_bwd(None, 1, 65535 * 2048 + 1, 3, 4, *[p] * 15) == _lib.MSS_ERR_UNSUPPORTED
 
 
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="its pointers are not memory: only for a machine without a GPU")
+@pytest.mark.parametrize("n", [1, 16, 40])
+def test_reference_backward_takes_the_size_it_reports(lib, n):
+    """A workspace of mss_scan_bwd_workspace_bytes is never too small, whichever of mss_bwd's two
+    plans is the larger (here the call ends at the missing GPU instead)."""
+    p = ctypes.c_void_p(256)
+    for b in (1, 2, 8):
+        for d in (64, 256, 1000, 1536, 2560):
+            for l in (512, 2051, 8192, 16384):
+                size = lib.mss_scan_bwd_workspace_bytes(b, l, d, n)
+                s = lib.mss_scan_bwd_ws(None, b, l, d, n, *[p] * 15, p, size)
+                assert s == _lib.MSS_ERR_HIP, (b, d, l, s)
+
+
 def test_strerror(lib):
     assert lib.mss_strerror(0) == b"ok"
     assert b"invalid" in lib.mss_strerror(1)

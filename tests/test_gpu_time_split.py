@@ -1,11 +1,15 @@
 """Scans whose rows are split in time because their channels alone would leave the GPU idle:
 every output and gradient against the float64 oracle, at the edges of the split plans."""
+import ctypes
+
+import numpy as np
 import pytest
 import torch
 
 from mamba_amd import _lib
+from oracle import scan64
 from mamba_amd.selective_scan_hip import selective_scan_fn
-from test_gpu_parity import check_fused, close, fused_case, log, oracle_fused, run_fused, tol
+from test_gpu_parity import check_fused, close, fused_case, log, oracle_fused, ref_recipe, run_fused, tol
 from test_gpu_complex import check as check_complex, complex_case
 from test_zz_no_alloc import GRADS, _backward, _forward, _inputs
 
@@ -128,3 +132,33 @@ def test_complex_backward_in_a_smaller_workspace():
         x0, x1 = (torch.view_as_real(r[k]) if r[k].is_complex() else r[k] for r in res)
         assert bool(torch.isfinite(x0).all())
         assert (x0 - x1).abs().max() < 1e-5 * x0.abs().max(), k
+
+
+@pytest.mark.parametrize("b,d,l,n", [(1, 256, 8192, 16), (2, 96, 4100, 20)])
+def test_reference_backward_split_in_time(b, d, l, n):
+    """mss_scan_bwd and mss_scan_bwd_ws at shapes whose time-split plan needs less workspace than
+    the whole-row one (the second: over two groups of states), in the size the library reports."""
+    log(f"case reference backward b={b} d={d} l={l} n={n}")
+    lib = _lib.register_hip_kernel()
+    A, deltas, Bs, Cs, u, x0 = ref_recipe(15, batch=b, length=l, dim=d, n=n)
+    rng = np.random.default_rng(16)
+    dy, dfin = rng.standard_normal((b, l, d)).astype(np.float32), rng.standard_normal((b, d, n)).astype(np.float32)
+    T = lambda a: torch.as_tensor(np.ascontiguousarray(a)).cuda()
+    tr = lambda a: T(np.swapaxes(a, 1, 2))
+    ins = [T(A), tr(deltas), tr(Bs), tr(Cs), tr(u), T(x0)]
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    y, fin = torch.empty(b, d, l, device="cuda"), torch.empty(b, d, n, device="cuda")
+    cs = torch.empty(b, d, -(-l // 2048), n, 2, device="cuda")
+    _lib.check(lib.mss_scan_fwd(None, 0, b, l, d, n, *map(P, ins), P(y), P(fin), P(cs)), "mss_scan_fwd")
+    cot = [tr(dy), T(dfin)]
+    res = []
+    for ws in (None, torch.empty(int(lib.mss_scan_bwd_workspace_bytes(b, l, d, n)), dtype=torch.uint8, device="cuda")):
+        outs = [torch.full_like(t, float("nan")) for t in ins]
+        args = (None, b, l, d, n, *map(P, ins), P(cs), *map(P, cot), *map(P, outs))
+        _lib.check(lib.mss_scan_bwd(*args) if ws is None else lib.mss_scan_bwd_ws(*args, P(ws), ws.numel()), "mss_scan_bwd")
+        torch.cuda.synchronize()
+        res.append(outs)
+    grads, ab = scan64.reference_api_backward(A, deltas, Bs, Cs, u, x0, dy, dfin, abs_terms=True)
+    for name, o, w, g in zip(["dA", "ddeltas", "dBs", "dCs", "du", "dinitial_x"], *res, grads):
+        assert torch.equal(o, w), name
+        close(name, o if o.shape == g.shape else o.transpose(1, 2), g, scale=ab.get(name))
