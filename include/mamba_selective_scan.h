@@ -152,8 +152,11 @@ typedef struct mss_bwd_args {
   mss_strides strides;   /* the forward's strides; also those of dout/du/ddelta/dz, dB/dC */
 } mss_bwd_args;
 
-/* Size of the scratch mss_bwd needs for these shapes and for whether seq_lens is given
- * (0 on invalid arguments). */
+/* Size of the scratch mss_bwd asks for with these shapes and with or without seq_lens (0 on
+ * invalid arguments): that of its first plan, in which few channels with long rows are split in
+ * time. In a workspace too small for it mss_bwd keeps the rows whole if that plan fits (the same
+ * results up to the rounding of the message handed from split to split), and returns
+ * MSS_ERR_WORKSPACE if neither does; either may be the smaller. mss_cbwd likewise. */
 size_t mss_bwd_workspace_bytes(const mss_bwd_args* args);
 
 /* Launch plan mss_bwd would use for these arguments: waves per workgroup of the backward
@@ -188,13 +191,14 @@ int mss_bwd(const mss_bwd_args* args, void* stream);
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). No
  * counterpart in the reference. args->workspace is ignored: the workspace is a fixed
  * per-device array of MSS_NOALLOC_SCRATCH_BYTES inside the library, held by every device
- * the library runs this entry point on until the process ends. Shapes whose workspace
- * (mss_bwd_workspace_bytes) exceeds it return MSS_ERR_SCRATCH_LIMIT before any launch.
- * Results equal mss_bwd's bit for bit (same kernels, same plan). All calls on one device
- * share the one array: calls whose executions overlap on a device (concurrent streams, or
- * threads) race and must be serialised by the caller. The array's device address is looked
- * up once per device and kept for the life of the process: after hipDeviceReset on a device
- * (which unloads the library's code objects) this entry point must not be called there. */
+ * the library runs this entry point on until the process ends. It runs what mss_bwd runs in a
+ * workspace of that size, bit for bit: shapes whose workspace (mss_bwd_workspace_bytes) fits it,
+ * and shapes whose rows, kept whole, do. The others return MSS_ERR_SCRATCH_LIMIT before any
+ * launch. All calls on one device share the one array: calls whose executions overlap on a
+ * device (concurrent streams, or threads) race and must be serialised by the caller. The array's
+ * device address is looked up once per device and kept for the life of the process: after
+ * hipDeviceReset on a device (which unloads the library's code objects) this entry point must
+ * not be called there. */
 int mss_bwd_noalloc(const mss_bwd_args* args, void* stream);
 
 /* mss_bwd in two stream-ordered phases sharing a caller-provided workspace (NULL ->

@@ -574,9 +574,11 @@ int mss_bwd(const mss_bwd_args* args, void* stream) {
 int mss_bwd_noalloc(const mss_bwd_args* args, void* stream) {
   const int s = validate_bwd(args);
   if (s != MSS_OK) return s;
-  const BwdLayout l = bwd_layout_call(args->batch, args->dim, args->seqlen, args->dstate, args->seq_lens != nullptr,
-                                      false, false);
-  if (l.total > kScratchBytes) return MSS_ERR_SCRATCH_LIMIT;
+  BwdLayout l;
+  bool split;
+  if (!bwd_layout_in(kScratchBytes, args->batch, args->dim, args->seqlen, args->dstate, args->seq_lens != nullptr,
+                     false, &l, &split))
+    return MSS_ERR_SCRATCH_LIMIT;
   void* ws = nullptr;
   const int t = scratch_of_current_device(&ws);
   if (t != MSS_OK) return t;

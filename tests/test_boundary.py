@@ -190,6 +190,16 @@ def test_noalloc_backward_rejects_shapes_beyond_its_scratch(lib):
             _lib.MSS_NOALLOC_SCRATCH_BYTES
 
 
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="its pointers are not memory: only for a machine without a GPU")
+def test_noalloc_backward_takes_what_fits_its_scratch(lib):
+    """Shapes whose reported workspace fits the scratch are not refused, whatever the whole-row
+    plan would need (134 MB for the first two; here the call ends at the missing GPU)."""
+    for b, d, l, n in ((1, 1536, 8192, 16), (1, 96, 131072, 16), (2, 768, 16384, 16), (1, 96, 131072, 32)):
+        a = bwd_args(batch=b, dim=d, seqlen=l, dstate=n)
+        assert lib.mss_bwd_workspace_bytes(a) <= _lib.MSS_NOALLOC_SCRATCH_BYTES
+        assert lib.mss_bwd_noalloc(a, None) == _lib.MSS_ERR_HIP, (b, d, l, n)
+
+
 def test_workspace_size_depends_on_shapes_only(lib):
     a = bwd_args(batch=4, dim=1536, seqlen=2048, dstate=16)
     n1 = lib.mss_bwd_workspace_bytes(a)

@@ -50,6 +50,22 @@ def test_backward_in_a_smaller_workspace(n):
         assert err < 1e-5, k
 
 
+def test_noalloc_backward_split_in_time():
+    """A shape whose time-split plan fits the fixed scratch and whose whole-row plan does not: the
+    plan and the bits of mss_bwd in a workspace of the reported size."""
+    lib = _lib.register_hip_kernel()
+    b, d, l, n = 1, 96, 131072, 16
+    log(f"case noalloc split b={b} d={d} l={l} n={n}")
+    x, dout, dlast = _inputs(6, b, d, l, n)
+    carries, y_pre, out = _forward(lib, x, b, d, l, n)
+    size = int(lib.mss_bwd_workspace_bytes(_lib.BwdArgs(batch=b, dim=d, seqlen=l, dstate=n)))
+    args = (x, carries, y_pre, out, dout, dlast, b, d, l, n)
+    want = _backward(lib, lib.mss_bwd, *args, workspace=torch.empty(size, dtype=torch.uint8, device="cuda"))
+    got = _backward(lib, lib.mss_bwd_noalloc, *args)
+    for k in GRADS:
+        assert bool(torch.isfinite(want[k]).all()) and torch.equal(got[k], want[k]), k
+
+
 @pytest.mark.parametrize("n", [1, 3, 16])
 @pytest.mark.parametrize("grad", [False, True])
 def test_state_groups_of_a_forward(n, grad):
