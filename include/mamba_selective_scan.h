@@ -48,7 +48,7 @@
 extern "C" {
 #endif
 
-#define MSS_ABI_VERSION 16
+#define MSS_ABI_VERSION 17
 /* dstate limits (MSS_ERR_UNSUPPORTED beyond, MSS_ERR_INVALID_ARGUMENT beyond 256):
  * MSS_MAX_DSTATE_WIDE for the float32 real-A scans — mss_fwd / mss_bwd / mss_bwd_noalloc with
  * io and bc dtype MSS_F32, and the reference-signature mss_scan_* entry points (whose C

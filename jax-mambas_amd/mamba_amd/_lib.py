@@ -13,7 +13,7 @@ from pathlib import Path
 
 LIBRARY_NAME = "libmamba_selective_scan_hip.so"
 
-MSS_ABI_VERSION = 16
+MSS_ABI_VERSION = 17
 MSS_OK = 0
 MSS_ERR_INVALID_ARGUMENT = 1
 MSS_ERR_UNSUPPORTED = 2
@@ -218,6 +218,12 @@ def register_hip_kernel(library_path=None):
         searched = ", ".join(str(c) for c in candidates)
         raise FileNotFoundError(f"The selective-scan HIP library is not built; searched: {searched}")
     lib = ctypes.CDLL(str(path))
+    # first: a library of another version may lack symbols bound below
+    lib.mss_abi_version.argtypes = []
+    lib.mss_abi_version.restype = ctypes.c_int
+    if lib.mss_abi_version() != MSS_ABI_VERSION:
+        raise ImportError(f"{path} has ABI version {lib.mss_abi_version()}, this front-end "
+                          f"expects {MSS_ABI_VERSION}; rebuild the library")
     lib.mss_fwd.argtypes = [ctypes.POINTER(FwdArgs), _p]
     lib.mss_fwd.restype = ctypes.c_int
     lib.mss_transpose.argtypes = [ctypes.POINTER(TransposeEntry), _i32, _p]
@@ -297,11 +303,6 @@ def register_hip_kernel(library_path=None):
     lib.mss_strerror.restype = ctypes.c_char_p
     lib.mss_last_hip_error.argtypes = []
     lib.mss_last_hip_error.restype = ctypes.c_char_p
-    lib.mss_abi_version.argtypes = []
-    lib.mss_abi_version.restype = ctypes.c_int
-    if lib.mss_abi_version() != MSS_ABI_VERSION:
-        raise ImportError(f"{path} has ABI version {lib.mss_abi_version()}, this front-end "
-                          f"expects {MSS_ABI_VERSION}; rebuild the library")
     _LIBRARY = lib
     _LIBRARY_PATH = path
     return lib

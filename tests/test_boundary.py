@@ -62,6 +62,20 @@ def test_missing_library_raises_file_not_found(tmp_path):
         _lib._LIBRARY = saved
 
 
+def test_library_of_another_version_is_refused(tmp_path):
+    """By its version, before anything looks for a symbol that it may not have."""
+    src, old = tmp_path / "old.c", tmp_path / _lib.LIBRARY_NAME
+    src.write_text("int mss_abi_version(void) { return 16; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(old), str(src)], check=True)
+    saved = _lib._LIBRARY
+    try:
+        _lib._LIBRARY = None
+        with pytest.raises(ImportError, match="ABI version 16"):
+            _lib.register_hip_kernel(old)
+    finally:
+        _lib._LIBRARY = saved
+
+
 def fwd_args(**kw):
     base = dict(batch=2, dim=3, seqlen=10, dstate=4, u=1, delta=1, A=1, B=1, C=1, out=1)
     base.update(kw)
