@@ -48,7 +48,7 @@
 extern "C" {
 #endif
 
-#define MSS_ABI_VERSION 17
+#define MSS_ABI_VERSION 18
 /* dstate limits (MSS_ERR_UNSUPPORTED beyond, MSS_ERR_INVALID_ARGUMENT beyond 256):
  * MSS_MAX_DSTATE_WIDE for the float32 real-A scans — mss_fwd / mss_bwd / mss_bwd_noalloc with
  * io and bc dtype MSS_F32, and the reference-signature mss_scan_* entry points (whose C
@@ -165,6 +165,17 @@ size_t mss_bwd_workspace_bytes(const mss_bwd_args* args);
  * reference, whose backward launch shape is fixed by its traits
  * (native/upstream_mamba/selective_scan_bwd_kernel.cuh:499-535). */
 int mss_bwd_plan(const mss_bwd_args* args, int32_t* waves, int32_t* chan_per_block);
+
+/* The plan mss_bwd (complex_a: mss_cbwd) runs in a workspace of `available` bytes, from the shapes
+ * and seq_lens alone; launches nothing. Of a float32 call with more than MSS_MAX_DSTATE states:
+ * that of its larger group. MSS_ERR_WORKSPACE: no plan fits, and *info is the smaller one. */
+typedef struct mss_bwd_plan_info {
+  int32_t waves, chan_per_block;     /* as mss_bwd_plan gives them */
+  int32_t n_split, chunks_per_split; /* time splits of a row (1: kept whole), in 512-step chunks */
+  int32_t chunks_per_map, reserved;  /* chunks of an adjoint map (with n_split > 1) */
+  size_t workspace_bytes;
+} mss_bwd_plan_info;
+int mss_bwd_plan_in(const mss_bwd_args* args, int32_t complex_a, size_t available, mss_bwd_plan_info* info);
 
 int mss_fwd(const mss_fwd_args* args, void* stream);
 

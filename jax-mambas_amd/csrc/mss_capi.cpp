@@ -539,6 +539,25 @@ int mss_bwd_plan(const mss_bwd_args* args, int32_t* waves, int32_t* chan_per_blo
   return MSS_OK;
 }
 
+int mss_bwd_plan_in(const mss_bwd_args* a, int32_t complex_a, size_t available, mss_bwd_plan_info* info) {
+  if (a == nullptr || info == nullptr || (complex_a != 0 && complex_a != 1)) return MSS_ERR_INVALID_ARGUMENT;
+  const bool cplx = complex_a != 0;
+  const int s = cplx ? check_dims(a->batch, a->dim, a->seqlen, a->dstate)
+                     : check_dims(a->batch, a->dim, a->seqlen, a->dstate, max_dstate_for(a->io_dtype, a->bc_dtype, false));
+  if (s != MSS_OK) return s;
+  BwdLayout l;
+  bool split;
+  const bool fits = bwd_layout_in(available, a->batch, a->dim, a->seqlen, a->dstate, a->seq_lens != nullptr, cplx, &l,
+                                  &split);
+  if (!fits) {
+    const BwdLayout first =
+        bwd_layout_call(a->batch, a->dim, a->seqlen, a->dstate, a->seq_lens != nullptr, cplx);
+    if (first.total < l.total) l = first;
+  }
+  *info = {l.waves, l.chan_per_block, l.n_split, l.chunks_per_split, l.n_split > 1 ? l.chunks_per_msg : 0, 0, l.total};
+  return fits ? MSS_OK : MSS_ERR_WORKSPACE;
+}
+
 int mss_fwd(const mss_fwd_args* args, void* stream) {
   const int s = validate_fwd(args);
   if (s != MSS_OK) return s;

@@ -13,7 +13,7 @@ from pathlib import Path
 
 LIBRARY_NAME = "libmamba_selective_scan_hip.so"
 
-MSS_ABI_VERSION = 17
+MSS_ABI_VERSION = 18
 MSS_OK = 0
 MSS_ERR_INVALID_ARGUMENT = 1
 MSS_ERR_UNSUPPORTED = 2
@@ -36,6 +36,7 @@ MSS_XENT_FUSED_MAX_VOCAB = 65536
 EXPORTED_SYMBOLS = (
     "mss_bwd_workspace_bytes",
     "mss_bwd_plan",
+    "mss_bwd_plan_in",
     "mss_fwd",
     "mss_transpose",
     "mss_fwd_workspace_bytes",
@@ -173,6 +174,11 @@ class ShadowEntry(ctypes.Structure):
                 ("tile0", ctypes.c_int64)]
 
 
+class BwdPlanInfo(ctypes.Structure):
+    _fields_ = [("waves", _i32), ("chan_per_block", _i32), ("n_split", _i32), ("chunks_per_split", _i32),
+                ("chunks_per_map", _i32), ("reserved", _i32), ("workspace_bytes", ctypes.c_size_t)]
+
+
 class TransposeEntry(ctypes.Structure):
     _fields_ = [("src", _p), ("dst", _p), ("batch", _i32), ("rows", _i32), ("cols", _i32), ("reserved", _i32)]
 
@@ -245,6 +251,8 @@ def register_hip_kernel(library_path=None):
         getattr(lib, name).restype = ctypes.c_size_t
     lib.mss_bwd_plan.argtypes = [ctypes.POINTER(BwdArgs), ctypes.POINTER(_i32), ctypes.POINTER(_i32)]
     lib.mss_bwd_plan.restype = ctypes.c_int
+    lib.mss_bwd_plan_in.argtypes = [ctypes.POINTER(BwdArgs), _i32, ctypes.c_size_t, ctypes.POINTER(BwdPlanInfo)]
+    lib.mss_bwd_plan_in.restype = ctypes.c_int
     lib.mss_scan_fwd.argtypes = [_p, _i32, _i32, _i32, _i32, _i32] + [_p] * 9
     lib.mss_scan_fwd.restype = ctypes.c_int
     lib.mss_scan_fwd_repeat.argtypes = [_p, _i32, _i32, _i32, _i32, _i32, _i32] + [_p] * 9

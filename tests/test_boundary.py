@@ -334,6 +334,34 @@ def test_reference_backward_takes_the_size_it_reports(lib, n):
                 assert s == _lib.MSS_ERR_HIP, (b, d, l, s)
 
 
+def test_bwd_plan_in(lib):
+    """The plan in a given workspace: the time-split one where it fits, else the whole-row one, else
+    the smaller of the two with an error."""
+    info = _lib.BwdPlanInfo()
+    big = 1 << 62
+    for cplx, (b, d, l, n) in ((0, (1, 256, 8192, 16)), (0, (2, 40, 4000, 20)), (1, (1, 24, 1600, 4))):
+        a = _lib.BwdArgs(batch=b, dim=d, seqlen=l, dstate=n)
+        size = (lib.mss_cbwd_workspace_bytes if cplx else lib.mss_bwd_workspace_bytes)(a)
+        assert lib.mss_bwd_plan_in(a, cplx, big, info) == 0 and info.n_split > 1 and info.workspace_bytes == size
+        assert info.n_split * info.chunks_per_split >= -(-l // 512) > (info.n_split - 1) * info.chunks_per_split
+        s = lib.mss_bwd_plan_in(a, cplx, size - 1, info)
+        if s == _lib.MSS_OK:  # the rows whole, in less
+            assert info.n_split == 1 and info.chunks_per_map == 0 and info.workspace_bytes < size
+        else:
+            assert s == _lib.MSS_ERR_WORKSPACE and info.workspace_bytes == size
+        assert lib.mss_bwd_plan_in(a, cplx, 0, info) == _lib.MSS_ERR_WORKSPACE
+        least = info.workspace_bytes
+        assert lib.mss_bwd_plan_in(a, cplx, least, info) == 0 and info.workspace_bytes == least
+        assert lib.mss_bwd_plan_in(a, cplx, least - 1, info) == _lib.MSS_ERR_WORKSPACE
+    a = _lib.BwdArgs(batch=4, dim=1536, seqlen=2048, dstate=16)
+    assert lib.mss_bwd_plan_in(a, 0, big, info) == 0
+    assert (info.waves, info.chan_per_block, info.n_split, info.chunks_per_split) == (12, 24, 1, 4)
+    bad = _lib.MSS_ERR_INVALID_ARGUMENT
+    assert lib.mss_bwd_plan_in(None, 0, big, info) == bad and lib.mss_bwd_plan_in(a, 0, big, None) == bad
+    assert lib.mss_bwd_plan_in(a, 2, big, info) == bad
+    assert lib.mss_bwd_plan_in(bwd_args(dstate=17), 1, big, info) != 0
+
+
 def test_strerror(lib):
     assert lib.mss_strerror(0) == b"ok"
     assert b"invalid" in lib.mss_strerror(1)

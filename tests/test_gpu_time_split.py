@@ -18,8 +18,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("b,d,l,n,lens,dtype,zoh", [
     (1, 5, 513, 16, None, "f32", False),       # two chunks, the second of one step
-    (8, 192, 2051, 16, None, "f32", False),    # two splits of three chunks (the second: two and a bit)
-    (8, 192, 8190, 4, None, "bf16", False),    # several chunks to an adjoint map
+    (8, 192, 2051, 16, None, "f32", False),    # five splits of one chunk, the last of three steps
+    (8, 192, 8190, 4, None, "bf16", False),    # sixteen splits of one chunk
     (1, 70, 4096, 11, None, "bf16", True),     # eight splits of one whole chunk, two accumulator copies
     (3, 100, 4100, 16, [4100, 1, 2560], "f32", False),  # rows ending before, at and inside a split
     (3, 100, 4100, 8, [0, 4099, 513], "bf16", True),
@@ -30,6 +30,74 @@ def test_time_split_scan(b, d, l, n, lens, dtype, zoh):
     ts, out, last = run_fused(x, dout, dlast, dtype, zoh)
     fw, g = oracle_fused(x, dout, dlast, zoh)
     check_fused(ts, out, last, fw, g, *tol(dtype))
+
+
+def bwd_plan(b, d, l, n, lens=None, cplx=False):
+    """(splits of a row, chunks of a split, chunks of an adjoint map) of the backward."""
+    info = _lib.BwdPlanInfo()
+    a = _lib.BwdArgs(batch=b, dim=d, seqlen=l, dstate=n, seq_lens=None if lens is None else 1)
+    _lib.check(_lib.register_hip_kernel().mss_bwd_plan_in(a, int(cplx), 1 << 62, info), "mss_bwd_plan_in")
+    return info.n_split, info.chunks_per_split, info.chunks_per_map
+
+
+@pytest.mark.parametrize("b,d,l,n,lens,dtype,zoh,plan", [
+    (8, 100, 12003, 2, None, "f32", False, (4, 6, 2)),
+    (3, 300, 11003, 3, [11003, 7400, 1300], "bf16", True, (11, 2, 2)),   # rows ending inside a map's chunks
+    (8, 100, 12000, 3, [12000, 11000, 4097, 4096, 9000, 6000, 1, 2600], "f32", False, (6, 4, 2)),
+    (1, 768, 12000, 1, None, "bf16", False, (4, 6, 2)),
+    (2, 400, 12001, 17, None, "f32", False, (4, 6, 2)),                  # two groups of states
+])
+def test_splits_and_maps_of_several_chunks(b, d, l, n, lens, dtype, zoh, plan):
+    log(f"case several chunks b={b} d={d} l={l} n={n} lens={lens} {dtype} zoh={zoh}")
+    assert bwd_plan(b, d, l, n, lens) == plan
+    x, dout, dlast = fused_case(2000 + l + n, b, d, l, n, dtype, lens=lens, zoh=zoh)
+    ts, out, last = run_fused(x, dout, dlast, dtype, zoh)
+    check_fused(ts, out, last, *oracle_fused(x, dout, dlast, zoh), *tol(dtype))
+
+
+@pytest.mark.parametrize("b,d,l,n,lens,zoh,plan", [
+    (4, 256, 2051, 3, None, False, (2, 4, 2)),
+    (8, 40, 4100, 3, [4100, 4096, 3600, 2561, 1, 2000, 4000, 1025], True, (5, 2, 2)),
+])
+def test_complex_splits_and_maps_of_several_chunks(b, d, l, n, lens, zoh, plan):
+    log(f"case complex several chunks b={b} d={d} l={l} n={n} lens={lens} zoh={zoh}")
+    assert bwd_plan(b, d, l, n, lens, cplx=True) == plan
+    x, dout, dlast = complex_case(4000 + l + n, b, d, l, n, lens=lens)
+    check_complex(x, dout, dlast, zoh)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("how", ["channel-outer", "one element on"])
+def test_split_rows_of_other_layouts(cplx, how):
+    """Channel-outer rows ([D][B][L]) and rows one element past an aligned address, split in time:
+    the bits of contiguous aligned ones (their rows have odd lengths: the same instance of every
+    kernel)."""
+    log(f"case split layouts cplx={cplx} {how}")
+    b, d, l, n = 2, 40, 4099, 4
+    assert bwd_plan(b, d, l, n, cplx=cplx)[0] > 1
+    g = torch.Generator(device="cuda").manual_seed(8)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x = dict(u=r(b, d, l), delta=r(b, d, l), z=r(b, d, l), B=r(b, n, l), C=r(b, n, l))
+    dout = r(b, d, l)
+    A, D, bias = -torch.exp(r(d, n)), r(d), 0.5 * r(d) - 2
+    A = torch.complex(A, 2 * r(d, n)) if cplx else A
+
+    def other(t):
+        if how == "channel-outer":
+            return t.permute(1, 0, 2).contiguous().permute(1, 0, 2)
+        buf = torch.empty(t.numel() + 1, device="cuda")
+        buf[1:].copy_(t.reshape(-1))
+        return buf[1:].view(t.shape)
+
+    def grads(form):
+        ts = {k: form(v).detach().requires_grad_(True) for k, v in x.items()}
+        out, last = selective_scan_fn(ts["u"], ts["delta"], A, ts["B"], ts["C"], D=D, z=ts["z"], delta_bias=bias,
+                                      delta_softplus=True, return_last_state=True)
+        out.backward(form(dout))
+        return [out.detach(), last, *[t.grad for t in ts.values()]]
+
+    for i, (a, w) in enumerate(zip(grads(torch.clone), grads(other))):
+        assert torch.equal(a, w), i
 
 
 @pytest.mark.parametrize("n", [16, 20])
@@ -129,8 +197,12 @@ def test_complex_backward_in_a_smaller_workspace():
                                                                   None, None, None, None, False, False)
     p = lambda v: (torch.view_as_real(v) if v.is_complex() else v).data_ptr()
     res = []
-    up = lambda v: (v + 255) // 256 * 256
-    whole = up((b * 2 * n * l + 63) // 64 * 64 * 4 * 2) + up(b * d * n * 8) + 2 * up(b * d * 4)
+    info = _lib.BwdPlanInfo()
+    dims = _lib.BwdArgs(batch=b, dim=d, seqlen=l, dstate=n)
+    split_size = int(lib.mss_cbwd_workspace_bytes(dims))
+    _lib.check(lib.mss_bwd_plan_in(dims, 1, split_size - 1, info), "mss_bwd_plan_in")
+    assert info.n_split == 1
+    whole = info.workspace_bytes
     delta = t["delta"].abs()
     for size in (None, whole):
         g = {k: torch.full_like(v, float("nan")) for k, v in dict(u=t["u"], delta=delta, A=t["A"], B=t["B"], C=t["C"]).items()}
