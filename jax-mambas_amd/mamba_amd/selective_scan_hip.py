@@ -344,12 +344,19 @@ _TENSOR_TYPES = (torch.Tensor, torch.nn.Parameter)
 def _plain_eager(*tensors):
     """Whether nothing traces, transforms or intercepts a call on these tensors, so that it may
     skip the dispatcher: no compile or jit tracing, no functorch level (vmap, grad, forward-mode),
-    no dispatch or function mode, no tensor subclass."""
+    no dispatch or function mode, no tensor subclass, no lazily negated view (the dispatcher
+    materialises those; a conjugated A or initial state is refused before this)."""
     return (not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and torch.autograd.forward_ad._current_level < 0
-            and all(t is None or type(t) in _TENSOR_TYPES for t in tensors))
+            and all(t is None or (type(t) in _TENSOR_TYPES and not t.is_neg()) for t in tensors))
+
+
+def _unflagged(*grads):
+    """Whether gradients, as autograd hands them in, are what their memory says: not lazily negated,
+    conjugated or zero."""
+    return all(g is None or not (g.is_neg() or g.is_conj() or g._is_zerotensor()) for g in grads)
 
 
 def _save_for_scan_backward(ctx, inputs, out, carries, y_pre):
@@ -374,7 +381,7 @@ def _scan_backward(ctx, dout, dlast, _dcarries=None, _dy_pre=None):
     args = (u, delta, A, B, C, D, z, delta_bias, initial_state, seq_lens, carries, y_pre, out, dout, dlast,
             ctx.delta_softplus, ctx.zoh)
     # (with create_graph the op is called, which refuses a second differentiation)
-    direct = not torch.is_grad_enabled() and _plain_eager(*args[:15])
+    direct = not torch.is_grad_enabled() and _unflagged(dout, dlast) and _plain_eager(*args[:15])
     g = _scan_bwd(*args) if direct else torch.ops.mamba_amd.selective_scan_bwd(*args)
     du, ddelta, dA, dB, dC, dD, dz, dbias, dinit = g
     pick = lambda t, given: t if given is not None else None

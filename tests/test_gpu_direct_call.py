@@ -88,3 +88,56 @@ def test_functorch_gets_the_op():
     except RuntimeError:
         return  # refused by the op, as before
     assert torch.equal(got, want)
+
+
+def test_conjugate_cotangent_of_the_last_state():
+    """A program that conjugates the last state hands back a lazily conjugated gradient, which the
+    dispatcher resolves for the op and nothing resolves for a direct call."""
+    t = _inputs(True)
+    _, last = selective_scan_fn(**t, delta_softplus=True, return_last_state=True)
+    w = torch.randn(last.shape, dtype=last.dtype, device="cuda", generator=torch.Generator("cuda").manual_seed(5))
+    leaves = [v for k, v in t.items() if k != "z"]
+    got = torch.autograd.grad((last.conj() * w).real.sum(), leaves, retain_graph=True, allow_unused=True)
+    want = torch.autograd.grad(last, leaves, w, allow_unused=True)  # d/dlast of Re(conj(last) w) is w
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+
+
+def test_negated_views():
+    """The imaginary part of a conjugate is a view whose sign is a flag: read with it, as an input
+    (one channel: contiguous at any stride) and as a gradient."""
+    t = {k: v.detach()[:, :1].contiguous() if k in ("u", "delta", "z") else v.detach() for k, v in _inputs(False).items()}
+    t["A"] = t["A"][:1]
+    for k in ("D", "delta_bias"):
+        t[k] = torch.complex(t[k][:1], -t[k][:1]).conj().imag
+        assert t[k].is_neg() and t[k].is_contiguous()
+    plain = {k: v.resolve_neg() for k, v in t.items()}
+    leaf = plain["u"].requires_grad_(True)
+    t["u"] = leaf
+    outs = [selective_scan_fn(**x, delta_softplus=True) for x in (t, plain)]
+    assert torch.equal(*outs)
+    grads = [torch.autograd.grad(torch.complex(o, o).conj().imag.sum(), leaf)[0] for o in outs]
+    assert torch.equal(*grads)
+
+
+@pytest.mark.parametrize("transform", ["vmap", "forward-mode"])
+def test_transforms_meet_the_op(transform):
+    """What vmap and forward-mode differentiation make of the op, they make of the public call."""
+    t = {k: v.detach() for k, v in _inputs(False).items()}
+    op = lambda u: torch.ops.mamba_amd.selective_scan_fwd(u, *[t[k] for k in ("delta", "A", "B", "C", "D", "z", "delta_bias")],
+                                                          None, None, True, False)[0]
+    fn = lambda u: selective_scan_fn(**{**t, "u": u}, delta_softplus=True)
+
+    def outcome(f):
+        try:
+            if transform == "vmap":
+                return torch.vmap(f)(torch.stack([t["u"], 2 * t["u"]]))
+            with torch.autograd.forward_ad.dual_level():
+                return torch.autograd.forward_ad.unpack_dual(f(torch.autograd.forward_ad.make_dual(t["u"], t["u"]))).tangent
+        except (RuntimeError, NotImplementedError) as e:
+            return type(e)
+
+    got, want = outcome(fn), outcome(op)
+    assert torch.equal(got, want) if isinstance(want, torch.Tensor) else got is want
