@@ -341,14 +341,30 @@ def _(u, delta, A, B, C, D, z, delta_bias, initial_state, seq_lens, carries, y_p
 _TENSOR_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
+def _probes():
+    """torch's own questions behind _plain_eager (private names: None where this torch lacks one, and
+    then every call takes the op)."""
+    try:
+        c = torch._C
+        torch.autograd.forward_ad._current_level
+        return (c._get_tracing_state, c._functorch.peek_interpreter_stack, c._len_torch_dispatch_stack,
+                c._len_torch_function_stack)
+    except AttributeError:
+        return None
+
+
+_PROBES = _probes()
+
+
 def _plain_eager(*tensors):
     """Whether nothing traces, transforms or intercepts a call on these tensors, so that it may
     skip the dispatcher: no compile or jit tracing, no functorch level (vmap, grad, forward-mode),
     no dispatch or function mode, no tensor subclass, no lazily negated view (the dispatcher
     materialises those; a conjugated A or initial state is refused before this)."""
-    return (not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+    if torch.compiler.is_compiling() or _PROBES is None:
+        return False
+    tracing, functorch, dispatch_modes, function_modes = _PROBES
+    return (tracing() is None and functorch() is None and dispatch_modes() == 0 and function_modes() == 0
             and torch.autograd.forward_ad._current_level < 0
             and all(t is None or (type(t) in _TENSOR_TYPES and not t.is_neg()) for t in tensors))
 

@@ -33,3 +33,9 @@ def test_other_tensors():
     for g in (conj, conj.imag, torch._efficientzerotensor((2,))):
         assert not ssh._unflagged(None, g)
     assert ssh._unflagged(torch.randn(2), None)
+
+
+def test_a_torch_without_these_internals_takes_the_op(monkeypatch):
+    monkeypatch.delattr(torch._C, "_len_torch_dispatch_stack")
+    monkeypatch.setattr(ssh, "_PROBES", ssh._probes())
+    assert not ssh._plain_eager(torch.randn(2))
