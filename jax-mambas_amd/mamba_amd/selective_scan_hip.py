@@ -348,7 +348,7 @@ def _probes():
         c = torch._C
         torch.autograd.forward_ad._current_level
         return (c._get_tracing_state, c._functorch.peek_interpreter_stack, c._len_torch_dispatch_stack,
-                c._len_torch_function_stack)
+                c._len_torch_function_stack, c._autograd._profiler_enabled)
     except AttributeError:
         return None
 
@@ -359,13 +359,13 @@ _PROBES = _probes()
 def _plain_eager(*tensors):
     """Whether nothing traces, transforms or intercepts a call on these tensors, so that it may
     skip the dispatcher: no compile or jit tracing, no functorch level (vmap, grad, forward-mode),
-    no dispatch or function mode, no tensor subclass, no lazily negated view (the dispatcher
+    no dispatch or function mode, no profiler (which names ops), no tensor subclass, no lazily negated view (the dispatcher
     materialises those; a conjugated A or initial state is refused before this)."""
     if torch.compiler.is_compiling() or _PROBES is None:
         return False
-    tracing, functorch, dispatch_modes, function_modes = _PROBES
+    tracing, functorch, dispatch_modes, function_modes, profiling = _PROBES
     return (tracing() is None and functorch() is None and dispatch_modes() == 0 and function_modes() == 0
-            and torch.autograd.forward_ad._current_level < 0
+            and not profiling() and torch.autograd.forward_ad._current_level < 0
             and all(t is None or (type(t) in _TENSOR_TYPES and not t.is_neg()) for t in tensors))
 
 

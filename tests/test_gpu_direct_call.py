@@ -141,3 +141,10 @@ def test_transforms_meet_the_op(transform):
 
     got, want = outcome(fn), outcome(op)
     assert torch.equal(got, want) if isinstance(want, torch.Tensor) else got is want
+
+
+def test_a_profiler_sees_the_op():
+    t = _inputs(False)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        selective_scan_fn(**t, delta_softplus=True)
+    assert any(e.key == "mamba_amd::selective_scan_fwd" for e in prof.key_averages())

@@ -20,6 +20,8 @@ def test_intercepted():
     torch.func.grad(lambda v: (seen.append(ssh._plain_eager(x)), v.sum())[1])(x)
     torch.vmap(lambda v: (seen.append(ssh._plain_eager(x)), v)[1])(x)
     assert seen == [False, False]
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        assert not ssh._plain_eager(x)
     assert ssh._plain_eager(x)
 
 
