@@ -4,6 +4,7 @@ import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
 
+from mamba_amd import selective_scan_hip as ssh
 from mamba_amd.selective_scan_hip import selective_scan_fn
 
 pytestmark = pytest.mark.gpu
@@ -78,16 +79,18 @@ def test_saved_tensor_hooks_see_the_residuals():
     assert t["u"].grad is not None
 
 
-def test_functorch_gets_the_op():
+def test_functorch_gets_the_op(monkeypatch):
+    """torch.func.grad is refused by the op's autograd (a function without setup_context), as when
+    the op is called by name; the direct path is not taken."""
     t = {k: v.detach() for k, v in _inputs(False).items()}
+    for name in ("_Scan", "_scan_fwd"):  # what a direct call would reach (the op refuses before its kernel)
+        monkeypatch.setattr(ssh, name, None)
     f = lambda u: selective_scan_fn(**{**t, "u": u}, delta_softplus=True).sum()
-    u = t["u"].clone().requires_grad_(True)
-    (want,) = torch.autograd.grad(f(u), [u])
-    try:
-        got = torch.func.grad(f)(t["u"])
-    except RuntimeError:
-        return  # refused by the op, as before
-    assert torch.equal(got, want)
+    op = lambda u: torch.ops.mamba_amd.selective_scan_fwd(u, *[t[k] for k in ("delta", "A", "B", "C", "D", "z", "delta_bias")],
+                                                          None, None, True, False)[0].sum()
+    for call in (f, op):
+        with pytest.raises(RuntimeError, match="setup_context"):
+            torch.func.grad(call)(t["u"])
 
 
 def test_conjugate_cotangent_of_the_last_state():
