@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
         const float* pq = p.split_msg + (chan * N + lane) * 2;
 #pragma unroll 4
         for (int m = m_end - 1; m >= c_lo / p.chunks_per_msg; --m)
-          mu0 = __builtin_fmaf(pq[m * m_ld], mu0, pq[m * m_ld + 1]);
+          mu0 = through_map(pq[m * m_ld], pq[m * m_ld + 1], mu0);
       }
       s_mu[cl][lane] = mu0;
       s_dA[cl][lane] = 0.f;

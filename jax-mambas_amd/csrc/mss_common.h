@@ -136,6 +136,21 @@ __device__ __forceinline__ int row_longest_first(const int* __restrict__ seq_len
   return hit ? __builtin_amdgcn_readfirstlane(__ffsll(static_cast<long long>(hit)) - 1) : rank;
 }
 
+// A state (or adjoint) h through a time split, whose map is h -> P h + H. The product P of that many
+// a_bar may overflow where nothing grows because h is zero: zero stays zero then, as it does step
+// by step.
+__device__ __forceinline__ float through_map(float P, float H, float h) {
+  return h == 0.f ? H : __builtin_fmaf(P, h, H);
+}
+// The same for complex values: map = (Re P, Im P, Re H, Im H).
+__device__ __forceinline__ void through_map(const float4& map, float& hr, float& hi) {
+  const bool zero = hr == 0.f && hi == 0.f;
+  const float nr = __builtin_fmaf(map.x, hr, __builtin_fmaf(-map.y, hi, map.z));
+  const float ni = __builtin_fmaf(map.x, hi, __builtin_fmaf(map.y, hr, map.w));
+  hr = zero ? map.z : nr;
+  hi = zero ? map.w : ni;
+}
+
 // ---------------------------------------------------------------------------------
 // Scalar math.
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

@@ -150,13 +150,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
       const float4* map = reinterpret_cast<const float4*>(p.split_map) + chan * N + lane;
       const size_t m_ld = static_cast<size_t>(p.batch) * p.dim * N;
       const int m_end = min(static_cast<int>(blockIdx.z), (n_live + p.chunks_per_split - 1) / p.chunks_per_split);
-      for (int m = 0; m < m_end; ++m) {
-        const float4 ph = map[m * m_ld];
-        const float nr = __builtin_fmaf(ph.x, run_r, __builtin_fmaf(-ph.y, run_i, ph.z));
-        const float ni = __builtin_fmaf(ph.x, run_i, __builtin_fmaf(ph.y, run_r, ph.w));
-        run_r = nr;
-        run_i = ni;
-      }
+      for (int m = 0; m < m_end; ++m) through_map(map[m * m_ld], run_r, run_i);
     }
   }
   for (int c = c_lo; c < c_end; ++c) {
@@ -559,13 +553,7 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
       const float4* pq = reinterpret_cast<const float4*>(p.split_msg) + (static_cast<size_t>(b) * p.dim + d) * N + n;
       const size_t m_ld = static_cast<size_t>(p.batch) * p.dim * N;
       const int m_end = (n_live - p.chunks_per_split + p.chunks_per_msg - 1) / p.chunks_per_msg;
-      for (int m = m_end - 1; m >= c_lo / p.chunks_per_msg; --m) {
-        const float4 x = pq[m * m_ld];
-        const float nr = __builtin_fmaf(x.x, mr, __builtin_fmaf(-x.y, mi, x.z));
-        const float ni = __builtin_fmaf(x.x, mi, __builtin_fmaf(x.y, mr, x.w));
-        mr = nr;
-        mi = ni;
-      }
+      for (int m = m_end - 1; m >= c_lo / p.chunks_per_msg; --m) through_map(pq[m * m_ld], mr, mi);
     }
     s_mu[k][n][0] = mr;
     s_mu[k][n][1] = mi;

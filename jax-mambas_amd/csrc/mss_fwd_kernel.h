@@ -149,7 +149,7 @@ void fwd_kernel(FwdParams p) {
       const float* map = p.split_map + (chan * N + n) * 2;
       const int m_end = min(static_cast<int>(blockIdx.z), (n_active_chunks + p.chunks_per_split - 1) / p.chunks_per_split);
 #pragma unroll 4
-      for (int m = 0; m < m_end; ++m) h0 = __builtin_fmaf(map[m * m_ld], h0, map[m * m_ld + 1]);
+      for (int m = 0; m < m_end; ++m) h0 = through_map(map[m * m_ld], map[m * m_ld + 1], h0);
     }
     s_run[w][n] = h0;
     const float an = p.A[static_cast<size_t>(d) * N + n];

@@ -250,3 +250,42 @@ def test_reference_backward_split_in_time(b, d, l, n):
     for name, o, w, g in zip(["dA", "ddeltas", "dBs", "dCs", "du", "dinitial_x"], *res, grads):
         assert torch.equal(o, w), name
         close(name, o if o.shape == g.shape else o.transpose(1, 2), g, scale=ab.get(name))
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("backward", [False, True])
+def test_growth_over_a_split_from_nothing(cplx, backward):
+    """A growing state (Re A > 0) that is zero, and an adjoint that is zero, stay zero over a split
+    or map whose product of a_bar overflows float32 (e^120; a chunk's e^60 does not): the outputs of
+    the same call with those steps' delta zero."""
+    b, d, l, n = ((8, 40, 4100, 3) if cplx else (1, 768, 12000, 1)) if backward else ((1, 256, 4096, 2) if cplx else (1, 500, 4096, 4))
+    if backward:
+        assert bwd_plan(b, d, l, n, cplx=cplx)[2] == 2
+        still = slice(3072, 4096) if cplx else slice(10240, 11264)  # the two chunks of a map
+    else:
+        lib = _lib.register_hip_kernel()
+        a = _lib.FwdArgs(batch=b, dim=d, seqlen=l, dstate=n)
+        per = (2, 4) if cplx else (3, 2)  # chunks of a split, floats of a map
+        need = (lib.mss_cfwd_workspace_bytes if cplx else lib.mss_fwd_workspace_bytes)(a)
+        assert need == (-(-(l // 512) // per[0]) - 1) * b * d * n * per[1] * 4
+        still = slice(0, per[0] * 512)
+    log(f"case growth cplx={cplx} backward={backward}")
+    g = torch.Generator(device="cuda").manual_seed(21)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    u, delta, B, C, dout = r(b, d, l), 1e-3 * r(b, d, l).abs(), r(b, n, l), r(b, n, l), r(b, d, l)
+    A = torch.full((d, n), 60 / 512, device="cuda")
+    A = torch.complex(A, r(d, n)) if cplx else A
+    if backward:
+        u.zero_()
+        dout[..., still.start:] = 0
+    else:
+        u[..., still] = 0
+    res = []
+    for step in (0.0, 1.0):
+        delta[..., still] = step
+        leaves = [t.clone().requires_grad_(backward) for t in (u, delta, A, B, C)]
+        out, last = selective_scan_fn(*leaves, return_last_state=True)
+        res.append([out, last, *(torch.autograd.grad(out, leaves, dout) if backward else ())])
+    for i, (want, got) in enumerate(zip(*res)):
+        want, got = (torch.view_as_real(t.detach()) if t.is_complex() else t.detach() for t in (want, got))
+        assert bool(torch.isfinite(want).all()) and torch.equal(got, want), i
