@@ -138,12 +138,14 @@ __device__ __forceinline__ void stage_chunk(const bc_t* __restrict__ Bb, const b
 // full tensors, p.a_ld / p.state_ld / p.carry_cs; dz only where p.dz is given); 2 = a later
 // group (as 1, and du/ddelta add to the values already in their buffers).
 //
-// kWhole: L is a multiple of the chunk and the B/C rows can be copied to LDS directly, so no
-// lane ever meets the row's end (those paths' registers spill the 16-wave kernel). Measured on
-// MI355X (B=8 D=2048 L=4096 bf16): 871 us with every row loaded and unpacked by itself, so that
-// five memory latencies followed one another, 798 with the rows fetched together; the general
-// instance 887 there. B=3 D=1000 L=2051 bf16: 225 us with element-wise accesses, 144.
-template <int kW, bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup, bool kWhole>
+// kRows, as in the forward: kWholeRows where L is a multiple of the chunk and the B/C rows can be
+// copied to LDS directly, so that no lane ever meets the row's end (those paths' registers spill the
+// 16-wave kernel). Measured on MI355X (B=8 D=2048 L=4096 bf16): 871 us with every row loaded and
+// unpacked by itself, so that five memory latencies followed one another, 807 with the rows fetched
+// together; the general instance 887 there. kSlotRows: L=4032 850 us, the general instance 894;
+// L=4096 with float32 B/C 815 and 875. kAnyRows: B=3 D=1000 L=2051 bf16 225 us with element-wise
+// accesses, 144.
+template <int kW, bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup, int kRows>
 __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
   constexpr bool kAcc = kGroup == 2;
   constexpr int kT = kBwdT;
@@ -177,7 +179,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
   const long long carry_cs = kGroup ? p.carry_cs : static_cast<long long>(N) * p.n_seg;
   const bool has_dz = kGroup ? p.dz != nullptr : true;  // (z given: dz given, ungrouped)
   const int len = p.seq_lens ? min(max(p.seq_lens[b], 0), L) : L;
-  const bool dma = kWhole || p.vec_bc != 0;
+  const bool dma = kRows != kAnyRows || p.vec_bc != 0;
   const bc_t* __restrict__ Bb = static_cast<const bc_t*>(p.B) + b * p.bc_sb;
   const bc_t* __restrict__ Cb = static_cast<const bc_t*>(p.C) + b * p.bc_sb;
 
@@ -238,9 +240,9 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
   for (int c = c_end - 1; c >= c_lo; --c) {
     const int t0 = c * kChunk;
     const int tl = t0 + seg * kT;  // first step of this lane's segment
-    const bool fast = kWhole || t0 + kChunk <= L;  // wave-uniform
+    const bool fast = kRows == kWholeRows || t0 + kChunk <= L;  // wave-uniform
     const int seg_idx = t0 / kT + seg;               // index into a carries row
-    const bool seg_ok = kWhole || seg_idx < p.n_seg;
+    const bool seg_ok = kRows == kWholeRows || seg_idx < p.n_seg;
 
     if (c >= n_live) {
       // Whole chunk past this row's length: zero gradients; the adjoint message passes
@@ -254,11 +256,11 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
 #pragma unroll
         for (int j = 0; j < kT; ++j) zero[j] = 0.f;
         if constexpr (!kAcc) {  // (accumulating: adding zero changes nothing)
-          store_seg<kT>(static_cast<io_t*>(p.du) + row, tl, L, fast, zero);
-          store_seg<kT>(static_cast<io_t*>(p.ddelta) + row, tl, L, fast, zero);
+          store_seg<kT>(static_cast<io_t*>(p.du) + row, tl, L, fast, zero, kRows);
+          store_seg<kT>(static_cast<io_t*>(p.ddelta) + row, tl, L, fast, zero, kRows);
         }
         if constexpr (kHasZ)
-          if (has_dz) store_seg<kT>(static_cast<io_t*>(p.dz) + row, tl, L, fast, zero);
+          if (has_dz) store_seg<kT>(static_cast<io_t*>(p.dz) + row, tl, L, fast, zero, kRows);
         if (c == 0 && p.dinit && lane < N)
           p.dinit[(static_cast<size_t>(b) * p.dim + d) * st_ld + lane] = s_mu[cl][lane];
       }
@@ -293,23 +295,23 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
         // the last channel reads the clamped channel's row and never stores or accumulates.
         // All rows are fetched before the first is used: one memory latency.
         Seg<kT, io_t> sd, su, sg, sz_, so;
-        fetch(sd, static_cast<const io_t*>(p.delta) + row, tl, L, kWhole);
-        fetch(su, static_cast<const io_t*>(p.u) + row, tl, L, kWhole);
-        fetch(sg, static_cast<const io_t*>(p.dout) + row, tl, L, kWhole);
+        fetch(sd, static_cast<const io_t*>(p.delta) + row, tl, L, kRows);
+        fetch(su, static_cast<const io_t*>(p.u) + row, tl, L, kRows);
+        fetch(sg, static_cast<const io_t*>(p.dout) + row, tl, L, kRows);
         if constexpr (kHasZ) {
-          fetch(sz_, static_cast<const io_t*>(p.z) + row, tl, L, kWhole);
-          fetch(so, static_cast<const io_t*>(p.out) + row, tl, L, kWhole);
+          fetch(sz_, static_cast<const io_t*>(p.z) + row, tl, L, kRows);
+          fetch(so, static_cast<const io_t*>(p.out) + row, tl, L, kRows);
         }
-        finish(sd, tl, L, fast, dlt);
-        finish(su, tl, L, fast, uu);
-        finish(sg, tl, L, fast, g);
+        finish(sd, tl, L, fast, dlt, kRows);
+        finish(su, tl, L, fast, uu, kRows);
+        finish(sg, tl, L, fast, g, kRows);
         if constexpr (kHasZ) {
           // g = dout * silu(z); dz = dout * y * sigmoid(z) * (1 + z * (1 - sigmoid(z))). With the
           // forward's out = y z sigmoid(z): dz = dout * out * (1 / z + 1 - sigmoid(z)), and where
           // |z| < kZTiny (out / z imprecise) y itself, which the forward kept there.
           float zr[kT], yp[kT];
-          finish(sz_, tl, L, fast, zr);
-          finish(so, tl, L, fast, yp);
+          finish(sz_, tl, L, fast, zr, kRows);
+          finish(so, tl, L, fast, yp, kRows);
           const io_t* __restrict__ ykept = static_cast<const io_t*>(p.y_pre) + row;
 #pragma unroll
           for (int j = 0; j < kT; ++j) {
@@ -322,7 +324,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
             yp[j] = valid ? d : 0.f;
             g[j] = go * zr[j] * sz;
           }
-          if (active && has_dz) store_seg<kT>(static_cast<io_t*>(p.dz) + row, tl, L, fast, yp);
+          if (active && has_dz) store_seg<kT>(static_cast<io_t*>(p.dz) + row, tl, L, fast, yp, kRows);
         }
 #pragma unroll
         for (int j = 0; j < kT; ++j) {
@@ -458,7 +460,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       // ---- per-step gradients of the row
       if constexpr (!kZOH) {
         // Euler needs u only from here on: reload it rather than hold it across the loop.
-        load_seg<kT>(static_cast<const io_t*>(p.u) + row, tl, L, fast, uu, kWhole);
+        load_seg<kT>(static_cast<const io_t*>(p.u) + row, tl, L, fast, uu, kRows);
       }
       float dD_acc = 0.f, db_acc = 0.f;
       float duv[kT], ddv[kT];
@@ -487,15 +489,15 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       }
       if constexpr (kAcc) {
         float prev[kT];
-        load_seg<kT>(static_cast<const io_t*>(p.du) + row, tl, L, fast, prev, kWhole);
+        load_seg<kT>(static_cast<const io_t*>(p.du) + row, tl, L, fast, prev, kRows);
 #pragma unroll
         for (int j = 0; j < kT; ++j) duv[j] += prev[j];
-        load_seg<kT>(static_cast<const io_t*>(p.ddelta) + row, tl, L, fast, prev, kWhole);
+        load_seg<kT>(static_cast<const io_t*>(p.ddelta) + row, tl, L, fast, prev, kRows);
 #pragma unroll
         for (int j = 0; j < kT; ++j) ddv[j] += prev[j];
       }
-      store_seg<kT>(static_cast<io_t*>(p.du) + row, tl, L, fast, duv);
-      store_seg<kT>(static_cast<io_t*>(p.ddelta) + row, tl, L, fast, ddv);
+      store_seg<kT>(static_cast<io_t*>(p.du) + row, tl, L, fast, duv, kRows);
+      store_seg<kT>(static_cast<io_t*>(p.ddelta) + row, tl, L, fast, ddv, kRows);
       const float dD_sum = wave_sum_to_last(dD_acc);
       const float db_sum = wave_sum_to_last(db_acc);
       if (lane == 63) {
@@ -531,7 +533,7 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       }
       const int t = t0 + (63 - ln) * kT + 4 * qq;
       float* dst = part + which * nl + static_cast<size_t>(n) * L + t;
-      store_seg<4>(dst - t, t, L, kWhole, v);
+      store_seg<4>(dst - t, t, L, kRows == kWholeRows, v, kRows);
     }
     wait_vmem_all();
     __syncthreads();
@@ -733,15 +735,15 @@ __global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ p
   }
 }
 
-template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup, bool kWhole>
+template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup, int kRows>
 static hipError_t launch_bwd_w(const BwdParams& p, hipStream_t stream) {
   dim3 grid(p.n_blocks_d, p.batch, p.n_split);
   if (p.waves == 16) {
     if (!bwd_waves_fit(16, p.dstate) || p.chan_per_block % 16 != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((bwd_kernel<16, kZOH, kHasZ, io_t, bc_t, kGroup, kWhole>), grid, dim3(16 * 64), 0, stream, p);
+    hipLaunchKernelGGL((bwd_kernel<16, kZOH, kHasZ, io_t, bc_t, kGroup, kRows>), grid, dim3(16 * 64), 0, stream, p);
   } else {
     if (p.waves != 12 || p.chan_per_block % 12 != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((bwd_kernel<12, kZOH, kHasZ, io_t, bc_t, kGroup, kWhole>), grid, dim3(12 * 64), 0, stream, p);
+    hipLaunchKernelGGL((bwd_kernel<12, kZOH, kHasZ, io_t, bc_t, kGroup, kRows>), grid, dim3(12 * 64), 0, stream, p);
   }
   return hipGetLastError();
 }
@@ -750,9 +752,11 @@ template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup>
 static hipError_t launch_bwd_a(const BwdParams& p, hipStream_t stream) {
   if constexpr (kGroup == 0 && sizeof(io_t) == sizeof(bc_t)) {
     if (p.vec_bc && p.seqlen % kBwdChunk == 0)
-      return launch_bwd_w<kZOH, kHasZ, io_t, bc_t, kGroup, true>(p, stream);
+      return launch_bwd_w<kZOH, kHasZ, io_t, bc_t, kGroup, kWholeRows>(p, stream);
   }
-  return launch_bwd_w<kZOH, kHasZ, io_t, bc_t, kGroup, false>(p, stream);
+  if (p.vec_bc && slots_fit<io_t>(p.seqlen))
+    return launch_bwd_w<kZOH, kHasZ, io_t, bc_t, kGroup, kSlotRows>(p, stream);
+  return launch_bwd_w<kZOH, kHasZ, io_t, bc_t, kGroup, kAnyRows>(p, stream);
 }
 
 template <bool kZOH, bool kHasZ, typename io_t, typename bc_t>

@@ -113,7 +113,7 @@ __device__ __forceinline__ void wave_scan_caffine(float& pr, float& pi, float& h
 // (run_r, run_i). kG > 1: that many waves share a channel, each taking every kG-th state, their
 // outputs added in order through LDS at the end of a chunk; the row may be split in time as well
 // (FwdParams::split_map, here complex: [n_split - 1][batch][dim][dstate][P re, im, H re, im]).
-template <bool kZOH, typename io_t, typename bc_t, bool kWhole, int kG>
+template <bool kZOH, typename io_t, typename bc_t, int kRows, int kG>
 __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -156,23 +156,23 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
   for (int c = c_lo; c < c_end; ++c) {
     const int t0 = c * kCChunk;
     const int tl = t0 + lane * kCT;
-    const bool fast = kWhole || t0 + kCChunk <= L;
+    const bool fast = kRows == kWholeRows || t0 + kCChunk <= L;
     float y[kCT];
     if (c >= n_live) {
       // The whole chunk is past this row's length: the state is frozen, the output zero
       // (the backward reads no residual here, so y_pre is left unwritten).
 #pragma unroll
       for (int j = 0; j < kCT; ++j) y[j] = 0.f;
-      if (grp == 0) store_seg<kCT>(out_row, tl, L, fast, y);
+      if (grp == 0) store_seg<kCT>(out_row, tl, L, fast, y, kRows);
       continue;
     }
     float dlt[kCT], uu[kCT];
     float ssum = 0.f;
     Seg<kCT, io_t> sd, su;
-    fetch(sd, dl_row, tl, L, kWhole);
-    fetch(su, u_row, tl, L, kWhole);
-    finish(sd, tl, L, fast, dlt);
-    finish(su, tl, L, fast, uu);
+    fetch(sd, dl_row, tl, L, kRows);
+    fetch(su, u_row, tl, L, kRows);
+    finish(sd, tl, L, fast, dlt, kRows);
+    finish(su, tl, L, fast, uu, kRows);
 #pragma unroll
     for (int j = 0; j < kCT; ++j) {
       const bool valid = tl + j < len;
@@ -186,18 +186,18 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
     // B and C rows of the next state are loaded one state ahead.
     Seg<kCT, bc_t> sbn, scn;
     if (grp < N) {
-      fetch(sbn, Bb + grp * p.bc_sn, tl, L, kWhole);
-      fetch(scn, Cb + grp * p.bc_sn, tl, L, kWhole);
+      fetch(sbn, Bb + grp * p.bc_sn, tl, L, kRows);
+      fetch(scn, Cb + grp * p.bc_sn, tl, L, kRows);
     }
     for (int n = grp; n < N; n += kG) {
       const CoefA cf = load_coef(p.A, static_cast<size_t>(d) * N + n);
       float ar[kCT], ai[kCT], br[kCT], bi[kCT];
       float bv[kCT], cv[kCT];
-      finish(sbn, tl, L, fast, bv);
-      finish(scn, tl, L, fast, cv);
+      finish(sbn, tl, L, fast, bv, kRows);
+      finish(scn, tl, L, fast, cv, kRows);
       if (n + kG < N) {
-        fetch(sbn, Bb + (n + kG) * p.bc_sn, tl, L, kWhole);
-        fetch(scn, Cb + (n + kG) * p.bc_sn, tl, L, kWhole);
+        fetch(sbn, Bb + (n + kG) * p.bc_sn, tl, L, kRows);
+        fetch(scn, Cb + (n + kG) * p.bc_sn, tl, L, kRows);
       }
       float hr = 0.f, hi = 0.f;
       {
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
         xr = rr;
         xi = ri;
       }
-      if (p.carries && (kWhole || tl < L)) {
+      if (p.carries && (kRows == kWholeRows || tl < L)) {
         float2* cp = reinterpret_cast<float2*>(p.carries) + (chan * N + n) * p.n_seg + tl / kCT;
         *cp = make_float2(xr, xi);
       }
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
       if (p.z) {
 #pragma unroll
         for (int e = 0; e < kV; ++e)
-          zv[e] = (kWhole || t + e < L) ? to_f32((static_cast<const io_t*>(p.z) + row)[t + e]) : 0.f;
+          zv[e] = (kRows == kWholeRows || t + e < L) ? to_f32((static_cast<const io_t*>(p.z) + row)[t + e]) : 0.f;
       }
       __syncthreads();  // the previous chunk's partial outputs have been read
 #pragma unroll
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
 #pragma unroll
         for (int q = 0; q < kG; ++q) v += s_y[q][(tc + e) % kCT][(tc + e) / kCT];
         v = t + e < len ? v : 0.f;
-        if (kWhole || t + e < L) {
+        if (kRows == kWholeRows || t + e < L) {
           if (p.z) {
             if (p.y_pre) store_as(static_cast<io_t*>(p.y_pre) + row + t + e, v);
             v = t + e < len ? v * (zv[e] * sigmoid(zv[e])) : 0.f;
@@ -291,16 +291,16 @@ __global__ __launch_bounds__(kCFwdW * 64) void cfwd_kernel(FwdParams p) {
         float yp[kCT];
 #pragma unroll
         for (int j = 0; j < kCT; ++j) yp[j] = (tl + j < len) ? y[j] : 0.f;
-        store_seg<kCT>(static_cast<io_t*>(p.y_pre) + row, tl, L, fast, yp);
+        store_seg<kCT>(static_cast<io_t*>(p.y_pre) + row, tl, L, fast, yp, kRows);
       }
       float zv[kCT];
-      load_seg<kCT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zv, kWhole);
+      load_seg<kCT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zv, kRows);
 #pragma unroll
       for (int j = 0; j < kCT; ++j) y[j] *= zv[j] * sigmoid(zv[j]);
     }
 #pragma unroll
     for (int j = 0; j < kCT; ++j) y[j] = (tl + j < len) ? y[j] : 0.f;
-    store_seg<kCT>(out_row, tl, L, fast, y);
+    store_seg<kCT>(out_row, tl, L, fast, y, kRows);
   }
   if (p.last && lane < N && c_end == n_chunks && lane % kG == grp) {
     p.last[(chan * N + lane) * 2] = run_r;
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(kCMapW * 64) void cbwd_msg_kernel(BwdParams p) {
 // counted that iteration done in LDS (no workgroup barrier per iteration). After every
 // chunk the rows (copies summed in order) go to this workgroup's partial rows; a second
 // kernel sums the partials over workgroups in a fixed order.
-template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, bool kWhole>
+template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kRows>
 __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
   constexpr int W = kCBwdW;
   __shared__ __attribute__((aligned(16))) float s_acc[kCAccRows][2][kCChunk];
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
   for (int c = c_end - 1; c >= c_lo; --c) {
     const int t0 = c * kCChunk;
     const int ts = t0 + seg * kCT;
-    const bool fast = kWhole || t0 + kCChunk <= L;
+    const bool fast = kRows == kWholeRows || t0 + kCChunk <= L;
     const bool live = c < n_live;  // workgroup-uniform
     for (int r = 0; r < rounds; ++r) {
       const int k = r * W + w;
@@ -592,9 +592,9 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
           float zero[kCT];
 #pragma unroll
           for (int j = 0; j < kCT; ++j) zero[j] = 0.f;
-          store_seg<kCT>(du_row, ts, L, fast, zero);
-          store_seg<kCT>(ddl_row, ts, L, fast, zero);
-          if constexpr (kHasZ) store_seg<kCT>(static_cast<io_t*>(p.dz) + row, ts, L, fast, zero);
+          store_seg<kCT>(du_row, ts, L, fast, zero, kRows);
+          store_seg<kCT>(ddl_row, ts, L, fast, zero, kRows);
+          if constexpr (kHasZ) store_seg<kCT>(static_cast<io_t*>(p.dz) + row, ts, L, fast, zero, kRows);
         }
         continue;
       }
@@ -602,16 +602,16 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
       const float bias = p.delta_bias ? p.delta_bias[dd] : 0.f;
       float xraw[kCT], dlt[kCT], uu[kCT], g[kCT];
       Seg<kCT, io_t> sd, su, sg, sz_, sy;
-      fetch(sd, static_cast<const io_t*>(p.delta) + row, ts, L, kWhole);
-      fetch(su, static_cast<const io_t*>(p.u) + row, ts, L, kWhole);
-      fetch(sg, static_cast<const io_t*>(p.dout) + row, ts, L, kWhole);
+      fetch(sd, static_cast<const io_t*>(p.delta) + row, ts, L, kRows);
+      fetch(su, static_cast<const io_t*>(p.u) + row, ts, L, kRows);
+      fetch(sg, static_cast<const io_t*>(p.dout) + row, ts, L, kRows);
       if constexpr (kHasZ) {
-        fetch(sz_, static_cast<const io_t*>(p.z) + row, ts, L, kWhole);
-        fetch(sy, static_cast<const io_t*>(p.y_pre) + row, ts, L, kWhole);
+        fetch(sz_, static_cast<const io_t*>(p.z) + row, ts, L, kRows);
+        fetch(sy, static_cast<const io_t*>(p.y_pre) + row, ts, L, kRows);
       }
-      finish(sd, ts, L, fast, xraw);
-      finish(su, ts, L, fast, uu);
-      finish(sg, ts, L, fast, g);
+      finish(sd, ts, L, fast, xraw, kRows);
+      finish(su, ts, L, fast, uu, kRows);
+      finish(sg, ts, L, fast, g, kRows);
       float ssum = 0.f;
 #pragma unroll
       for (int j = 0; j < kCT; ++j) {
@@ -625,15 +625,15 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
       }
       if constexpr (kHasZ) {
         float zv[kCT], yp[kCT], dz[kCT];
-        finish(sz_, ts, L, fast, zv);
-        finish(sy, ts, L, fast, yp);
+        finish(sz_, ts, L, fast, zv, kRows);
+        finish(sy, ts, L, fast, yp, kRows);
 #pragma unroll
         for (int j = 0; j < kCT; ++j) {
           const float sz = sigmoid(zv[j]);
           dz[j] = g[j] * yp[j] * sz * __builtin_fmaf(zv[j], 1.f - sz, 1.f);
           g[j] = g[j] * zv[j] * sz;
         }
-        if (active) store_seg<kCT>(static_cast<io_t*>(p.dz) + row, ts, L, fast, dz);
+        if (active) store_seg<kCT>(static_cast<io_t*>(p.dz) + row, ts, L, fast, dz, kRows);
       }
       float du[kCT], ddl[kCT];
 #pragma unroll
@@ -652,9 +652,9 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
       float2 hnx = make_float2(0.f, 0.f);
       if (kAhead && active) {
         const int n0 = w % N;
-        fetch(sbn, Bb + n0 * p.bc_sn, ts, L, kWhole);
-        fetch(scn, Cb + n0 * p.bc_sn, ts, L, kWhole);
-        if (kWhole || ts < L) hnx = carry_seg[static_cast<size_t>(n0) * p.n_seg];
+        fetch(sbn, Bb + n0 * p.bc_sn, ts, L, kRows);
+        fetch(scn, Cb + n0 * p.bc_sn, ts, L, kRows);
+        if (kRows == kWholeRows || ts < L) hnx = carry_seg[static_cast<size_t>(n0) * p.n_seg];
       }
       for (int it = 0; it < N; ++it) {
         const int n = (it + w) % N;
@@ -664,20 +664,20 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
           float bv[kCT], cv[kCT];
           float hinr, hini;
           if constexpr (kAhead) {
-            finish(sbn, ts, L, fast, bv);
-            finish(scn, ts, L, fast, cv);
+            finish(sbn, ts, L, fast, bv, kRows);
+            finish(scn, ts, L, fast, cv, kRows);
             hinr = hnx.x;
             hini = hnx.y;
             if (it + 1 < N) {
               const int nn = (it + 1 + w) % N;
-              fetch(sbn, Bb + nn * p.bc_sn, ts, L, kWhole);
-              fetch(scn, Cb + nn * p.bc_sn, ts, L, kWhole);
-              if (kWhole || ts < L) hnx = carry_seg[static_cast<size_t>(nn) * p.n_seg];
+              fetch(sbn, Bb + nn * p.bc_sn, ts, L, kRows);
+              fetch(scn, Cb + nn * p.bc_sn, ts, L, kRows);
+              if (kRows == kWholeRows || ts < L) hnx = carry_seg[static_cast<size_t>(nn) * p.n_seg];
             }
           } else {
-            load_seg<kCT>(Bb + n * p.bc_sn, ts, L, fast, bv, kWhole);
-            load_seg<kCT>(Cb + n * p.bc_sn, ts, L, fast, cv, kWhole);
-            const float2 h0 = kWhole || ts < L ? carry_seg[static_cast<size_t>(n) * p.n_seg] : make_float2(0.f, 0.f);
+            load_seg<kCT>(Bb + n * p.bc_sn, ts, L, fast, bv, kRows);
+            load_seg<kCT>(Cb + n * p.bc_sn, ts, L, fast, cv, kRows);
+            const float2 h0 = kRows == kWholeRows || ts < L ? carry_seg[static_cast<size_t>(n) * p.n_seg] : make_float2(0.f, 0.f);
             hinr = h0.x;
             hini = h0.y;
           }
@@ -836,8 +836,8 @@ __global__ __launch_bounds__(kCBwdW * 64) void cbwd_kernel(BwdParams p) {
           dsum += dx;
           gsum = __builtin_fmaf(g[j], uu[j], gsum);
         }
-        store_seg<kCT>(du_row, ts, L, fast, du);
-        store_seg<kCT>(ddl_row, ts, L, fast, ddl);
+        store_seg<kCT>(du_row, ts, L, fast, du, kRows);
+        store_seg<kCT>(ddl_row, ts, L, fast, ddl, kRows);
         const float sd = wave_sum(gsum), sb = wave_sum(dsum);
         if (lane == 0) {
           s_dD[k] += sd;
@@ -987,11 +987,14 @@ static hipError_t launch_cfwd_g(const FwdParams& p, hipStream_t stream) {
   const dim3 grid((p.dim + kChan - 1) / kChan, p.batch, kG > 1 ? p.n_split : 1);
   if constexpr (sizeof(io_t) == sizeof(bc_t)) {
     if (p.seqlen % kCChunk == 0) {
-      hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, true, kG>), grid, dim3(kCFwdW * 64), 0, stream, p);
+      hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, kWholeRows, kG>), grid, dim3(kCFwdW * 64), 0, stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, false, kG>), grid, dim3(kCFwdW * 64), 0, stream, p);
+  if (slots_fit<io_t>(p.seqlen) && slots_fit<bc_t>(p.seqlen))
+    hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, kSlotRows, kG>), grid, dim3(kCFwdW * 64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((cfwd_kernel<kZOH, io_t, bc_t, kAnyRows, kG>), grid, dim3(kCFwdW * 64), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -1057,11 +1060,14 @@ static hipError_t launch_cbwd_t(const BwdParams& p, hipStream_t stream) {
   dim3 grid(p.n_blocks_d, p.batch, p.n_split);
   if constexpr (sizeof(io_t) == sizeof(bc_t)) {
     if (p.seqlen % kCChunk == 0) {
-      hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t, true>), grid, dim3(kCBwdW * 64), 0, stream, p);
+      hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t, kWholeRows>), grid, dim3(kCBwdW * 64), 0, stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t, false>), grid, dim3(kCBwdW * 64), 0, stream, p);
+  if (slots_fit<io_t>(p.seqlen) && slots_fit<bc_t>(p.seqlen))
+    hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t, kSlotRows>), grid, dim3(kCBwdW * 64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((cbwd_kernel<kZOH, kHasZ, io_t, bc_t, kAnyRows>), grid, dim3(kCBwdW * 64), 0, stream, p);
   return hipGetLastError();
 }
 

@@ -83,14 +83,16 @@ __device__ __forceinline__ void stage_round(const bc_t* __restrict__ Bb, const b
 }
 
 // kMaxS: the per-wave state tables' size (kMaxN, or kMaxNWide for float32 scans with more
-// states). kWhole: L is a multiple of the chunk and the B/C rows can be copied to LDS directly,
-// so no lane ever meets the row's end (the paths that handle it spill registers: B=8 D=2560
-// L=4096 float32 with lengths 306 us, the general instance 351). The general instance takes
-// B=3 D=1000 L=2051 bf16 in 92 us; element-wise accesses to such rows took 146.
+// states). kRows: kWholeRows, L is a multiple of the chunk and the B/C rows can be copied to LDS
+// directly, so no lane ever meets the row's end (the paths that handle it spill registers: B=8 D=2560
+// L=4096 float32 with lengths 306 us, the general instance 351); kSlotRows, the same B/C rows and L a
+// multiple of 16 bytes of activations (B=8 D=2048 L=4032 N=16 float32: 482 us, the general instance
+// 517; more than 16 states and rows of two types have no whole-row instance); kAnyRows, the general
+// one: B=3 D=1000 L=2051 bf16 in 92 us; element-wise accesses to such rows took 146.
 // kG: waves that share a channel, each taking every kG-th state of a staging round; their partial
 // outputs are added in order through LDS at the end of a chunk. 1 where the channels alone fill
 // the GPU (the waves of a channel repeat its delta and u loads and the softplus).
-template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS, bool kWhole, int kG>
+template <int kT, int kW, int kNB, int kOcc, bool kZOH, typename io_t, typename bc_t, int kMaxS, int kRows, int kG>
 __global__ __launch_bounds__(kW * 64) __attribute__((amdgpu_waves_per_eu(kOcc, kOcc)))
 void fwd_kernel(FwdParams p) {
   constexpr int kChunk = 64 * kT;
@@ -158,7 +160,7 @@ void fwd_kernel(FwdParams p) {
   }
   const float Dv = p.D ? p.D[d] : 0.f;
   const float bias = p.delta_bias ? p.delta_bias[d] : 0.f;
-  const bool dma = kWhole || p.vec_bc != 0;
+  const bool dma = kRows != kAnyRows || p.vec_bc != 0;
   float dsum_total = 0.f;  // sum of delta over all finished steps (reference residual)
 
   // Rounds of kNB states per chunk, padded to an even count so round g of every chunk
@@ -176,7 +178,7 @@ void fwd_kernel(FwdParams p) {
   for (int c = c_lo; c < c_end; ++c) {
     const int t0 = c * kChunk;
     const int tl = t0 + lane * kT;
-    const bool fast = kWhole || t0 + kChunk <= L;  // wave-uniform
+    const bool fast = kRows == kWholeRows || t0 + kChunk <= L;  // wave-uniform
     // Reference residual slot written at this chunk's end (2048-step boundary or end of
     // the sequence), -1 if none.
     const int chunk_end = t0 + kChunk;
@@ -191,7 +193,7 @@ void fwd_kernel(FwdParams p) {
         float zero[kT];
 #pragma unroll
         for (int j = 0; j < kT; ++j) zero[j] = 0.f;
-        if (p.out && grp == 0) store_seg<kT>(out_row, tl, L, fast, zero);
+        if (p.out && grp == 0) store_seg<kT>(out_row, tl, L, fast, zero, kRows);
         if (p.ref_states && lane == 63 && ref_idx >= 0) {
           for (int n = 0; n < N; ++n) {
             if (!own(n)) continue;
@@ -214,8 +216,8 @@ void fwd_kernel(FwdParams p) {
     const bool z_lds = kZLds && active && fast && p.vec_z && p.z != nullptr && p.out != nullptr;
     if (active) {
       Seg<kT, io_t> sd, su;
-      fetch(sd, dl_row, tl, L, kWhole);
-      fetch(su, u_row, tl, L, kWhole);
+      fetch(sd, dl_row, tl, L, kRows);
+      fetch(su, u_row, tl, L, kRows);
       if (kZLds && z_lds) {
         const io_t* zsrc = static_cast<const io_t*>(p.z) + row + tl;
 #pragma unroll
@@ -223,8 +225,8 @@ void fwd_kernel(FwdParams p) {
           __builtin_amdgcn_global_load_lds((gbl_void_t)(zsrc + q * (16 / static_cast<int>(sizeof(io_t)))),
                                            (lds_void_t)(&s_z[w][q * 64]), 16, 0, 0);
       }
-      finish(sd, tl, L, fast, dlt);
-      finish(su, tl, L, fast, y);
+      finish(sd, tl, L, fast, dlt, kRows);
+      finish(su, tl, L, fast, y, kRows);
 #pragma unroll
       for (int j = 0; j < kT; ++j) {
         const bool valid = tl + j < len;
@@ -286,7 +288,7 @@ void fwd_kernel(FwdParams p) {
             float* crow = p.carries + (chan * N + n) * p.n_seg + tl / kSegSteps;
 #pragma unroll
             for (int q = 0; q < kT / kSegSteps; ++q)
-              if (kWhole || tl / kSegSteps + q < p.n_seg) crow[q] = hseg[q];
+              if (kRows == kWholeRows || tl / kSegSteps + q < p.n_seg) crow[q] = hseg[q];
           }
         }
         const float run_new = readlane(hend, 63);
@@ -323,7 +325,7 @@ void fwd_kernel(FwdParams p) {
       if (active && p.z) {
 #pragma unroll
         for (int e = 0; e < kV; ++e)
-          zv[e] = (kWhole || t + e < L) ? to_f32((static_cast<const io_t*>(p.z) + row)[t + e]) : 0.f;
+          zv[e] = (kRows == kWholeRows || t + e < L) ? to_f32((static_cast<const io_t*>(p.z) + row)[t + e]) : 0.f;
       }
 #pragma unroll
       for (int j = 0; j < kT; ++j) s_y[w][j][lane] = y[j];
@@ -339,7 +341,7 @@ void fwd_kernel(FwdParams p) {
               store_as(static_cast<io_t*>(p.y_pre) + row + t + e, v);
             v *= zv[e] * sigmoid(zv[e]);
           }
-          if (kWhole || t + e < L) store_as(out_row + t + e, t + e < len ? v : 0.f);
+          if (kRows == kWholeRows || t + e < L) store_as(out_row + t + e, t + e < len ? v : 0.f);
         }
       }
     } else if (active && p.out) {
@@ -369,7 +371,7 @@ void fwd_kernel(FwdParams p) {
             }
           }
         } else {
-          load_seg<kT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zv, kWhole);
+          load_seg<kT>(static_cast<const io_t*>(p.z) + row, tl, L, fast, zv, kRows);
         }
         if (p.y_pre) {
           // The backward takes y sigma(z) from out / z; y itself is kept only where z is too
@@ -384,7 +386,7 @@ void fwd_kernel(FwdParams p) {
       }
 #pragma unroll
       for (int j = 0; j < kT; ++j) y[j] = (tl + j < len) ? y[j] : 0.f;
-      store_seg<kT>(out_row, tl, L, fast, y);
+      store_seg<kT>(out_row, tl, L, fast, y, kRows);
     }
   }
 }
@@ -486,13 +488,17 @@ static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   }
   if constexpr (kMaxS == kMaxN && sizeof(io_t) == sizeof(bc_t)) {
     if (p.vec_bc && p.seqlen % (64 * kT) == 0) {
-      hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, true, kG>), grid, dim3(kW * 64), 0,
-                         stream, p);
+      hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, kWholeRows, kG>), grid, dim3(kW * 64),
+                         0, stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, false, kG>), grid, dim3(kW * 64), 0,
-                     stream, p);
+  if (p.vec_bc && slots_fit<io_t>(p.seqlen))
+    hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, kSlotRows, kG>), grid, dim3(kW * 64), 0,
+                       stream, p);
+  else
+    hipLaunchKernelGGL((fwd_kernel<kT, kW, kNB, kOcc, kZOH, io_t, bc_t, kMaxS, kAnyRows, kG>), grid, dim3(kW * 64), 0,
+                       stream, p);
   return hipGetLastError();
 }
 
