@@ -458,15 +458,22 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       if (c == 0 && p.dinit && lane < N) p.dinit[chan * st_ld + lane] = s_mu[cl][lane];
 
       // ---- per-step gradients of the row
+      // With a gate, the addresses below are formed anew: those of the row's first loads, kept over
+      // the state loop instead, spilled registers of the 16-wave kernel (float32, ZOH 160 bytes a
+      // lane -> 132, Euler 88 -> 44; B=8 D=2048 L=4096 N=8 Euler 630 -> 615 us; bf16 at L=4032 847
+      // -> 830). bf16 rows of whole chunks are faster as they were (N=16 812 us, 814).
+      int t0_grads = t0;
+      if constexpr (kHasZ && (sizeof(io_t) == 4 || kRows == kSlotRows)) asm volatile("" : "+s"(t0_grads));
+      const int tg = t0_grads + seg * kT;
       if constexpr (!kZOH) {
         // Euler needs u only from here on: reload it rather than hold it across the loop.
-        load_seg<kT>(static_cast<const io_t*>(p.u) + row, tl, L, fast, uu, kRows);
+        load_seg<kT>(static_cast<const io_t*>(p.u) + row, tg, L, fast, uu, kRows);
       }
       float dD_acc = 0.f, db_acc = 0.f;
       float duv[kT], ddv[kT];
 #pragma unroll
       for (int j = 0; j < kT; ++j) {
-        const bool valid = tl + j < len;
+        const bool valid = tg + j < len;
         const float uv = valid ? uu[j] : 0.f;
         float du_j, dd_j;
         if constexpr (kZOH) {
@@ -489,15 +496,15 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       }
       if constexpr (kAcc) {
         float prev[kT];
-        load_seg<kT>(static_cast<const io_t*>(p.du) + row, tl, L, fast, prev, kRows);
+        load_seg<kT>(static_cast<const io_t*>(p.du) + row, tg, L, fast, prev, kRows);
 #pragma unroll
         for (int j = 0; j < kT; ++j) duv[j] += prev[j];
-        load_seg<kT>(static_cast<const io_t*>(p.ddelta) + row, tl, L, fast, prev, kRows);
+        load_seg<kT>(static_cast<const io_t*>(p.ddelta) + row, tg, L, fast, prev, kRows);
 #pragma unroll
         for (int j = 0; j < kT; ++j) ddv[j] += prev[j];
       }
-      store_seg<kT>(static_cast<io_t*>(p.du) + row, tl, L, fast, duv, kRows);
-      store_seg<kT>(static_cast<io_t*>(p.ddelta) + row, tl, L, fast, ddv, kRows);
+      store_seg<kT>(static_cast<io_t*>(p.du) + row, tg, L, fast, duv, kRows);
+      store_seg<kT>(static_cast<io_t*>(p.ddelta) + row, tg, L, fast, ddv, kRows);
       const float dD_sum = wave_sum_to_last(dD_acc);
       const float db_sum = wave_sum_to_last(db_acc);
       if (lane == 63) {
@@ -735,12 +742,22 @@ __global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ p
   }
 }
 
+// Whole rows have an instance of the 16-wave kernel, but for ZOH and gated float32 rows, where it
+// spills more than the slot one (B=4 D=2048 L=7680 N=4 652 us and 627, N=16 1519 and 1503).
+template <bool kZOH, bool kHasZ, typename io_t>
+constexpr bool whole_rows16() {
+  return !(kZOH && kHasZ && sizeof(io_t) == 4);
+}
+
 template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup, int kRows>
 static hipError_t launch_bwd_w(const BwdParams& p, hipStream_t stream) {
   dim3 grid(p.n_blocks_d, p.batch, p.n_split);
   if (p.waves == 16) {
     if (!bwd_waves_fit(16, p.dstate) || p.chan_per_block % 16 != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((bwd_kernel<16, kZOH, kHasZ, io_t, bc_t, kGroup, kRows>), grid, dim3(16 * 64), 0, stream, p);
+    if constexpr (kRows != kWholeRows || whole_rows16<kZOH, kHasZ, io_t>())
+      hipLaunchKernelGGL((bwd_kernel<16, kZOH, kHasZ, io_t, bc_t, kGroup, kRows>), grid, dim3(16 * 64), 0, stream, p);
+    else
+      return hipErrorInvalidValue;
   } else {
     if (p.waves != 12 || p.chan_per_block % 12 != 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL((bwd_kernel<12, kZOH, kHasZ, io_t, bc_t, kGroup, kRows>), grid, dim3(12 * 64), 0, stream, p);
@@ -751,7 +768,7 @@ static hipError_t launch_bwd_w(const BwdParams& p, hipStream_t stream) {
 template <bool kZOH, bool kHasZ, typename io_t, typename bc_t, int kGroup>
 static hipError_t launch_bwd_a(const BwdParams& p, hipStream_t stream) {
   if constexpr (kGroup == 0 && sizeof(io_t) == sizeof(bc_t)) {
-    if (p.vec_bc && p.seqlen % kBwdChunk == 0)
+    if (p.vec_bc && p.seqlen % kBwdChunk == 0 && (p.waves != 16 || whole_rows16<kZOH, kHasZ, io_t>()))
       return launch_bwd_w<kZOH, kHasZ, io_t, bc_t, kGroup, kWholeRows>(p, stream);
   }
   if (p.vec_bc && slots_fit<io_t>(p.seqlen))
