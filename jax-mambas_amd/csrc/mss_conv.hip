@@ -12,8 +12,8 @@
 // (Seg in mss_common.h); grid (step tiles, channels, batch). The K-1 halo steps around a
 // thread's vector come from its neighbours through LDS. Bound by HBM. Rows without 16-byte
 // alignment used to go one step to a thread, every thread reading its own halos: measured on
-// MI355X (bf16, 1536 channels, B=8 L=2047) forward 73 us, backward 191; so: 23 and 35
-// (17 and 31 at L=2048).
+// MI355X (bf16, 1536 channels, B=8 L=2047) forward 73 us, backward 176; so: 18 and 32
+// (17 and 29 at L=2048, where rows are whole vectors: kRows, mss_common.h).
 // Backward recomputes pre from x (no residual), forms g = dy * act'(pre), and writes
 //   dx[t] = sum_k w[k] * g[t + (K-1) - k],   and per-block partials of
 //   dw[k] = sum_t g[t] * x[t - (K-1) + k],   dbias = sum_t g[t]
@@ -48,7 +48,7 @@ struct ConvShare {
   static constexpr int kH = kK > 1 ? kK - 1 : 1;
 };
 
-template <int kK, int kE, bool kSilu, typename io_t>
+template <int kK, int kE, bool kSilu, typename io_t, int kRows>
 __global__ __launch_bounds__(kConvThreads) void conv_fwd_kernel(ConvParams p) {
   using Sh = ConvShare<kK, kE>;
   __shared__ float s_tail[Sh::kRows][Sh::kH];
@@ -56,7 +56,8 @@ __global__ __launch_bounds__(kConvThreads) void conv_fwd_kernel(ConvParams p) {
   const int d = blockIdx.y;
   const int b = blockIdx.z;
   const int tid = threadIdx.x;
-  const int t0 = (blockIdx.x * kConvThreads + tid) * kE;
+  const int threads = blockDim.x;
+  const int t0 = (blockIdx.x * threads + tid) * kE;
   const bool live = t0 < L;
   if (!Sh::kOn && !live) return;  // (no barrier without halos)
   const long long row = b * p.sb + d * p.sd;
@@ -71,7 +72,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_fwd_kernel(ConvParams p) {
   float xe[kE + kK - 1];  // x[t0 - (K-1) .. t0 + kE)
   float v[kE];
   const bool full = t0 + kE <= L;
-  load_seg<kE>(xr, t0, L, full, v);
+  load_seg<kE>(xr, t0, L, full, v, kRows);
   if constexpr (Sh::kOn) {
 #pragma unroll
     for (int k = 0; k < kK - 1; ++k) s_tail[tid][k] = v[kE - (kK - 1) + k];
@@ -94,10 +95,10 @@ __global__ __launch_bounds__(kConvThreads) void conv_fwd_kernel(ConvParams p) {
     for (int k = 0; k < kK; ++k) pre = __builtin_fmaf(w[k], xe[j + k], pre);
     out[j] = (t0 + j < len) ? (kSilu ? pre * sigmoid(pre) : pre) : 0.f;
   }
-  store_seg<kE>(yr, t0, L, full, out);
+  store_seg<kE>(yr, t0, L, full, out, kRows);
 }
 
-template <int kK, int kE, bool kSilu, typename io_t>
+template <int kK, int kE, bool kSilu, typename io_t, int kRows>
 __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvParams p) {
   using Sh = ConvShare<kK, kE>;
   __shared__ float s_red[kConvThreads / 64][kK + 1];
@@ -107,7 +108,8 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvParams p) {
   const int d = blockIdx.y;
   const int b = blockIdx.z;
   const int tid = threadIdx.x;
-  const int t0 = (blockIdx.x * kConvThreads + tid) * kE;
+  const int threads = blockDim.x;
+  const int t0 = (blockIdx.x * threads + tid) * kE;
   const long long row = b * p.sb + d * p.sd;
   const io_t* __restrict__ xr = static_cast<const io_t*>(p.x) + row;
   const io_t* __restrict__ gr = static_cast<const io_t*>(p.dy) + row;
@@ -132,10 +134,10 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvParams p) {
   float v[kE], dv[kE];
   {
     Seg<kE, io_t> sx, sg;
-    fetch(sx, xr, t0, L);
-    fetch(sg, gr, t0, L);
-    finish(sx, t0, L, full, v);
-    finish(sg, t0, L, full, dv);
+    fetch(sx, xr, t0, L, kRows);
+    fetch(sg, gr, t0, L, kRows);
+    finish(sx, t0, L, full, v, kRows);
+    finish(sg, t0, L, full, dv, kRows);
   }
 #pragma unroll
   for (int j = 0; j < kE; ++j) {
@@ -144,7 +146,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvParams p) {
   }
   // The last thread of the workgroup (or every thread without halos) reads what comes
   // after its vector; the others take the next thread's gradient terms below.
-  const bool own_after = !Sh::kOn || tid == kConvThreads - 1;
+  const bool own_after = !Sh::kOn || tid == threads - 1;
   if constexpr (Sh::kOn) {
 #pragma unroll
     for (int k = 0; k < kK - 1; ++k) s_xt[tid][k] = v[kE - (kK - 1) + k];
@@ -194,7 +196,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvParams p) {
       for (int k = 0; k < kK; ++k) dw[k] = __builtin_fmaf(ge[j], xe[j + k], dw[k]);
       dw[kK] += ge[j];
     }
-    store_seg<kE>(dxr, t0, L, full, dx);
+    store_seg<kE>(dxr, t0, L, full, dx, kRows);
   }
   // block sums of dw / dbias -> partial slot (d, b, blockIdx.x)
 #pragma unroll
@@ -207,8 +209,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvParams p) {
   __syncthreads();
   if (threadIdx.x <= kK) {
     float s = 0.f;
-#pragma unroll
-    for (int i = 0; i < kConvThreads / 64; ++i) s += s_red[i][threadIdx.x];
+    for (int i = 0; i < threads / 64; ++i) s += s_red[i][threadIdx.x];
     const size_t slot = (static_cast<size_t>(d) * p.batch + b) * gridDim.x + blockIdx.x;
     p.part[slot * (kK + 1) + threadIdx.x] = s;
   }
@@ -233,21 +234,31 @@ __global__ __launch_bounds__(256) void conv_reduce_kernel(const float* __restric
 
 int conv_tile_steps(int io_bf16) { return kConvThreads * (io_bf16 ? 8 : 4); }
 
-template <int kK, bool kSilu, typename io_t>
+template <int kK, bool kSilu, typename io_t, int kRows>
 static hipError_t launch_conv_t(const ConvParams& p, bool bwd, hipStream_t stream) {
   constexpr int kV = sizeof(io_t) == 2 ? 8 : 4;
-  const dim3 grid((p.seqlen + kConvThreads * kV - 1) / (kConvThreads * kV), p.dim, p.batch);
+  // No more waves to a workgroup than its row fills: the idle ones of short rows cost more than the
+  // work (four waves always, measured on MI355X, bf16: B=8 D=1536 L=100 forward 9.4 us and backward
+  // 26, now 7.5 and 14; B=64 D=768 L=5 34 and 92, now 24 and 37).
+  const int waves = p.seqlen < kConvThreads * kV ? (p.seqlen + 64 * kV - 1) / (64 * kV) : kConvThreads / 64;
+  const dim3 grid((p.seqlen + kConvThreads * kV - 1) / (kConvThreads * kV), p.dim, p.batch), block(64 * waves);
   if (bwd)
-    hipLaunchKernelGGL((conv_bwd_kernel<kK, kV, kSilu, io_t>), grid, dim3(kConvThreads), 0, stream, p);
+    hipLaunchKernelGGL((conv_bwd_kernel<kK, kV, kSilu, io_t, kRows>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((conv_fwd_kernel<kK, kV, kSilu, io_t>), grid, dim3(kConvThreads), 0, stream, p);
+    hipLaunchKernelGGL((conv_fwd_kernel<kK, kV, kSilu, io_t, kRows>), grid, block, 0, stream, p);
   return hipGetLastError();
+}
+
+template <int kK, bool kSilu, typename io_t>
+static hipError_t launch_conv_r(const ConvParams& p, bool bwd, hipStream_t stream) {
+  return slots_fit<io_t>(p.seqlen) ? launch_conv_t<kK, kSilu, io_t, kSlotRows>(p, bwd, stream)
+                                   : launch_conv_t<kK, kSilu, io_t, kAnyRows>(p, bwd, stream);
 }
 
 template <int kK, typename io_t>
 static hipError_t launch_conv_k(const ConvParams& p, bool bwd, bool silu, hipStream_t stream) {
-  return silu ? launch_conv_t<kK, true, io_t>(p, bwd, stream)
-              : launch_conv_t<kK, false, io_t>(p, bwd, stream);
+  return silu ? launch_conv_r<kK, true, io_t>(p, bwd, stream)
+              : launch_conv_r<kK, false, io_t>(p, bwd, stream);
 }
 
 template <typename io_t>

@@ -68,6 +68,13 @@ def test_conv_at_any_alignment(l, dtype, layout):
     conv_case(3, 5, l, 4, dtype, layout=layout, lens=[l, l - 1, l // 2], seed=l)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("l", [1, 8, 256, 257, 512, 520, 768, 1024, 1028, 1032, 1536, 2048, 2052])
+def test_conv_workgroups_of_fewer_waves(l, dtype):
+    """Rows that fill one to four waves of a workgroup, whole vectors or not, and just more."""
+    conv_case(2, 5, l, 4, dtype, lens=[l, l // 2], seed=l)
+
+
 @pytest.mark.parametrize("l,n,lens,io,bc", [
     (l, n, lens, io, bc)
     for l, n, lens in [(8, 4, None), (504, 16, None), (520, 5, [520, 509]), (1032, 3, None), (1024, 16, None), (1028, 4, None),
