@@ -32,7 +32,7 @@ BwdPlan bwd_plan(int batch, int dim, int seqlen, int dstate, int varlen, bool sp
 hipError_t launch_cfwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
 hipError_t launch_cbwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
 BwdPlan cbwd_plan(int batch, int dim, int seqlen, bool split);
-FwdPlan cfwd_plan(int batch, int dim, int seqlen);
+FwdPlan cfwd_plan(int batch, int dim, int seqlen, int dstate);
 hipError_t launch_cssm_step(const StepParams& p, bool zoh, bool io_bf16, bool bc_bf16, hipStream_t stream);
 hipError_t launch_conv(const ConvParams& p, bool bwd, bool silu, bool io_bf16,
                        hipStream_t stream);
@@ -232,7 +232,7 @@ int validate_bwd(const mss_bwd_args* a, bool cplx = false) {
 }
 
 mss::FwdPlan fwd_plan_of(const mss_fwd_args* a, bool cplx) {
-  return cplx ? mss::cfwd_plan(a->batch, a->dim, a->seqlen) : mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate);
+  return cplx ? mss::cfwd_plan(a->batch, a->dim, a->seqlen, a->dstate) : mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate);
 }
 
 // Room for the split maps of a call whose sizes are valid.

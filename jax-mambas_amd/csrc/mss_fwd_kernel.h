@@ -502,6 +502,23 @@ static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Whether four waves share a channel (`groups` workgroups with one wave each): where the grid still
+// fits one pass of the narrow shape, and each wave's states outweigh the delta and u rows, softplus
+// and output exchange that the four repeat. That takes more states the more workgroups a CU holds
+// already (one, two, three), fewer for bf16 rows; a ZOH state weighs three. Measured on MI355X, B=1
+// L=4096, one wave and four: D=768 float32 N=6 42 and 44 us, N=8 47 and 44; bf16 N=3 32 and 32, N=8 50
+// and 39; D=1536 float32 N=4 37 and 48, N=16 80 and 79, ZOH N=8 88 and 75; bf16 N=11 65 and 63, N=16 81
+// and 72. D=400 L=2048 float32 N=1 12.9 and 14.0, N=4 17.7 and 15.2.
+template <typename io_t>
+static bool fwd_shares_channels(const FwdParams& p, long long groups, bool zoh) {
+  const long long wgs = kFwdG * groups;
+  if (wgs > kFwdNarrowSlots) return false;
+  if (p.n_split > 1) return true;
+  constexpr bool kHalf = sizeof(io_t) == 2;
+  const int least = wgs <= kCUs ? 2 : wgs <= 2 * kCUs ? (kHalf ? 4 : 8) : (kHalf ? 12 : 20);
+  return p.dstate * (zoh ? 3 : 1) >= least;
+}
+
 template <bool kZOH, typename io_t, typename bc_t>
 static hipError_t launch_fwd_z(const FwdParams& p, hipStream_t stream) {
   if (p.dstate > kMaxN) {
@@ -517,16 +534,15 @@ static hipError_t launch_fwd_z(const FwdParams& p, hipStream_t stream) {
   // Float32 rows take the narrow shape at every grid size (measured on MI355X: B=16 D=2560
   // L=8192 with variable lengths 1.69 -> 1.39 ms, B=8 D=2048 L=4096 0.54 -> 0.48 ms); bf16
   // rows take it only when the grid fits one pass of it (B=8 D=2048 L=4096 428 vs 436 us,
-  // B=8 D=1536 L=2048 167 vs 175 us wide vs narrow). Four waves share a channel where that
-  // still fits one pass: B=1 D=1536 L=16384 bf16 333 -> 275 us (two waves: 311; eight over rounds
-  // of eight states: 364), B=1 D=256 L=8192 float32 133 -> 66 (108; 52). Over two passes they
-  // lose: a B=3 D=1000 L=2051 bf16 training call takes 249 us with one wave, 268 with four.
+  // B=8 D=1536 L=2048 167 vs 175 us wide vs narrow). Four waves to a channel: B=1 D=1536 L=16384
+  // bf16 333 -> 275 us (two waves: 311; eight over rounds of eight states: 364). Over two passes
+  // they lose: a B=3 D=1000 L=2051 bf16 training call takes 249 us with one wave, 268 with four.
   const long long groups = static_cast<long long>(p.batch) * ((p.dim + MSS_FWD_W - 1) / MSS_FWD_W);
   if constexpr (sizeof(io_t) == 2) {
     if (groups > kFwdNarrowSlots)
       return launch_fwd_t<MSS_FWD_T_WIDE, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_WIDE, kZOH, io_t, bc_t>(p, stream);
   }
-  if (kFwdG * groups <= kFwdNarrowSlots)
+  if (fwd_shares_channels<io_t>(p, groups, kZOH))
     return launch_fwd_t<MSS_FWD_T_NARROW, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_NARROW, kZOH, io_t, bc_t, kMaxN, kFwdG>(
         p, stream);
   return launch_fwd_t<MSS_FWD_T_NARROW, MSS_FWD_W, MSS_FWD_NB, MSS_FWD_OCC_NARROW, kZOH, io_t, bc_t>(p, stream);

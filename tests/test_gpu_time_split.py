@@ -289,3 +289,24 @@ def test_growth_over_a_split_from_nothing(cplx, backward):
     for i, (want, got) in enumerate(zip(*res)):
         want, got = (torch.view_as_real(t.detach()) if t.is_complex() else t.detach() for t in (want, got))
         assert bool(torch.isfinite(want).all()) and torch.equal(got, want), i
+
+
+@pytest.mark.parametrize("b,d,l,n,dtype,zoh,cplx", [
+    (1, 300, 700, 1, "f32", False, False), (1, 300, 700, 2, "f32", False, False),   # a workgroup a CU or fewer
+    (1, 600, 700, 7, "f32", False, False), (1, 600, 700, 8, "f32", False, False),   # two
+    (1, 600, 700, 3, "bf16", False, False), (1, 600, 700, 4, "bf16", False, False),
+    (1, 1100, 700, 6, "f32", True, False), (1, 1100, 700, 7, "f32", True, False),   # three
+    (1, 1100, 700, 11, "bf16", False, False), (1, 1100, 700, 12, "bf16", False, False),
+    (1, 300, 700, 2, "f32", False, True), (1, 300, 700, 3, "f32", False, True),     # two waves a SIMD or fewer
+    (1, 600, 700, 3, "f32", False, True), (1, 600, 700, 3, "f32", True, True), (1, 200, 700, 2, "f32", False, True),
+])
+def test_states_at_which_waves_share_a_channel(b, d, l, n, dtype, zoh, cplx):
+    """Either side of the state counts from which four waves share a channel."""
+    log(f"case sharing b={b} d={d} l={l} n={n} {dtype} zoh={zoh} cplx={cplx}")
+    if cplx:
+        x, dout, dlast = complex_case(4200 + d + n, b, d, l, n, dtype)
+        check_complex(x, dout, dlast, zoh, dtype)
+        return
+    x, dout, dlast = fused_case(4200 + d + n, b, d, l, n, dtype, zoh=zoh)
+    ts, out, last = run_fused(x, dout, dlast, dtype, zoh)
+    check_fused(ts, out, last, *oracle_fused(x, dout, dlast, zoh), *tol(dtype))
