@@ -458,12 +458,13 @@ __global__ __launch_bounds__(kW * 64) void bwd_kernel(BwdParams p) {
       if (c == 0 && p.dinit && lane < N) p.dinit[chan * st_ld + lane] = s_mu[cl][lane];
 
       // ---- per-step gradients of the row
-      // With a gate, the addresses below are formed anew: those of the row's first loads, kept over
-      // the state loop instead, spilled registers of the 16-wave kernel (float32, ZOH 160 bytes a
-      // lane -> 132, Euler 88 -> 44; B=8 D=2048 L=4096 N=8 Euler 630 -> 615 us; bf16 at L=4032 847
-      // -> 830). bf16 rows of whole chunks are faster as they were (N=16 812 us, 814).
+      // With a gate and 16 waves the addresses below are formed anew: those of the row's first loads,
+      // kept over the state loop instead, spilled registers (float32, ZOH 160 bytes a lane -> 132,
+      // Euler 88 -> 44; B=8 D=2048 L=4096 N=8 Euler 630 -> 615 us; bf16 at L=4032 847 -> 830). bf16
+      // rows of whole chunks are faster as they were (N=16 812 us, 814), and so are 12 waves, which
+      // have the registers to keep u as well (B=1 D=781 L=281 N=5 float32 33.3 us, 34.8).
       int t0_grads = t0;
-      if constexpr (kHasZ && (sizeof(io_t) == 4 || kRows == kSlotRows)) asm volatile("" : "+s"(t0_grads));
+      if constexpr (kW == 16 && kHasZ && (sizeof(io_t) == 4 || kRows == kSlotRows)) asm volatile("" : "+s"(t0_grads));
       const int tg = t0_grads + seg * kT;
       if constexpr (!kZOH) {
         // Euler needs u only from here on: reload it rather than hold it across the loop.
@@ -819,12 +820,15 @@ static int chan_per_block_for(int waves, int batch, int dim, long long target) {
 // The plan of a grid whose whole-row workgroups would leave half the CUs or more idle: rows are
 // split in time as well, so that the grid fills one pass. More channel rounds K per workgroup
 // then mean more, shorter splits: fewer dB/dC partials to write and reduce, against more steps
-// in the adjoint maps (every split but the first). The modelled microseconds, from MI355X
-// measurements at B=1 D=1536 L=16384 N=16 bf16: a 12-wave round of a chunk 7 + 1.1 N, the maps
-// 0.25 per million (step, state), partials at 4.5 TB/s each way. There the backward took 840 us
-// as 128 whole-row workgroups (scan 787, reduction 53) and takes 525 as 16 splits of 8 rounds
-// (maps 130, scan 385, reduction 10; two splits of one round: 540); B=2 D=768 L=1024 float32 ZOH
-// 83 -> 62. Grids over half the CUs stay whole: the maps cost a third of the scan.
+// in the adjoint maps (every split but the first). The modelled microseconds: a 12-wave round of a
+// chunk 7 + 1.1 N, the maps 0.25 per million (step, state), partials at 4.5 TB/s each way, from
+// MI355X measurements at B=1 D=1536 L=16384 N=16 bf16. A round measured over N (gated rows, 256
+// workgroups): bf16 Euler N=1 9.2, N=4 10.9, N=8 15.1, N=16 23.3, so within 2 us of the model; float32
+// 3.5 us more, ZOH 0.9 a state more, which the plan does not look at (of 400 random shapes with
+// batch * dim up to 4096 no backward was over 3 % slower than with whole rows). There the backward
+// took 840 us as 128 whole-row workgroups (scan 787, reduction 53) and takes 470 to 520 as 16 splits of 8
+// rounds; B=2 D=768 L=1024 float32 ZOH 83 -> 62. Grids over half the CUs stay whole: the maps cost a
+// third of the scan.
 static BwdPlan bwd_split_plan(int batch, int dim, int seqlen, int dstate, int n_chunks) {
   BwdPlan best{};
   double best_us = 0;
