@@ -193,7 +193,8 @@ int mss_transpose(const mss_transpose_entry* entries, int32_t n, void* stream);
 
 /* mss_fwd with a workspace, in which few channels with long rows are split in time (the same
  * results up to the rounding of the state handed from split to split). The workspace holds
- * mss_fwd_workspace_bytes(args) bytes, 16-byte aligned; 0 bytes: none is needed or read. */
+ * mss_fwd_workspace_bytes(args) bytes (from the shapes, types and discretization), 16-byte
+ * aligned; 0 bytes: none is needed or read. */
 size_t mss_fwd_workspace_bytes(const mss_fwd_args* args);
 int mss_fwd_ws(const mss_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
 int mss_bwd(const mss_bwd_args* args, void* stream);

@@ -27,7 +27,7 @@ hipError_t launch_bwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16
                            hipStream_t stream);
 hipError_t launch_bwd_reduce(const BwdParams& p, int bc_bf16, int a_width, int a_ld, int acc_bias,
                              void* dA, void* dB, void* dC, float* dD, float* dbias, hipStream_t stream);
-FwdPlan fwd_plan(int batch, int dim, int seqlen, int dstate);
+FwdPlan fwd_plan(int batch, int dim, int seqlen, int dstate, bool zoh);
 BwdPlan bwd_plan(int batch, int dim, int seqlen, int dstate, int varlen, bool split);
 hipError_t launch_cfwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
 hipError_t launch_cbwd_scan(const BwdParams& p, int zoh, int io_bf16, int bc_bf16, hipStream_t stream);
@@ -232,7 +232,8 @@ int validate_bwd(const mss_bwd_args* a, bool cplx = false) {
 }
 
 mss::FwdPlan fwd_plan_of(const mss_fwd_args* a, bool cplx) {
-  return cplx ? mss::cfwd_plan(a->batch, a->dim, a->seqlen, a->dstate) : mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate);
+  return cplx ? mss::cfwd_plan(a->batch, a->dim, a->seqlen, a->dstate)
+              : mss::fwd_plan(a->batch, a->dim, a->seqlen, a->dstate, a->discretization == MSS_ZOH);
 }
 
 // Room for the split maps of a call whose sizes are valid.

@@ -974,10 +974,11 @@ hipError_t launch_cssm_step(const StepParams& p, bool zoh, bool io_bf16, bool bc
 // 512 channels (two waves a SIMD), two up to 256. One wave and four, B=1 L=1024 float32: D=128 N=1 5.7
 // and 6.0 us, N=2 7.0 and 6.1; D=300 N=2 7.4 and 7.7, N=3 8.7 and 7.9; D=600 N=3 9.3 and 10.3, N=4 10.8
 // and 10.6; D=1280 N=1 8.5 and 12.0, N=4 15.9 and 14.9. Rows are split in time where even those leave
-// four fifths idle (256 channels or fewer), as fwd_plan does for real states (one state: four chunks
-// off the chain at least). Measured on MI355X, N=16 float32: B=1 D=400 L=8000 356 us
-// with a wave to a channel, 165 with four; whole and split (maps among it) B=1 D=300 L=4096 60 and
-// 57 (four splits), D=600 L=2048 43 and 58, L=8192 173 and 209 (two splits).
+// more than a third of the SIMDs idle (160 channels or fewer) and at least three chunks go off the
+// chain (one state: four), as fwd_plan does for real states. Measured on MI355X, N=16 float32: B=1
+// D=400 L=8000 356 us with a wave to a channel, 165 with four; whole and split (maps among it) B=1
+// D=64 L=1536 14.4 and 14.5, L=2048 18 and 15, L=8192 67 and 30; D=160 L=4096 36 and 36, L=8192 70 and
+// 64; D=200 L=4096 37 and 48, L=8192 72 and 71; D=256 L=8192 71 and 89.
 constexpr int kCFwdSlots = 5 * 4 * kCUs;
 
 static bool cfwd_groups(const FwdParams& p, bool zoh) {
@@ -991,10 +992,10 @@ FwdPlan cfwd_plan(int batch, int dim, int seqlen, int dstate) {
   const int n_chunks = (seqlen + kCChunk - 1) / kCChunk;
   FwdPlan plan{1, n_chunks};
   const long long waves = 4LL * batch * dim;
-  if (5 * waves > kCFwdSlots) return plan;
+  if (8 * waves > kCFwdSlots) return plan;
   const int s = static_cast<int>(kCFwdSlots / waves < n_chunks ? kCFwdSlots / waves : n_chunks);
   const int per = (n_chunks + s - 1) / s;
-  if (n_chunks - per < (dstate == 1 ? 4 : 2)) return plan;
+  if (n_chunks - per < (dstate == 1 ? 4 : 3)) return plan;
   return FwdPlan{(n_chunks + per - 1) / per, per};
 }
 

@@ -30,18 +30,19 @@ hipError_t launch_fwd(const FwdParams& p, int zoh, int io_bf16, int bc_bf16, hip
 }
 
 // Rows are split in time where even four waves a channel leave two thirds of the GPU idle (512
-// channels or fewer): splits for one pass of workgroups, as long as at least three chunks of the
-// row's chain go (a chunk takes about 4 us there, the maps' launch and one chunk of them 8).
-// Measured on MI355X, N=16 float32, whole and split (maps among it): B=1 D=256 L=8192 84 us and 53,
-// D=128 L=2048 23 and 14, D=500 L=5000 66 and 60; two splits no longer pay (D=700 L=4096 60 and 62,
-// D=768 L=16384 237 and 241). With one or two states a chunk is shorter and the splits of several
+// channels or fewer; ZOH, whose maps cost more, three quarters: 384): splits for one pass of
+// workgroups, as long as at least three chunks of the row's chain go (a chunk takes about 4 us
+// there, the maps' launch and one chunk of them 8). Measured on MI355X, gated N=16 float32, whole and
+// split (maps among it): B=1 D=256 L=8192 84 us and 53 (without the gate 71 and 50), D=128 L=2048 22
+// and 14, D=512 L=8192 86 and 79; ZOH D=256 L=8192 115 and 88, D=400 116 and 129; two splits no longer
+// pay (D=700 L=4096 60 and 62, D=768 L=16384 237 and 241). With one or two states a chunk is shorter and the splits of several
 // chunks must take four off the chain (D=512 L=2560 N=1: 15.9 us whole with a wave to a channel, 17.4
 // in three splits).
-FwdPlan fwd_plan(int batch, int dim, int seqlen, int dstate) {
+FwdPlan fwd_plan(int batch, int dim, int seqlen, int dstate, bool zoh) {
   const int n_chunks = (seqlen + kPartChunk - 1) / kPartChunk;
   FwdPlan plan{1, n_chunks};
   const long long groups = static_cast<long long>(batch) * ((dim + MSS_FWD_W - 1) / MSS_FWD_W) * kFwdG;
-  if (dstate > kMaxN || 3 * groups > kFwdNarrowSlots) return plan;
+  if (dstate > kMaxN || (zoh ? 4 : 3) * groups > kFwdNarrowSlots) return plan;
   const int s = static_cast<int>(kFwdNarrowSlots / groups < n_chunks ? kFwdNarrowSlots / groups : n_chunks);
   const int per = (n_chunks + s - 1) / s;
   if (n_chunks - per < (dstate <= 2 && per > 1 ? 4 : 3)) return plan;

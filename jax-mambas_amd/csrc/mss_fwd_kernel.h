@@ -505,18 +505,26 @@ static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
 // Whether four waves share a channel (`groups` workgroups with one wave each): where the grid still
 // fits one pass of the narrow shape, and each wave's states outweigh the delta and u rows, softplus
 // and output exchange that the four repeat. That takes more states the more workgroups a CU holds
-// already (one, two, three), fewer for bf16 rows; a ZOH state weighs three. Measured on MI355X, B=1
-// L=4096, one wave and four: D=768 float32 N=6 42 and 44 us, N=8 47 and 44; bf16 N=3 32 and 32, N=8 50
-// and 39; D=1536 float32 N=4 37 and 48, N=16 80 and 79, ZOH N=8 88 and 75; bf16 N=11 65 and 63, N=16 81
-// and 72. D=400 L=2048 float32 N=1 12.9 and 14.0, N=4 17.7 and 15.2.
+// already (one, two, three), fewer for ZOH and for bf16 rows. Measured on MI355X, B=1 L=4096, one wave
+// and four: D=400 (L=2048) float32 N=1 12.9 and 14.0 us, N=4 17.7 and 15.2; D=768 float32 N=6 42 and
+// 44, N=8 47 and 44, ZOH N=2 38 and 41, N=3 46 and 42, bf16 N=3 32 and 32, N=8 50 and 39; D=1536 float32
+// N=4 37 and 48, N=16 80 and 79 (L=1024 22 and 24; L=4097, the general instance, 113 and 106), ZOH N=6
+// 73 and 71 (L=1024 20 and 22), N=8 88 and 75, bf16 N=11 65 and 63 (L=1024 18 and 20), N=16 81 and 72.
 template <typename io_t>
 static bool fwd_shares_channels(const FwdParams& p, long long groups, bool zoh) {
   const long long wgs = kFwdG * groups;
   if (wgs > kFwdNarrowSlots) return false;
   if (p.n_split > 1) return true;
   constexpr bool kHalf = sizeof(io_t) == 2;
-  const int least = wgs <= kCUs ? 2 : wgs <= 2 * kCUs ? (kHalf ? 4 : 8) : (kHalf ? 12 : 20);
-  return p.dstate * (zoh ? 3 : 1) >= least;
+  const bool general = !p.vec_bc || !slots_fit<io_t>(p.seqlen);
+  int least;
+  if (wgs <= kCUs)
+    least = zoh ? 1 : 2;
+  else if (wgs <= 2 * kCUs)
+    least = kHalf ? (zoh ? 2 : 4) : (zoh ? 3 : 8);
+  else
+    least = kHalf ? (zoh ? 4 : 12) : zoh ? 7 : general ? 16 : kMaxN + 1;
+  return p.dstate >= least;
 }
 
 template <bool kZOH, typename io_t, typename bc_t>

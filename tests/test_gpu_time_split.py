@@ -258,7 +258,7 @@ def test_growth_over_a_split_from_nothing(cplx, backward):
     """A growing state (Re A > 0) that is zero, and an adjoint that is zero, stay zero over a split
     or map whose product of a_bar overflows float32 (e^120; a chunk's e^60 does not): the outputs of
     the same call with those steps' delta zero."""
-    b, d, l, n = ((8, 40, 4100, 3) if cplx else (1, 768, 12000, 1)) if backward else ((1, 256, 4096, 2) if cplx else (1, 500, 4096, 4))
+    b, d, l, n = ((8, 40, 4100, 3) if cplx else (1, 768, 12000, 1)) if backward else ((1, 160, 8192, 2) if cplx else (1, 500, 4096, 4))
     if backward:
         assert bwd_plan(b, d, l, n, cplx=cplx)[2] == 2
         still = slice(3072, 4096) if cplx else slice(10240, 11264)  # the two chunks of a map
