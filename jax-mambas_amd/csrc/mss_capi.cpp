@@ -1254,8 +1254,9 @@ int mss_transpose(const mss_transpose_entry* entries, int32_t n, void* stream) {
     p.e[i].dst = e.dst;
     p.e[i].rows = e.rows;
     p.e[i].cols = e.cols;
-    p.e[i].tiles = (e.rows + 63LL) / 64 * ((e.cols + 63LL) / 64) * e.batch;
-    if (p.e[i].tiles >= (1LL << 31)) return MSS_ERR_UNSUPPORTED;
+    const long long per_batch = (e.rows + 63LL) / 64 * ((e.cols + 63LL) / 64);
+    if (per_batch >= (1LL << 31) || per_batch * e.batch >= (1LL << 31)) return MSS_ERR_UNSUPPORTED;
+    p.e[i].tiles = per_batch * e.batch;
     tiles += p.e[i].tiles;
   }
   for (int i = 0; i < n; ++i)

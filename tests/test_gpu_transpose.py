@@ -57,5 +57,8 @@ def test_transpose_validates():
                dict(dst=(1 << 20) + 128)):
         assert lib.mss_transpose(arr(e(**kw)), 1, None) == bad, kw
     assert lib.mss_transpose(arr(e(), e(src=1 << 22)), 2, None) == bad  # two destinations at one place
+    huge = (1 << 31) - 1
+    for kw in (dict(batch=huge, rows=huge, cols=huge), dict(rows=huge, cols=huge), dict(batch=huge, rows=1 << 20)):
+        assert lib.mss_transpose(arr(e(src=1 << 40, dst=1 << 60, **kw)), 1, None) == _lib.MSS_ERR_UNSUPPORTED, kw
     assert lib.mss_transpose(arr(e(rows=1 << 30, cols=1 << 20, src=1 << 40, dst=1 << 60)), 1, None) == \
         _lib.MSS_ERR_UNSUPPORTED
