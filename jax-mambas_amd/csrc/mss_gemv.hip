@@ -319,8 +319,9 @@ __device__ __forceinline__ void norm_load(const NormParams& q, int K, NormLoads<
 // bit. Every workgroup computes X (a few KB from the L2); workgroup 0 also stores hn and
 // rstd. A chain of latencies in front of the products, so it is kept short. Measured on MI355X,
 // the in-projection of a 130M decode step (3072 x 768, 8 tokens), 8.2 us: one root and division
-// a lane and no feature slot past K 7.5, the token sums without a branch between them 7.3, the
-// loads ahead of the weights' 6.5.
+// a lane and three feature slots instead of four 7.5, the token sums without a branch between them
+// 7.3, the loads ahead of the weights' 6.5. (Three slots serve up to 768 features, four the rest:
+// narrower streams load a slot or two clamped and leave it out of the sums, as all widths did.)
 template <int kN, bool kTransposed, int kFeat>
 __device__ __forceinline__ void norm_finish(const NormParams& q, int K, NormLoads<kN, kFeat>& o, bf16_t* X,
                                             float (*s_ss)[4]) {

@@ -20,8 +20,9 @@ Both run through two torch.library custom ops, ``torch.ops.mamba_amd.selective_s
 and ``selective_scan_bwd`` (the C ABI's mss_fwd/mss_bwd, or mss_cfwd/mss_cbwd for a complex
 A), with fake implementations (shapes, dtypes and row layouts) and registered autograd, so
 they are differentiable and traceable by torch.compile; gradients come from the HIP backward
-kernel. A plain eager call, which nothing traces, transforms or intercepts, reaches the same
-functions without the dispatcher. There is no CPU path: inputs must live on a ROCm GPU and the library must be built.
+kernel. A plain eager call, which nothing traces, transforms, intercepts or profiles, reaches the
+same functions without the dispatcher (and without a kernel that a program registers for the op).
+There is no CPU path: inputs must live on a ROCm GPU and the library must be built.
 """
 from __future__ import annotations
 
